@@ -1084,10 +1084,12 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     return s;
   }
 
-  // ops[0, nops): the segment's steps; out_buf: the buffer of tail[0]'s iterate at the end
-  template<typename DT_, typename VT_>
+  // ops[0, nops): the segment's steps; out_buf: the buffer of tail[0]'s iterate at the end.
+  // UNIT_: block j takes the j-th unit vector as the right-hand side and writes column j of the
+  // segment's matrix mat (row-major, n x n) instead of an iterate (see k_tail_apply).
+  template<typename DT_, typename VT_, bool UNIT_ = false>
   __global__ __launch_bounds__(kTailThreads) void k_tail(TailDesc<DT_, VT_> d, const u32* __restrict__ ops, u32 nops,
-                                                         u32 out_buf, const int* status)
+                                                         u32 out_buf, const int* status, DT_* __restrict__ mat = nullptr)
   {
     if(stopped(status)) return;
     extern __shared__ double tail_arena_[];
@@ -1105,7 +1107,7 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
         if(i == 0)
         {
           // the first smoothing step from x = 0 (as the restriction above writes it)
-          const DT_ b = d.rhs_in[r];
+          const DT_ b = UNIT_ ? DT_(r == blockIdx.x ? 1 : 0) : d.rhs_in[r];
           v[2 * l.n + r] = b;
           v[r] = di * b;
         }
@@ -1174,7 +1176,46 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     }
     const TailLevel<DT_, VT_>& t = d.lv[0];
     const DT_* xf = arena + t.off + out_buf * t.n;
-    for(u32 r = tid; r < t.n; r += kTailThreads) d.x_out[r] = xf[r];
+    for(u32 r = tid; r < t.n; r += kTailThreads)
+    {
+      if constexpr(UNIT_) mat[u64(r) * t.n + blockIdx.x] = xf[r];
+      else d.x_out[r] = xf[r];
+    }
+  }
+
+  // A segment of the cycle on the coarse tail is a linear map from tail[0]'s right-hand side to its
+  // iterate, fixed once the levels and the smoothers are: init forms its matrix column by column
+  // (k_tail with UNIT_, the arithmetic of the cycle) and the cycle applies it with one product, one
+  // wave per row.  k_tail itself is a chain of 20 to 40 dependent steps of 0.7 to 1.6 us on one CU,
+  // whatever the levels' sizes; the product reads at most 9.5 MB (1089 rows in FP64), which the L2s
+  // hold, over the whole chip.
+  constexpr u64 kTailMatRows = 2048;   // levels of at most this many rows (a 33 MB matrix in FP64)
+  template<typename DT_>
+  __global__ __launch_bounds__(256) void k_tail_apply(u32 n, const DT_* __restrict__ mat, const DT_* __restrict__ rhs,
+                                                      DT_* __restrict__ x, const int* status)
+  {
+    if(stopped(status)) return;
+    const u32 lane = threadIdx.x % u32(dev::kWave);
+    const u32 r = blockIdx.x * 4u + threadIdx.x / u32(dev::kWave);
+    if(r >= n) return;
+    const DT_* a = mat + u64(r) * n;
+    constexpr u32 U = 6;   // loads of a lane in flight (of each operand)
+    double s = 0.0;   // (costs nothing here, and the FP32 product then adds only its entries' rounding)
+    for(u32 j0 = lane; j0 < n; j0 += U * u32(dev::kWave))
+    {
+      DT_ av[U], bv[U];
+#pragma unroll
+      for(u32 k = 0; k < U; ++k)
+      {
+        const u32 j = j0 + k * u32(dev::kWave);
+        av[k] = j < n ? a[j] : DT_(0);
+        bv[k] = j < n ? rhs[j] : DT_(0);
+      }
+#pragma unroll
+      for(u32 k = 0; k < U; ++k) s = fmadd(double(av[k]), double(bv[k]), s);
+    }
+    s = dev::wave_sum(s);
+    if(lane == 0u) x[r] = DT_(s);
   }
 
   // ---- setup kernels -----------------------------------------------------------------------

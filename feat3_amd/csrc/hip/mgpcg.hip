@@ -1823,10 +1823,50 @@ namespace
     // operation stands for the coarse solve (k_coarse) or for such a segment.
     enum class Op : int { entry, sweep, defect, rest, rest_step, bottom, prol, copy_top };
     struct CycleOp { Op op; std::size_t lvl; u32 seg; };
-    struct TailSeg { u32 first, count, out_buf; };
+    struct TailSeg { u32 first, count, out_buf; int mat; };   // mat: its matrix in tail_mats, -1: k_tail
     std::vector<CycleOp> cycle_ops;
     std::vector<TailSeg> tail_segs;
     DevMem tail_ops;
+    std::vector<std::unique_ptr<DevMem>> tail_mats;
+
+    // The matrices of the tail's segments (mg::k_tail_apply), one for all segments with the same
+    // steps (a V-cycle has one segment, a W-cycle many of a few kinds).  Measured per segment (3D Q1
+    // L7 / 2D Q2 L9 in FP32, 2D Q1 L6 / 3D Q1 L7 in FP64): 4.7 / 4.1 / 4.4 / 4.8 us, with k_tail 34 /
+    // 55 / 67 / 99 us; forming a matrix takes 0.1 ms (729 rows, FP32) to 0.4 ms.  Tails of more than
+    // kTailMatRows rows (option tail_max_n; 4225 rows in FP32 would read 71 MB per segment, as long as
+    // k_tail takes) and further kinds beyond eight run k_tail.
+    int build_tail_mats(const std::vector<u32>& ops)
+    {
+      tail_mats.clear();
+      const u64 n = L[tail0]->n;
+      if(n > mg::kTailMatRows) return rt::kOk;
+      std::vector<const TailSeg*> kinds;
+      auto same = [&](const TailSeg& a, const TailSeg& b) {
+        return a.count == b.count && a.out_buf == b.out_buf &&
+               std::equal(ops.begin() + a.first, ops.begin() + a.first + a.count, ops.begin() + b.first);
+      };
+      if(tail_lds > 65536)
+        F3_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&mg::k_tail<DT, VT, true>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(tail_lds)));
+      for(TailSeg& g : tail_segs)
+      {
+        std::size_t k = 0;
+        while(k < kinds.size() && !same(*kinds[k], g)) ++k;
+        if(k == kinds.size())
+        {
+          if(k == 8) continue;
+          std::unique_ptr<DevMem> m(new DevMem());
+          F3_RC(m->alloc(sizeof(DT) * n * n));
+          mg::k_tail<DT, VT, true><<<unsigned(n), mg::kTailThreads, tail_lds, s>>>(tail, tail_ops.template as<u32>() + g.first,
+                                                                                   g.count, g.out_buf, nullptr, m->template as<DT>());
+          F3_RC(rt::check_launch());
+          tail_mats.push_back(std::move(m));
+          kinds.push_back(&g);
+        }
+        g.mat = int(k);
+      }
+      return rt::kOk;
+    }
 
     // the whole cycle over every level, the coarse solve at the coarsest
     std::vector<CycleOp> cycle_schedule() const
@@ -1944,7 +1984,7 @@ namespace
           if(!open)
           {
             cycle_ops.push_back(CycleOp{Op::bottom, tail0, u32(tail_segs.size())});
-            tail_segs.push_back(TailSeg{u32(ops.size()), 0, 0});
+            tail_segs.push_back(TailSeg{u32(ops.size()), 0, 0, -1});
             tin[tail0] = 0;
             open = true;
           }
@@ -1965,7 +2005,8 @@ namespace
         if(!ops.empty())
         {
           F3_CHECK(hipMemcpyAsync(tail_ops.p, ops.data(), sizeof(u32) * ops.size(), hipMemcpyHostToDevice, s));
-          F3_CHECK(hipStreamSynchronize(s));
+          F3_RC(build_tail_mats(ops));
+          F3_CHECK(hipStreamSynchronize(s));   // ops leaves scope
         }
       }
       // the top level's iterate must end in its xfinal buffer, which the PCG reads: follow it
@@ -2033,7 +2074,10 @@ namespace
             break;
           }
           case Op::bottom:
-            if(tail0 + 1 < nl)
+            if(tail0 + 1 < nl && tail_segs[c.seg].mat >= 0)
+              mg::k_tail_apply<DT><<<unsigned((f.n + 3) / 4), kBlock, 0, s>>>(u32(f.n), tail_mats[tail_segs[c.seg].mat]->template as<DT>(),
+                                                                             f.rhs.template as<DT>(), f.xfinal, status);
+            else if(tail0 + 1 < nl)
             {
               const TailSeg& g = tail_segs[c.seg];
               mg::k_tail<DT, VT><<<1, mg::kTailThreads, tail_lds, s>>>(tail, tail_ops.template as<u32>() + g.first, g.count,
@@ -2073,8 +2117,8 @@ namespace
     // Cycles are launched operation by operation, with an event wherever the level or the
     // category changes (a run of smoothing steps on one level is one span): an event costs the
     // stream a few microseconds, as much as a small level's operation, so one per operation
-    // would inflate the coarse levels' times.  The solve itself is not touched (its graphs
-    // record no events).
+    // would inflate the coarse levels' times.  The span times are scaled to the duration of the
+    // cycle without events.  The solve itself is not touched (its graphs record no events).
     std::vector<hipEvent_t> stat_ev;
     static int op_category(Op op)
     {
@@ -2117,20 +2161,30 @@ namespace
       std::vector<double> t(4 * nl, 0.0), cnt(4 * nl, 0.0), by(nl, 0.0), fl(nl, 0.0);
       F3_RC(enqueue_vcycle(r.template as<double>(), nullptr));   // warm-up
       F3_CHECK(hipStreamSynchronize(s));
-      double total = 0.0;
+      // the cycle as it runs, and then with the events; the spans' times are scaled to the former, so
+      // that they add up to the cycle without the events' own cost
+      float plain = 0.f;
+      F3_CHECK(hipEventRecord(t0, s));
+      for(int rep = 0; rep < reps; ++rep) F3_RC(enqueue_vcycle(r.template as<double>(), nullptr));
+      F3_CHECK(hipEventRecord(t1, s));
+      F3_CHECK(hipStreamSynchronize(s));
+      F3_CHECK(hipEventElapsedTime(&plain, t0, t1));
+      const double total = double(plain);
+      double with_events = 0.0;
       for(int rep = 0; rep < reps; ++rep)
       {
         F3_RC(enqueue_vcycle(r.template as<double>(), nullptr, &stat_ev, &span_start));
         F3_CHECK(hipStreamSynchronize(s));
         float ms = 0.f;
-        F3_CHECK(hipEventElapsedTime(&ms, stat_ev[0], stat_ev[nspan]));
-        total += ms;
         for(std::size_t k = 0; k < nspan; ++k)
         {
           F3_CHECK(hipEventElapsedTime(&ms, stat_ev[k], stat_ev[k + 1]));
           t[span_slot[k]] += double(ms);
+          with_events += double(ms);
         }
       }
+      if(with_events > 0.0)
+        for(double& v : t) v *= total / with_events;
       // counts, bytes and flops of the cycle's mathematical operations (the full schedule, tail
       // levels included)
       const u64 vb = sizeof(DT);

@@ -19,6 +19,7 @@
 
 #include "device_common.hpp"
 #include "mg_kernels.hpp"
+#include "lattice_kernels.hpp"
 #include "runtime.hpp"
 #include "feat3_hip.h"
 
@@ -418,6 +419,7 @@ namespace
     u32 tmo[3] = {1, 1, 1}, tmi[3] = {1, 1, 1};
     u32 tw_bytes = 0;
     u32 tk = 0;   // the largest number of entries of a factor row
+    int tdeg = 0; // a prolongation whose factors are exactly those of the Q1 (1) or Q2 (2) space, else 0
     DevMem tcnt[3], tidx[3], tw[3];
 
     // thin >= 0: upload a compact copy with the entries band_keeps(v, row diagonal, thin) only:
@@ -1072,6 +1074,45 @@ namespace
     }
   };
 
+  // 1 or 2 if the 1D prolongation factors of every axis are exactly those of the Q1 / Q2 space on
+  // the bisected line (what mg::lat evaluates without tables), else 0
+  template<typename DT>
+  int transfer_degree(const u32 mo[3], const u32 mi[3], const std::vector<u32> cnt[3], const std::vector<u32> idx[3],
+                      const std::vector<DT> w[3], int dim)
+  {
+    constexpr u32 W = mg::kTensorW;
+    for(int deg = 1; deg <= 2; ++deg)
+    {
+      bool ok = true;
+      for(int a = 0; a < dim && ok; ++a)
+      {
+        ok = mo[a] == mo[0] && mi[a] == mi[0] && mo[a] == 2 * mi[a] - 1 && (mi[a] - 1) % u32(deg) == 0;
+        for(u32 i = 0; i < mo[a] && ok; ++i)
+        {
+          u32 c[3] = {0, 0, 0}, n = 0;
+          DT v[3] = {DT(0), DT(0), DT(0)};
+          if(deg == 1)
+          {
+            c[0] = i / 2; v[0] = DT((i & 1u) ? 0.5 : 1.0); n = 1;
+            if(i & 1u) { c[1] = i / 2 + 1; v[1] = DT(0.5); n = 2; }
+          }
+          else if((i & 1u) == 0u) { c[0] = i / 2; v[0] = DT(1); n = 1; }
+          else
+          {
+            for(u32 k = 0; k < 3; ++k) c[k] = 2 * (i / 4) + k;
+            const bool first = (i & 3u) == 1u;
+            v[0] = DT(first ? 0.375 : -0.125); v[1] = DT(0.75); v[2] = DT(first ? -0.125 : 0.375);
+            n = 3;
+          }
+          ok = cnt[a][i] == n;
+          for(u32 k = 0; k < n && ok; ++k) ok = idx[a][u64(i) * W + k] == c[k] && w[a][u64(i) * W + k] == v[k];
+        }
+      }
+      if(ok) return deg;
+    }
+    return 0;
+  }
+
   // Tensor-product structure of a transfer pair on structured hierarchies.  P (fine x coarse)
   // of a Q1/Q2 hierarchy on the unit square or cube, numbered lexicographically on its node
   // lattice (the solver's lattice order), is Pz (x) Py (x) Px with 1D factors of 1-3 entries per
@@ -1178,6 +1219,7 @@ namespace
       F3_RC(R.template set_tensor<DT>(mi, mo, rcnt, ridx, rw, s, &ok));
       if(!ok) return rt::kOk;
       P.tensor = R.tensor = true;
+      P.tdeg = transfer_degree<DT>(mo, mi, cnt, idx, w, d);
       return rt::kOk;
     }
     return rt::kOk;
@@ -1438,6 +1480,9 @@ namespace
     // (0: they run regardless; the PCG kernels behind them still check it, so the results are the
     // same, and a cycle launched after the last iteration does its work for nothing)
     bool vcycle_status = true;
+    // levels on a lattice smoothed in bricks, several steps per launch (lattice_kernels.hpp); 0:
+    // one launch per step on the level's format
+    bool lattice = true;
     // launch shape of the transfer matrices: lanes per row (-1: as the level matrices) and row
     // positions per block (0: derived from the row count).  128 rows per block (more, smaller
     // blocks than the default grid on the mid-size levels) measured V-cycle 3D Q1 L7 584 -> 580 us,
@@ -1486,6 +1531,12 @@ namespace
     DevCsr<VT> A, P, R;
     DevMem mask, dinv, rhs, x, t, def;
     DT* xfinal = nullptr; // buffer holding this level's solution after its post-smoothing
+    // smoothing in bricks: the kind of brick (-1: none), nodes per axis, the matrix values (one row
+    // in k, d; a table per class or [tap][node] in coef)
+    int lat = -1;
+    u32 m = 0;
+    DT k[27] = {}, d = DT(0);
+    DevMem coef;
   };
 
   template<typename DT, typename VT>
@@ -1639,6 +1690,7 @@ namespace
       }
       L.back()->xfinal = L.back()->x.template as<DT>();
       F3_RC(setup_tail(lv));
+      for(std::size_t i = 0; cfg.lattice && i < tail0; ++i) F3_RC(setup_lattice(*L[i]));
       F3_RC(build_cycle());
 
       // outer PCG
@@ -1821,7 +1873,7 @@ namespace
     // _apply_prol and _apply_smooth_peak).  The operations on the levels of the coarse tail
     // (tail0 and below) are grouped into segments that one k_tail launch each runs; a bottom
     // operation stands for the coarse solve (k_coarse) or for such a segment.
-    enum class Op : int { entry, sweep, defect, rest, rest_step, bottom, prol, copy_top };
+    enum class Op : int { entry, sweep, defect, rest, rest_step, bottom, prol };
     struct CycleOp { Op op; std::size_t lvl; u32 seg; };
     struct TailSeg { u32 first, count, out_buf; int mat; };   // mat: its matrix in tail_mats, -1: k_tail
     std::vector<CycleOp> cycle_ops;
@@ -2009,19 +2061,324 @@ namespace
           F3_CHECK(hipStreamSynchronize(s));   // ops leaves scope
         }
       }
-      // the top level's iterate must end in its xfinal buffer, which the PCG reads: follow it
-      // through the upper operations (a bottom operation on level 0 writes xfinal itself)
-      int where = 0;   // 0: x, 1: t, 2: xfinal
-      for(const CycleOp& c : cycle_ops)
-      {
-        if(c.lvl != 0) continue;
-        if(c.op == Op::entry) where = 0;
-        else if(c.op == Op::sweep && where != 2) where ^= 1;
-        else if(c.op == Op::bottom) where = 2;
-      }
-      if(where != 2 && (where == 1) != (L[0]->xfinal == L[0]->t.template as<DT>()))
-        cycle_ops.push_back(CycleOp{Op::copy_top, 0, 0});
+      build_plan();
       return rt::kOk;
+    }
+
+    // ---- levels smoothed in bricks (lattice_kernels.hpp) ----------------------------------
+    // kinds of bricks: 0 3D Q1 with all taps, 1 without the face neighbours (FP32 copies), 2 2D Q1
+    // with one row of values, 3 2D Q1 with a row per node, 4 2D Q2 with a row per parity class
+    template<typename F>
+    int with_brick(int kind, F&& f)
+    {
+      switch(kind)
+      {
+        case 0: return f(lat::Brick<DT, 3, 1, 0, 16, 16, 16, 4, lat::kTapsAll>());
+        case 1:
+          if constexpr(sizeof(DT) == 4) return f(lat::Brick<DT, 3, 1, 0, 16, 16, 16, 4, lat::kTapsNoFaces>());
+          else return rt::kErrState;
+        case 2: return f(lat::Brick<DT, 2, 1, 0, 64, 32, 1, 2, lat::kTapsAll>());
+        case 3: return f(lat::Brick<DT, 2, 1, 2, 64, 32, 1, 2, lat::kTapsAll>());
+        case 4: return f(lat::Brick<DT, 2, 2, 1, 64, 32, 1, 4, lat::kTapsAll>());
+        default: return rt::kErrState;
+      }
+    }
+
+    // Decides whether a level is smoothed in bricks: its prolongation is that of a Q1 or 2D Q2 space
+    // on a lattice (checked entry by entry when its factors were built), its matrix couples only the
+    // nodes of a box, and all inner rows of a class are the same bit for bit with the Dirichlet nodes
+    // the lattice's boundary -- or, 2D Q1, any values.  Everything else keeps its format's kernels.
+    int setup_lattice(Level<DT, VT>& l)
+    {
+      l.lat = -1;
+      if(!l.P.tensor || l.P.tdeg == 0 || l.n >= (u64(1) << 31)) return rt::kOk;
+      const int dim = l.P.tmo[2] > 1 ? 3 : 2, rad = l.P.tdeg;
+      const u32 m = l.P.tmo[0];
+      if((dim == 3 && rad != 1) || m < 9) return rt::kOk;
+      const int nl = 2 * rad + 1, ntap = dim == 3 ? nl * nl * nl : nl * nl, per = rad == 2 ? 2 : 1, ncls = per == 2 ? 4 : 1;
+      // the row of an inner node of every class
+      std::vector<DT> rep(std::size_t(ncls) * ntap, DT(0)), repd(ncls, DT(0));
+      bool finite = true;
+      for(int c = 0; c < ncls; ++c)
+      {
+        const u64 x = 4 + u64(c & 1), y = 4 + u64(c >> 1), z = dim == 3 ? 4 : 0, r = (z * m + y) * m + x;
+        u32 e[2];
+        F3_CHECK(hipMemcpy(e, l.A.rp.template as<u32>() + r, sizeof(e), hipMemcpyDeviceToHost));
+        if(e[1] - e[0] > 64) return rt::kOk;
+        std::vector<u32> col(e[1] - e[0]);
+        std::vector<VT> val(e[1] - e[0]);
+        if(!col.empty())
+        {
+          F3_CHECK(hipMemcpy(col.data(), l.A.col.template as<u32>() + e[0], sizeof(u32) * col.size(), hipMemcpyDeviceToHost));
+          F3_CHECK(hipMemcpy(val.data(), l.A.val.template as<VT>() + e[0], sizeof(VT) * val.size(), hipMemcpyDeviceToHost));
+        }
+        F3_CHECK(hipMemcpy(&repd[c], l.dinv.template as<DT>() + r, sizeof(DT), hipMemcpyDeviceToHost));
+        for(std::size_t k = 0; k < col.size(); ++k)
+        {
+          const int dx = int(col[k] % m) - int(x), dy = int(col[k] / m % m) - int(y), dz = int(col[k] / (m * m)) - int(z);
+          if(std::abs(dx) > rad || std::abs(dy) > rad || std::abs(dz) > (dim == 3 ? rad : 0)) return rt::kOk;
+          const DT v = DT(val[k]);
+          finite = finite && std::isfinite(double(v));
+          rep[std::size_t(c) * ntap + ((dim == 3 ? dz + rad : 0) * nl + dy + rad) * nl + dx + rad] = v;
+        }
+        finite = finite && std::isfinite(double(repd[c]));
+      }
+      DevMem drep, drepd, dflag;
+      F3_RC(drep.alloc(sizeof(DT) * rep.size()));
+      F3_RC(drepd.alloc(sizeof(DT) * repd.size()));
+      F3_RC(dflag.alloc(sizeof(int)));
+      F3_CHECK(hipMemcpyAsync(drep.p, rep.data(), sizeof(DT) * rep.size(), hipMemcpyHostToDevice, s));
+      F3_CHECK(hipMemcpyAsync(drepd.p, repd.data(), sizeof(DT) * repd.size(), hipMemcpyHostToDevice, s));
+      F3_CHECK(hipMemsetAsync(dflag.p, 0, sizeof(int), s));
+      lat::k_lattice_check<DT, VT><<<setup_blocks(l.n), 256, 0, s>>>(
+        l.n, m, dim, rad, per, l.A.rp.template as<u32>(), l.A.col.template as<u32>(), l.A.val.template as<VT>(),
+        l.mask.template as<u32>(), l.dinv.template as<DT>(), drep.template as<DT>(), drepd.template as<DT>(), ntap,
+        dflag.template as<int>());
+      F3_RC(rt::check_launch());
+      int flag = 3;
+      F3_CHECK(hipMemcpyAsync(&flag, dflag.p, sizeof(int), hipMemcpyDeviceToHost, s));
+      F3_CHECK(hipStreamSynchronize(s));
+      if(flag & 1) return rt::kOk;
+      if(!finite || (flag & 2))
+      {
+        // a row per node: 2D Q1
+        if(dim != 2 || rad != 1) return rt::kOk;
+        F3_RC(l.coef.alloc(sizeof(DT) * l.n * u64(ntap)));
+        F3_CHECK(hipMemsetAsync(l.coef.p, 0, sizeof(DT) * l.n * u64(ntap), s));
+        lat::k_lattice_scatter<DT, VT><<<setup_blocks(l.n), 256, 0, s>>>(l.n, m, rad, l.A.rp.template as<u32>(),
+                                                                        l.A.col.template as<u32>(), l.A.val.template as<VT>(),
+                                                                        l.coef.template as<DT>());
+        F3_RC(rt::check_launch());
+        F3_CHECK(hipStreamSynchronize(s));
+        l.lat = 3;
+      }
+      else if(per == 2)
+      {
+        std::vector<DT> tab;
+        for(int c = 0; c < 4; ++c)
+        {
+          tab.insert(tab.end(), rep.begin() + c * ntap, rep.begin() + (c + 1) * ntap);
+          tab.push_back(repd[c]);
+        }
+        F3_RC(l.coef.alloc(sizeof(DT) * tab.size()));
+        F3_CHECK(hipMemcpy(l.coef.p, tab.data(), sizeof(DT) * tab.size(), hipMemcpyHostToDevice));
+        l.lat = 4;
+      }
+      else
+      {
+        for(int t = 0; t < ntap; ++t) l.k[t] = rep[t];
+        l.d = repd[0];
+        l.lat = dim == 2 ? 2 : 0;
+        if(dim == 3 && sizeof(DT) == 4)
+        {
+          bool faces = false;
+          for(int t = 0; t < ntap; ++t) faces = faces || (!((lat::kTapsNoFaces >> t) & 1u) && rep[t] != DT(0));
+          l.lat = faces ? 0 : 1;
+        }
+      }
+      l.m = m;
+      return with_brick(l.lat, [&](auto b) -> int {
+        typedef decltype(b) B;
+        if(B::LDS > 65536)
+          F3_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&lat::k_lattice<B>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, B::LDS));
+        return rt::kOk;
+      });
+    }
+
+    // tile extents, halo and block count of a launch of `sweeps` steps; false: the halo leaves no tile
+    struct LatTiles { int t[3]; int hl; u32 nb[3]; u64 blocks; };
+    template<typename B>
+    static bool lat_tiles(u32 m, int sweeps, bool rest, LatTiles& g)
+    {
+      int lo = sweeps * B::RAD + (rest ? B::RAD + B::RLO : 0);
+      const int hi = sweeps * B::RAD + (rest ? B::RAD + B::RHI : 0);
+      if(B::MODE == 1) lo = (lo + 1) / 2 * 2;   // columns start at an even node
+      const int ext[3] = {B::BX, B::BY, B::BZ};
+      g.hl = lo;
+      g.blocks = 1;
+      for(int a = 0; a < 3; ++a)
+      {
+        g.t[a] = a < B::DIM ? (ext[a] - lo - hi) / 2 * 2 : 1;
+        if(g.t[a] < (a < B::DIM ? 2 : 1)) return false;
+        g.nb[a] = a < B::DIM ? (m + u32(g.t[a]) - 1) / u32(g.t[a]) : 1u;
+        g.blocks *= g.nb[a];
+      }
+      return true;
+    }
+
+    // estimated time (us) of a launch: a launch's fixed cost, then the blocks' loads and steps at
+    // one block's rate per CU
+    template<typename B>
+    static double lat_cost(u32 m, int sweeps, bool rest)
+    {
+      LatTiles g;
+      if(!lat_tiles<B>(m, sweeps, rest, g)) return 1e30;
+      const double reads = double(B::NC) * (B::CZ + 2 * B::RAD) / B::CZ * (sizeof(DT) / 4);
+      const double step = B::PTS / 64.0 * reads * 2.0 / 2400.0;   // LDS cycles of a step
+      const double load = 0.3 + B::PTS * 3e-4 * (sizeof(DT) / 4) * (B::MODE == 2 ? 3 : 1);
+      const double block = load + (sweeps + (rest ? 1 : 0)) * step;
+      return 3.5 + std::max(1.5 * block, double(g.blocks) / 256.0 * block);
+    }
+
+    // One entry of the cycle as it is launched: an operation, or (lat) the operations of one level
+    // from its entry to its restriction or next operation elsewhere, taken in bricks
+    struct PlanOp
+    {
+      CycleOp c;
+      bool lat;
+      int in, sweeps;
+      bool rest, step;   // step: the restriction takes the next level's first step
+    };
+    std::vector<PlanOp> plan;
+
+    // groups the operations of the lattice levels; a run of steps is split into the launches of the
+    // least estimated time (lat_cost): all in one on the small levels, where the launches count, few
+    // per launch on the large ones, where the halos do
+    void build_plan()
+    {
+      plan.clear();
+      const std::size_t nl = L.size();
+      std::vector<char> zero(nl, 0);   // the level's first step from zero is left to its first launch
+      for(std::size_t k = 0; k < cycle_ops.size();)
+      {
+        const CycleOp c = cycle_ops[k];
+        if(c.lvl >= nl || L[c.lvl]->lat < 0 || c.op == Op::bottom)
+        {
+          plan.push_back(PlanOp{c, false, 0, 0, false, false});
+          ++k;
+          continue;
+        }
+        const std::size_t i = c.lvl;
+        int in = lat::kMem, sweeps = 0;
+        if(c.op == Op::entry) { in = lat::kEntry; ++k; }
+        else if(c.op == Op::prol) { in = lat::kProl; ++k; }
+        else if(zero[i]) in = lat::kZero;
+        zero[i] = 0;
+        while(k < cycle_ops.size() && cycle_ops[k].op == Op::sweep && cycle_ops[k].lvl == i) { ++sweeps; ++k; }
+        bool rest = false, step = false;
+        if(k + 1 < cycle_ops.size() && cycle_ops[k].op == Op::defect && cycle_ops[k].lvl == i)
+        {
+          rest = true;
+          step = cycle_ops[k + 1].op == Op::rest_step;
+          if(step && L[i + 1]->lat >= 0) { step = false; zero[i + 1] = 1; }
+          k += 2;
+        }
+        // the split: best[s] = least cost of the last s steps (the restriction in the last launch)
+        std::vector<double> best(sweeps + 1, 1e30);
+        std::vector<int> first(sweeps + 1, 0);
+        for(int q = 0; q <= sweeps; ++q)
+          for(int n = q ? 1 : 0; n <= q; ++n)
+          {
+            const bool last = n == q;
+            double t = 1e30;
+            (void)with_brick(L[i]->lat, [&](auto b) -> int { t = lat_cost<decltype(b)>(L[i]->m, n, last && rest); return 0; });
+            if(!last) t += best[q - n];
+            // (a launch of the restriction alone behind the last step)
+            else if(rest && q > 0)
+            {
+              double t0 = 1e30;
+              (void)with_brick(L[i]->lat, [&](auto b) -> int { t0 = lat_cost<decltype(b)>(L[i]->m, n, false); return 0; });
+              if(t0 + best[0] < t) t = t0 + best[0];
+            }
+            if(t < best[q]) { best[q] = t; first[q] = n; }
+          }
+        for(int q = sweeps; q > 0 || in >= 0;)
+        {
+          const int n = first[q];
+          bool with_rest = rest && n == q;
+          if(with_rest && q > 0)
+          {
+            double t = 1e30, t0 = 1e30;
+            (void)with_brick(L[i]->lat, [&](auto b) -> int {
+              t = lat_cost<decltype(b)>(L[i]->m, n, true);
+              t0 = lat_cost<decltype(b)>(L[i]->m, n, false);
+              return 0;
+            });
+            with_rest = t <= t0 + best[0];
+          }
+          plan.push_back(PlanOp{CycleOp{Op::sweep, i, 0}, true, in, n, with_rest, with_rest && step});
+          q -= n;
+          if(q == 0 && rest && !with_rest) plan.push_back(PlanOp{CycleOp{Op::sweep, i, 0}, true, lat::kMem, 0, true, step});
+          in = -1;
+          if(q > 0) in = lat::kMem;
+        }
+      }
+      // the buffer in which the top level's iterate ends is the one the PCG reads
+      if(tail0 > 0 || tail0 + 1 >= nl)
+      {
+        int where = 0;   // 0: x, 1: t
+        for(const PlanOp& o : plan)
+        {
+          if(o.c.lvl != 0) continue;
+          if(o.lat) { if(o.in == lat::kZero || o.in == lat::kEntry) where = 0; else if(o.sweeps > 0 || o.in == lat::kProl) where ^= 1; }
+          else if(o.c.op == Op::entry) where = 0;
+          else if(o.c.op == Op::sweep) where ^= 1;
+          else if(o.c.op == Op::bottom) where = L[0]->xfinal == L[0]->t.template as<DT>() ? 1 : 0;
+        }
+        L[0]->xfinal = where ? L[0]->t.template as<DT>() : L[0]->x.template as<DT>();
+      }
+    }
+
+    int launch_lattice(std::size_t i, const PlanOp& o, const double* def, std::vector<DT*>& cur, std::vector<DT*>& oth, const int* status)
+    {
+      Level<DT, VT>& f = *L[i];
+      return with_brick(f.lat, [&](auto b) -> int {
+        typedef decltype(b) B;
+        LatTiles g;
+        if(!lat_tiles<B>(f.m, o.sweeps, o.rest, g) || g.blocks >= (u64(1) << 31)) return rt::kErrState;
+        lat::Args<DT> a{};
+        a.m = f.m;
+        a.nbx = g.nb[0]; a.nby = g.nb[1];
+        for(int k = 0; k < 3; ++k) a.t[k] = g.t[k];
+        a.hl = g.hl;
+        a.in = o.in;
+        a.sweeps = o.sweeps;
+        a.restrict_ = o.rest ? 1 : 0;
+        a.rhs = f.rhs.template as<DT>();
+        a.rhs_out = f.rhs.template as<DT>();
+        a.def = def;
+        a.dinv = f.dinv.template as<DT>();
+        a.mask = f.mask.template as<u32>();
+        a.coef = f.coef.template as<DT>();
+        a.status = status;
+        for(int k = 0; k < 27; ++k) a.k[k] = f.k[k];
+        a.d = f.d;
+        if(o.in == lat::kZero || o.in == lat::kEntry)
+        {
+          cur[i] = f.x.template as<DT>();
+          oth[i] = f.t.template as<DT>();
+          a.write_x = 1;
+          a.xout = cur[i];
+        }
+        else
+        {
+          a.x = cur[i];
+          if(o.sweeps > 0 || o.in == lat::kProl)
+          {
+            a.write_x = 1;
+            a.xout = oth[i];
+            std::swap(cur[i], oth[i]);
+          }
+        }
+        if(o.in == lat::kProl || o.rest)
+        {
+          Level<DT, VT>& c = *L[i + 1];
+          a.mc = f.P.tmi[0];
+          if(o.in == lat::kProl) a.xc = cur[i + 1];
+          a.mask_c = c.mask.template as<u32>();
+          a.rhs_c = c.rhs.template as<DT>();
+          a.dinv_c = c.dinv.template as<DT>();
+          if(o.step)
+          {
+            a.x_c = c.x.template as<DT>();
+            cur[i + 1] = a.x_c;
+            oth[i + 1] = c.t.template as<DT>();
+          }
+        }
+        lat::k_lattice<B><<<unsigned(g.blocks), B::NT, B::LDS, s>>>(a);
+        return rt::kOk;
+      });
     }
 
     // evs (statistics only): an event is recorded before every operation k with span_start[k]
@@ -2033,12 +2390,18 @@ namespace
       const std::size_t nl = L.size();
       std::vector<DT*> cur(nl, nullptr), oth(nl, nullptr);
       std::size_t k = 0, e = 0;
-      for(const CycleOp& c : cycle_ops)
+      for(const PlanOp& o : plan)
       {
+        const CycleOp& c = o.c;
         const std::size_t i = c.lvl;
         Level<DT, VT>& f = *L[i];
         if(evs && (*span_start)[k]) F3_CHECK(hipEventRecord((*evs)[e++], s));
         ++k;
+        if(o.lat)
+        {
+          F3_RC(launch_lattice(i, o, def, cur, oth, status));
+          continue;
+        }
         switch(c.op)
         {
           case Op::entry:
@@ -2094,10 +2457,6 @@ namespace
                                                         status);
             }));
             break;
-          case Op::copy_top:
-            mg::k_copy_vec<DT><<<stream_blocks(f.n), kBlock, 0, s>>>(f.n, cur[0], f.xfinal, status);
-            std::swap(cur[0], oth[0]);
-            break;
         }
       }
       if(evs) F3_CHECK(hipEventRecord((*evs)[e], s));
@@ -2109,8 +2468,9 @@ namespace
     // Per level: time of smoothing, defect, grid transfer (restriction and prolongation, counted
     // on the finer level as the reference does) and coarse solve per cycle, the number of each
     // operation per cycle, and the cycle's algorithmic bytes and flops on that level.  Fused
-    // operations count where their main work is: the entry (conversion + first step) and the top
-    // copy as smoothing on level 0, a restriction with the next level's first smoothing step as
+    // operations count where their main work is: the entry (conversion + first step) as smoothing
+    // on level 0, a brick launch (lattice_kernels.hpp) with the transfers and the defect in it as
+    // smoothing of its level, a restriction with the next level's first smoothing step as
     // transfer (its step is counted as a smoothing step of the coarser level), and a segment of
     // the single-workgroup coarse tail as the coarse solve of the tail's top level (one kernel:
     // the levels inside it report counts, bytes and flops, their time is that of the segment).
@@ -2124,7 +2484,7 @@ namespace
     {
       switch(op)
       {
-        case Op::entry: case Op::sweep: case Op::copy_top: return 0;   // smoothing
+        case Op::entry: case Op::sweep: return 0;   // smoothing
         case Op::defect: return 1;
         case Op::rest: case Op::rest_step: case Op::prol: return 2;     // grid transfer
         case Op::bottom: return 3;                                       // coarse solve
@@ -2133,7 +2493,7 @@ namespace
     }
     int statistics(int reps, double* out, int cap) override
     {
-      const std::size_t nl = L.size(), nops = cycle_ops.size();
+      const std::size_t nl = L.size(), nops = plan.size();
       const int need = 3 + 10 * int(nl);
       if(reps < 1 || !out || cap < need) return rt::kErrArg;
       // spans: maximal runs of operations with the same level and category
@@ -2141,7 +2501,7 @@ namespace
       std::vector<std::size_t> span_slot;   // 4 * level + category of each span
       for(std::size_t k = 0; k < nops; ++k)
       {
-        const std::size_t slot = 4 * cycle_ops[k].lvl + std::size_t(op_category(cycle_ops[k].op));
+        const std::size_t slot = 4 * plan[k].c.lvl + std::size_t(op_category(plan[k].c.op));
         if(k == 0 || slot != span_slot.back())
         {
           span_start[k] = 1;
@@ -2213,7 +2573,6 @@ namespace
           case Op::bottom:
             cnt[4 * i + 3] += 1; by[i] += double(ncoarse * ncoarse * 8) + n * vb * 2; fl[i] += 2 * double(ncoarse * ncoarse);
             break;
-          case Op::copy_top: break;
         }
       }
       out[0] = double(nl);
@@ -2524,13 +2883,12 @@ namespace
       v[2] = L.front()->A.nnz;
       v[3] = u64(L.front()->A.lanes);
       v[4] = L.front()->A.sell_size;
-      u64 kern = 0, bytes = 0;
+      u64 bytes = 0;
       const u64 vb = sizeof(DT);
       for(const CycleOp& c : cycle_ops)
       {
         const Level<DT, VT>& f = *L[c.lvl];
         const u64 nc = c.lvl + 1 < L.size() ? L[c.lvl + 1]->n : 0;
-        ++kern;
         switch(c.op)
         {
           case Op::entry: bytes += f.n * (8 + vb * 3); break;
@@ -2540,10 +2898,9 @@ namespace
           case Op::rest_step: bytes += f.R.matrix_bytes() + f.n * vb + nc * vb * 4; break;
           case Op::bottom: bytes += ncoarse * ncoarse * 8 + ncoarse * vb * 2; break;
           case Op::prol: bytes += f.P.matrix_bytes() + nc * vb + f.n * vb * 2; break;
-          case Op::copy_top: bytes += f.n * vb * 2; break;
         }
       }
-      v[5] = kern;
+      v[5] = plan.size();
       v[6] = bytes;
       v[7] = outer_matrix().matrix_bytes() + n0 * 8 * 2 + n0 * 8 * 5 + n0 * (8 + vb) * 2 + n0 * (8 + vb * 2);
       v[8] = sizeof(DT);
@@ -2897,6 +3254,7 @@ int feat3_mgpcg_set_option(feat3_mgpcg* h, const char* name, double value)
   else if(k == "transfer_rows_per_block" && value >= 0) h->cfg.transfer_rows_per_block = u64(value);
   else if(k == "symmetric_band") h->cfg.symmetric_band = value != 0.0;
   else if(k == "band_dict") h->cfg.band_dict = value != 0.0;
+  else if(k == "lattice") h->cfg.lattice = value != 0.0;
   else if(k == "lane_shift") h->cfg.lane_shift = value != 0.0;
   else if(k == "plane_order" && (value == 0 || value == 1 || value == 2)) h->cfg.plane_order = int(value);
   else if(k == "band_stage_x" && (value == 0 || value == 1 || value == 2)) h->cfg.band_stage_x = int(value);

@@ -1,0 +1,96 @@
+"""Lattice levels smoothed in bricks (lattice_kernels.hpp, option lattice) against one launch per step
+on the banded format (lattice = 0): the same row sums, steps and transfers in the same order, so cycles
+are equal bit for bit.  The levels' sizes put the bricks' tiles at their edges: lattices smaller than a
+tile, one node more than a multiple of it, and many tiles."""
+import numpy as np
+import pytest
+
+from feat3_amd import problems as pb
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def torch():
+    torch = pytest.importorskip("torch")
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+    return torch
+
+
+def cycles(torch, H, d, inner, lattice, n=2, fmt="banded", **kw):
+    from feat3_amd.solver import MGPCG
+    s = MGPCG(H, inner=inner, fmt=fmt, options={"lattice": lattice, "tail_max_n": kw.pop("tail", 30)}, **kw).init()
+    dd = torch.from_numpy(d).cuda()
+    c = torch.empty_like(dd)
+    for _ in range(n):      # a second cycle starts from the first one's buffers
+        s.vcycle(c, dd)
+    out, k = c.cpu().numpy(), s.info()["kernels_per_vcycle"]
+    s.done()
+    return out, k
+
+
+def defect(H, seed=3):
+    d = np.random.default_rng(seed).uniform(-1.0, 1.0, H.n)
+    d[H.levels[0].bnd] = 0.0
+    return d
+
+
+@pytest.mark.parametrize("inner", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("dim,deg,lvl", [(2, 1, 4), (2, 1, 6), (2, 1, 8), (2, 2, 4), (2, 2, 6), (3, 1, 3), (3, 1, 4), (3, 1, 5), (3, 1, 6)])
+def test_bricks_are_bitwise_the_steps(torch, dim, deg, lvl, inner):
+    H = pb.hierarchy(dim, deg, lvl, 1)
+    d = defect(H)
+    for cycle, pre, post in (("v", 4, 4), ("v", 1, 1), ("f", 2, 3), ("w", 3, 2)):
+        if cycle == "w" and lvl > 5:
+            continue
+        a, ka = cycles(torch, H, d, inner, 1, cycle=cycle, pre=pre, post=post)
+        b, kb = cycles(torch, H, d, inner, 0, cycle=cycle, pre=pre, post=post)
+        assert ka < kb, (ka, kb)
+        assert np.array_equal(a, b), (cycle, pre, post, np.abs(a - b).max())
+
+
+@pytest.mark.parametrize("inner", ["f64", "f32"])
+@pytest.mark.parametrize("lvl", [4, 7])
+def test_variable_coefficient_bricks(torch, lvl, inner):
+    """A row of values per node (no two alike)."""
+    k = np.exp(np.random.default_rng(7).uniform(-1.0, 1.0, 1 << (2 * lvl)))
+    H = pb.hierarchy(2, 1, lvl, 1, kcell=k)
+    d = defect(H)
+    a, ka = cycles(torch, H, d, inner, 1)
+    b, kb = cycles(torch, H, d, inner, 0)
+    assert ka < kb and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("dim,deg,lvl", [(2, 1, 6), (2, 2, 5), (3, 1, 4)])
+def test_changed_rows_are_not_taken_as_uniform(torch, dim, deg, lvl):
+    """One inner row with another diagonal, and Dirichlet nodes besides the boundary: 3D and Q2 levels keep
+    their steps (one kernel each), 2D Q1 levels take rows of their own; the cycles stay equal."""
+    H = pb.hierarchy(dim, deg, lvl, 1)
+    A = H.levels[0].A
+    rows = np.repeat(np.arange(A.rows), np.diff(A.row_ptr.astype(np.int64)))
+    mid = A.rows // 2
+    A.val[(A.col_ind == rows) & (rows == mid)] *= 1.5
+    d = defect(H)
+    a, ka = cycles(torch, H, d, "f64", 1)
+    b, kb = cycles(torch, H, d, "f64", 0)
+    assert np.array_equal(a, b)
+    G = pb.hierarchy(dim, deg, lvl, 1)
+    G.levels[0].bnd = np.union1d(G.levels[0].bnd, np.array([mid + 1], np.uint32)).astype(np.uint32)
+    d = defect(G)
+    a, ka = cycles(torch, G, d, "f32", 1)
+    b, kb = cycles(torch, G, d, "f32", 0)
+    assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("fmt", ["csr", "sell"])
+@pytest.mark.parametrize("inner", ["f64", "f32"])
+def test_other_formats_agree(torch, fmt, inner):
+    """The general formats round their products before adding them, the bricks do not: a row sum of w = 27
+    terms differs by at most w eps of its absolute terms, the cycle by a few times that."""
+    H = pb.hierarchy(3, 1, 4, 1)
+    d = defect(H)
+    a, _ = cycles(torch, H, d, inner, 1, fmt=fmt)
+    b, _ = cycles(torch, H, d, inner, 0, fmt=fmt)
+    eps = np.finfo(np.float64 if inner == "f64" else np.float32).eps
+    assert np.linalg.norm(a - b) <= 27 * eps * np.linalg.norm(b)

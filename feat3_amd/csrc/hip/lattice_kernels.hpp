@@ -413,12 +413,230 @@ namespace lat
     }
   }
 
+  // ---- large 3D levels: one step per launch, columns in registers ------------------------------
+  //
+  // On a large 3D lattice the bricks' halos cost more than the launches they save (129^3 nodes, FP32:
+  // 29.5 us for two steps, 2.4 times the nodes).  Here a thread takes CX consecutive nodes of CZ
+  // planes: it loads each line of x it needs once (CX + 2 values by vector loads, 3 lines of CZ + 2
+  // planes), so a node costs 9 loaded values instead of 27, no halo is computed twice and the
+  // matrix row comes from scalar registers.  The lines of a plane are taken end to end (a group may
+  // run over a line's end; the nodes at line ends are boundary nodes, whose sums are not used).
+  // Blocks of one XCD take consecutive planes, whose x, rhs and result fit its L2.  Measured, 129^3
+  // nodes, value-coded band -> columns: FP32 step 13.6 -> 7.8 us (3 vectors, 25.8 MB: 3.3 TB/s), FP64
+  // step 35.4 -> 11.4 us and outer product 35.3 -> 11.8 us (51.5 and 34.3 MB); a copy of 1 GiB runs at
+  // 5.1 TB/s.  Shapes CX x CZ in FP32: 4x2 7.8, 2x4 7.8, 4x4 8.4, 4x8 11.3 us (few blocks, or few loads
+  // shared); FP64: 2x4 11.4, 2x2 11.6, 4x2 12.0, 2x8 13.9 us.
+  constexpr int kColThreads = 256;
+  template<typename DT_> struct ColShape { static constexpr int CX = sizeof(DT_) == 4 ? 4 : 2, CZ = sizeof(DT_) == 4 ? 2 : 4; };
+
+  enum ColOp : int { kColSweep = 0, kColDefect = 1, kColProduct = 2, kColInit = 3 };
+
+  template<typename DT_>
+  struct ColArgs
+  {
+    u32 m, mm, groups, gblocks;   // nodes per axis and plane, groups of CX nodes per plane, blocks per z chunk
+    u64 div;                      // mg::udiv_magic multiplier of m
+    const DT_* x;
+    const DT_* rhs;
+    DT_* out;
+    double* partials;             // kColProduct: out . x, kColInit: out . out (per block)
+    const int* status;
+    DT_ k[27];
+    DT_ d;
+  };
+
+  // W consecutive values from index i (any alignment); out of [0, n) the nearest value inside
+  template<int W, typename T>
+  __device__ __forceinline__ void load_line(const T* __restrict__ p, int i, int n, T (&o)[W])
+  {
+    if(i >= 0 && i + W <= n)
+    {
+      typedef T v2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
+      typedef T v4 __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+      constexpr int Q = sizeof(T) == 4 ? W / 4 * 4 : 0;
+      if constexpr(sizeof(T) == 4)
+      {
+#pragma unroll
+        for(int k = 0; k < Q; k += 4)
+        {
+          const v4 v = *reinterpret_cast<const v4*>(p + i + k);
+          o[k] = v[0]; o[k + 1] = v[1]; o[k + 2] = v[2]; o[k + 3] = v[3];
+        }
+      }
+#pragma unroll
+      for(int k = Q; k + 1 < W; k += 2)
+      {
+        const v2 v = *reinterpret_cast<const v2*>(p + i + k);
+        o[k] = v[0]; o[k + 1] = v[1];
+      }
+    }
+    else
+    {
+#pragma unroll
+      for(int k = 0; k < W; ++k)
+      {
+        const int j = i + k;
+        o[k] = p[j < 0 ? 0 : (j < n ? j : n - 1)];
+      }
+    }
+  }
+
+  template<typename DT_, u32 TAPS_, int OP_>
+  __global__ __launch_bounds__(kColThreads) void k_columns(ColArgs<DT_> a)
+  {
+    if(mg::stopped(a.status)) return;
+    constexpr int CX = ColShape<DT_>::CX, CZ = ColShape<DT_>::CZ;
+    const u32 blk = dev::xcd_remap(blockIdx.x, gridDim.x);
+    const u32 zc = blk / a.gblocks, g = (blk % a.gblocks) * u32(kColThreads) + threadIdx.x;
+    const int m = int(a.m), mm = int(a.mm), n = mm * m;
+    const int z0 = int(zc) * CZ, q0 = int(g) * CX;
+    double dot = 0.0;
+    if(g < a.groups)
+    {
+      DT_ s[CZ][CX], xc[CZ][CX];
+#pragma unroll
+      for(int j = 0; j < CZ; ++j)
+#pragma unroll
+        for(int c = 0; c < CX; ++c) { s[j][c] = DT_(0); xc[j][c] = DT_(0); }
+#pragma unroll
+      for(int pl = -1; pl <= CZ; ++pl)
+      {
+        const int z = z0 + pl;
+        if(z < 0 || z >= m) continue;   // (planes outside: only boundary nodes reach them)
+        DT_ v[3][CX + 2];
+#pragma unroll
+        for(int y = 0; y < 3; ++y) load_line<CX + 2>(a.x, z * mm + q0 + (y - 1) * m - 1, n, v[y]);
+        if(pl >= 0 && pl < CZ)
+        {
+#pragma unroll
+          for(int c = 0; c < CX; ++c) xc[pl][c] = v[1][c + 1];
+        }
+#pragma unroll
+        for(int l = 0; l < 3; ++l)
+        {
+          const int j = pl - l + 1;
+          if(j < 0 || j >= CZ) continue;
+#pragma unroll
+          for(int t = 0; t < 9; ++t)
+          {
+            if(!((TAPS_ >> (l * 9 + t)) & 1u)) continue;
+#pragma unroll
+            for(int c = 0; c < CX; ++c) s[j][c] = mg::fmadd(a.k[l * 9 + t], v[t / 3][c + t % 3], s[j][c]);
+          }
+        }
+      }
+      const u32 y0 = mg::udiv_magic(u32(q0), a.div), x0 = u32(q0) - y0 * a.m;
+#pragma unroll
+      for(int j = 0; j < CZ; ++j)
+      {
+        const int z = z0 + j;
+        if(z >= m) continue;
+        const int i = z * mm + q0;
+        DT_ b[CX], o[CX];
+        if constexpr(OP_ != kColProduct) load_line<CX>(a.rhs, i, n, b);
+        u32 x = x0, y = y0;
+#pragma unroll
+        for(int c = 0; c < CX; ++c)
+        {
+          const bool mid = x >= 1 && x + 1 < a.m && y >= 1 && y + 1 < a.m && z >= 1 && z + 1 < m;
+          if constexpr(OP_ == kColSweep) o[c] = xc[j][c] + (mid ? a.d : DT_(0)) * (b[c] - s[j][c]);
+          else if constexpr(OP_ == kColProduct) o[c] = mid ? s[j][c] : DT_(0);
+          else o[c] = mid ? b[c] - s[j][c] : DT_(0);
+          const bool in = q0 + c < mm;
+          if constexpr(OP_ == kColProduct) dot += in ? double(o[c]) * double(xc[j][c]) : 0.0;
+          if constexpr(OP_ == kColInit) dot += in ? double(o[c]) * double(o[c]) : 0.0;
+          ++x;
+          if(x == a.m) { x = 0; ++y; }
+        }
+        if(q0 + CX <= mm)
+        {
+          typedef DT_ vc __attribute__((ext_vector_type(CX), aligned(sizeof(DT_))));
+          vc w;
+#pragma unroll
+          for(int c = 0; c < CX; ++c) w[c] = o[c];
+          *reinterpret_cast<vc*>(a.out + i) = w;
+        }
+        else
+        {
+#pragma unroll
+          for(int c = 0; c < CX; ++c)
+            if(q0 + c < mm) a.out[i + c] = o[c];
+        }
+      }
+    }
+    if constexpr(OP_ == kColProduct || OP_ == kColInit) dev::block_partial(dot, a.partials);
+  }
+
+  // x_f += P x_c on a 3D Q1 lattice: a thread takes four consecutive nodes of a line, whose coarse
+  // nodes are three values of one, two or four coarse lines (terms in ascending column order; the
+  // weights are powers of two).  Boundary nodes keep their value.
+  template<typename DT_>
+  __global__ __launch_bounds__(256) void k_prolong_q1(u32 m, u32 mc, u32 quads, u64 div, const DT_* __restrict__ xc, DT_* __restrict__ xf,
+                                                      const int* status)
+  {
+#pragma clang fp contract(off)
+    if(mg::stopped(status)) return;
+    // grid: x over the quads of a plane, y the planes
+    const u32 t = blockIdx.x * 256u + threadIdx.x, z = blockIdx.y + 1u;
+    const u32 y = mg::udiv_magic(t, div) + 1u, x0 = (t - (y - 1u) * quads) * 4u;
+    if(y + 1u >= m) return;
+    const u32 oz = z & 1u, oy = y & 1u;
+    const u32 cy = y >> 1, cz = z >> 1, cx = x0 >> 1;
+    const bool has2 = cx + 2u < mc;
+    DT_ c[2][2][3];
+#pragma unroll
+    for(u32 b = 0; b < 2; ++b)
+#pragma unroll
+      for(u32 e = 0; e < 2; ++e)
+      {
+        const u32 i = ((cz + (b & oz)) * mc + cy + (e & oy)) * mc + cx;
+        c[b][e][0] = xc[i];
+        c[b][e][1] = xc[cx + 1u < mc ? i + 1u : i];
+        c[b][e][2] = xc[has2 ? i + 2u : i];
+      }
+    const u32 i0 = (z * m + y) * m + x0;
+    const DT_ wzy = DT_((oz ? 0.5f : 1.0f) * (oy ? 0.5f : 1.0f));
+    DT_ v[4];
+    load_line<4>(xf, int(i0), int(m * m * m), v);
+#pragma unroll
+    for(u32 k = 0; k < 4; ++k)
+    {
+      const u32 x = x0 + k;
+      DT_ s = DT_(0);
+#pragma unroll
+      for(u32 b = 0; b < 2; ++b)
+#pragma unroll
+        for(u32 e = 0; e < 2; ++e)
+        {
+          const DT_ w = (k & 1u) ? DT_(0.5f) * wzy : wzy;
+          const DT_ s1 = s + w * c[b][e][k >> 1];
+          const DT_ s2 = (k & 1u) ? s1 + w * c[b][e][(k >> 1) + 1u] : s1;
+          s = ((b && !oz) || (e && !oy)) ? s : s2;
+        }
+      v[k] = (x < 1u || x + 1u >= m) ? v[k] : v[k] + s;
+    }
+    if(x0 + 4u <= m)
+    {
+      typedef DT_ v4 __attribute__((ext_vector_type(4), aligned(sizeof(DT_))));
+      v4 w;
+#pragma unroll
+      for(int k = 0; k < 4; ++k) w[k] = v[k];
+      *reinterpret_cast<v4*>(xf + i0) = w;
+    }
+    else
+    {
+#pragma unroll
+      for(u32 k = 0; k < 4; ++k)
+        if(x0 + k < m) xf[i0 + k] = v[k];
+    }
+  }
+
   // ---- setup ---------------------------------------------------------------------------------
 
   // Flags raised: 1 an entry outside the box of RAD nodes around its row's node; 2 an inner row that
   // differs (any value or its dinv, as bit patterns) from its class's row in rep, or Dirichlet
   // nodes other than the lattice's boundary.  Classes: the coordinates' parities (per = 2) or one;
-  // rep[class][tap], repd[class] in the arithmetic type.
+  // rep[class][tap], repd[class] in the arithmetic type (dinv null: not compared).
   template<typename DT_, typename VT_>
   __global__ void k_lattice_check(u64 n, u32 m, int dim, int rad, int per, const u32* __restrict__ rp, const u32* __restrict__ col,
                                   const VT_* __restrict__ val, const u32* __restrict__ mask, const DT_* __restrict__ dinv,
@@ -446,8 +664,11 @@ namespace lat
       if(!dir)
         for(int t = 0; t < ntap; ++t)
           if(!((hit >> t) & 1u) && rep[cls * ntap + t] != DT_(0)) f |= 2;
-      const DT_ d = dinv[r];
-      if(dir ? !(d == DT_(0)) : !(d == repd[cls])) f |= 2;
+      if(dinv)
+      {
+        const DT_ d = dinv[r];
+        if(dir ? !(d == DT_(0)) : !(d == repd[cls])) f |= 2;
+      }
       if(f) atomicOr(flags, f);
     }
   }

@@ -1537,6 +1537,7 @@ namespace
     u32 m = 0;
     DT k[27] = {}, d = DT(0);
     DevMem coef;
+    bool cols = false;    // 3D levels of kColumnRows or more: one step per launch (lat::k_columns)
   };
 
   template<typename DT, typename VT>
@@ -1551,6 +1552,10 @@ namespace
     DevCsr<double> A64own;
     DevMem r, p, q, zcg, state, hist, partials;
     const DevCsr<double>* A64 = nullptr;
+    // the outer product by columns (lat::k_columns): its lattice (0: not) and the matrix row
+    u32 out_m = 0;
+    bool out_faces = false;
+    double out_k[27] = {};
     u64 n0 = 0, hist_cap = 0;
     // an iteration is captured as one graph: the preconditioner half of iteration k (z = M r,
     // beta, p update; for k = 0 gamma and p from the first preconditioner application), the
@@ -1732,6 +1737,7 @@ namespace
       }
       if(cfg.plane_order == 2)
         for(std::size_t i = shared ? 1 : 0; i < L.size(); ++i) F3_RC(L[i]->A.make_tiles(s));
+      F3_RC(setup_outer_columns());
       F3_RC(r.alloc(sizeof(double) * n0));
       F3_RC(p.alloc(sizeof(double) * n0));
       F3_RC(q.alloc(sizeof(double) * n0));
@@ -1741,7 +1747,8 @@ namespace
       F3_RC(hist.alloc(sizeof(double) * hist_cap));
       // one partial per block of the largest reducing launch: row kernels launch at most
       // 8192 blocks (mg::row_grid), the streaming ones at most 4096
-      const u64 max_blocks = 8192;
+      u64 max_blocks = 8192;
+      if(out_m) max_blocks = std::max<u64>(max_blocks, columns_blocks<double>(out_m));
       F3_RC(partials.alloc(sizeof(double) * max_blocks));
       if(!ring)
       {
@@ -1755,6 +1762,52 @@ namespace
       F3_CHECK(hipStreamSynchronize(s));
       drop_graphs();
       return rt::kOk;
+    }
+
+    int setup_outer_columns()
+    {
+      out_m = 0;
+      const Level<DT, VT>& f = *L.front();
+      if(!f.cols) return rt::kOk;
+      std::vector<double> rep, repd;
+      bool box = false, uniform = false;
+      F3_RC((lattice_rows<double, double>(*A64, f.mask, nullptr, 3, 1, f.m, rep, repd, &box, &uniform)));
+      if(!uniform) return rt::kOk;
+      for(int t = 0; t < 27; ++t) out_k[t] = rep[t];
+      out_faces = has_faces(rep);
+      out_m = f.m;
+      return rt::kOk;
+    }
+
+    // q = filter(A p) with block partials of q.p; returns the number of partials in nb
+    int outer_product(const mg::PcgState* S, unsigned& nb)
+    {
+      double* part = partials.template as<double>();
+      if(out_m)
+      {
+        nb = columns<lat::kColProduct, double>(out_m, out_k, 0.0, out_faces, p.template as<double>(), nullptr, q.template as<double>(),
+                                               part, reinterpret_cast<const int*>(&S->status));
+        return rt::kOk;
+      }
+      return with_rows<double, double>(outer_matrix(), [&](auto A, mg::RowGrid g) {
+        mg::k_pcg_spmv_dot<<<g.blocks, kBlock, 0, s>>>(A, g.per, mask0_ptr(), p.template as<double>(), q.template as<double>(),
+                                                       S, part);
+        nb = g.blocks;
+      });
+    }
+    // r = filter(b - A x) with block partials of r.r
+    int outer_defect(const double* b, const double* x, unsigned& nb)
+    {
+      double* part = partials.template as<double>();
+      if(out_m)
+      {
+        nb = columns<lat::kColInit, double>(out_m, out_k, 0.0, out_faces, x, b, r.template as<double>(), part, nullptr);
+        return rt::kOk;
+      }
+      return with_rows<double, double>(outer_matrix(), [&](auto A, mg::RowGrid g) {
+        mg::k_pcg_defect_norm<<<g.blocks, kBlock, 0, s>>>(A, g.per, mask0_ptr(), b, x, r.template as<double>(), part);
+        nb = g.blocks;
+      });
     }
 
     void drop_graphs()
@@ -2084,10 +2137,71 @@ namespace
       }
     }
 
-    // Decides whether a level is smoothed in bricks: its prolongation is that of a Q1 or 2D Q2 space
-    // on a lattice (checked entry by entry when its factors were built), its matrix couples only the
-    // nodes of a box, and all inner rows of a class are the same bit for bit with the Dirichlet nodes
-    // the lattice's boundary -- or, 2D Q1, any values.  Everything else keeps its format's kernels.
+    // The rows of a matrix on an m^dim lattice by class (the coordinates' parities for rad = 2, else
+    // one): rep[class][tap], repd[class] the rows and dinv values of an inner node each.  *box: the
+    // matrix couples only the nodes of a box of rad nodes; *uniform: in addition every inner row (and
+    // dinv, when given) is its class's row bit for bit, the values are finite and the Dirichlet nodes
+    // are the lattice's boundary.
+    template<typename T, typename V>
+    int lattice_rows(const DevCsr<V>& A, const DevMem& mask, const T* dinv, int dim, int rad, u32 m, std::vector<T>& rep,
+                     std::vector<T>& repd, bool* box, bool* uniform)
+    {
+      *box = *uniform = false;
+      const int nl = 2 * rad + 1, ntap = dim == 3 ? nl * nl * nl : nl * nl, per = rad == 2 ? 2 : 1, ncls = per == 2 ? 4 : 1;
+      rep.assign(std::size_t(ncls) * ntap, T(0));
+      repd.assign(ncls, T(0));
+      bool finite = true;
+      for(int c = 0; c < ncls; ++c)
+      {
+        const u64 x = 4 + u64(c & 1), y = 4 + u64(c >> 1), z = dim == 3 ? 4 : 0, r = (z * m + y) * m + x;
+        u32 e[2];
+        F3_CHECK(hipMemcpy(e, A.rp.template as<u32>() + r, sizeof(e), hipMemcpyDeviceToHost));
+        if(e[1] - e[0] > 64) return rt::kOk;
+        std::vector<u32> col(e[1] - e[0]);
+        std::vector<V> val(e[1] - e[0]);
+        if(!col.empty())
+        {
+          F3_CHECK(hipMemcpy(col.data(), A.col.template as<u32>() + e[0], sizeof(u32) * col.size(), hipMemcpyDeviceToHost));
+          F3_CHECK(hipMemcpy(val.data(), A.val.template as<V>() + e[0], sizeof(V) * val.size(), hipMemcpyDeviceToHost));
+        }
+        if(dinv) F3_CHECK(hipMemcpy(&repd[c], dinv + r, sizeof(T), hipMemcpyDeviceToHost));
+        for(std::size_t k = 0; k < col.size(); ++k)
+        {
+          const int dx = int(col[k] % m) - int(x), dy = int(col[k] / m % m) - int(y), dz = int(col[k] / (m * m)) - int(z);
+          if(std::abs(dx) > rad || std::abs(dy) > rad || std::abs(dz) > (dim == 3 ? rad : 0)) return rt::kOk;
+          const T v = T(val[k]);
+          finite = finite && std::isfinite(double(v));
+          rep[std::size_t(c) * ntap + ((dim == 3 ? dz + rad : 0) * nl + dy + rad) * nl + dx + rad] = v;
+        }
+        finite = finite && std::isfinite(double(repd[c]));
+      }
+      DevMem drep, drepd, dflag;
+      F3_RC(drep.alloc(sizeof(T) * rep.size()));
+      F3_RC(drepd.alloc(sizeof(T) * repd.size()));
+      F3_RC(dflag.alloc(sizeof(int)));
+      F3_CHECK(hipMemcpyAsync(drep.p, rep.data(), sizeof(T) * rep.size(), hipMemcpyHostToDevice, s));
+      F3_CHECK(hipMemcpyAsync(drepd.p, repd.data(), sizeof(T) * repd.size(), hipMemcpyHostToDevice, s));
+      F3_CHECK(hipMemsetAsync(dflag.p, 0, sizeof(int), s));
+      lat::k_lattice_check<T, V><<<setup_blocks(A.rows), 256, 0, s>>>(
+        A.rows, m, dim, rad, per, A.rp.template as<u32>(), A.col.template as<u32>(), A.val.template as<V>(),
+        mask.template as<u32>(), dinv, drep.template as<T>(), drepd.template as<T>(), ntap, dflag.template as<int>());
+      F3_RC(rt::check_launch());
+      int flag = 3;
+      F3_CHECK(hipMemcpyAsync(&flag, dflag.p, sizeof(int), hipMemcpyDeviceToHost, s));
+      F3_CHECK(hipStreamSynchronize(s));
+      *box = !(flag & 1);
+      *uniform = finite && flag == 0;
+      return rt::kOk;
+    }
+
+    // Decides whether a level is smoothed in bricks (or columns): its prolongation is that of a Q1 or 2D
+    // Q2 space on a lattice (checked entry by entry when its factors were built), its matrix couples
+    // only the nodes of a box, and all inner rows of a class are the same with the Dirichlet nodes the
+    // lattice's boundary -- or, 2D Q1, any values.  Everything else keeps its format's kernels.
+    // 3D levels from this many rows on take one step per launch: 129^3 nodes in FP32, two steps 29.5 us
+    // in a brick launch; 65^3 nodes, a level's way down and up 39 us in bricks, ten launches of 4 us
+    static constexpr u64 kColumnRows = u64(1) << 20;
+
     int setup_lattice(Level<DT, VT>& l)
     {
       l.lat = -1;
@@ -2095,51 +2209,12 @@ namespace
       const int dim = l.P.tmo[2] > 1 ? 3 : 2, rad = l.P.tdeg;
       const u32 m = l.P.tmo[0];
       if((dim == 3 && rad != 1) || m < 9) return rt::kOk;
-      const int nl = 2 * rad + 1, ntap = dim == 3 ? nl * nl * nl : nl * nl, per = rad == 2 ? 2 : 1, ncls = per == 2 ? 4 : 1;
-      // the row of an inner node of every class
-      std::vector<DT> rep(std::size_t(ncls) * ntap, DT(0)), repd(ncls, DT(0));
-      bool finite = true;
-      for(int c = 0; c < ncls; ++c)
-      {
-        const u64 x = 4 + u64(c & 1), y = 4 + u64(c >> 1), z = dim == 3 ? 4 : 0, r = (z * m + y) * m + x;
-        u32 e[2];
-        F3_CHECK(hipMemcpy(e, l.A.rp.template as<u32>() + r, sizeof(e), hipMemcpyDeviceToHost));
-        if(e[1] - e[0] > 64) return rt::kOk;
-        std::vector<u32> col(e[1] - e[0]);
-        std::vector<VT> val(e[1] - e[0]);
-        if(!col.empty())
-        {
-          F3_CHECK(hipMemcpy(col.data(), l.A.col.template as<u32>() + e[0], sizeof(u32) * col.size(), hipMemcpyDeviceToHost));
-          F3_CHECK(hipMemcpy(val.data(), l.A.val.template as<VT>() + e[0], sizeof(VT) * val.size(), hipMemcpyDeviceToHost));
-        }
-        F3_CHECK(hipMemcpy(&repd[c], l.dinv.template as<DT>() + r, sizeof(DT), hipMemcpyDeviceToHost));
-        for(std::size_t k = 0; k < col.size(); ++k)
-        {
-          const int dx = int(col[k] % m) - int(x), dy = int(col[k] / m % m) - int(y), dz = int(col[k] / (m * m)) - int(z);
-          if(std::abs(dx) > rad || std::abs(dy) > rad || std::abs(dz) > (dim == 3 ? rad : 0)) return rt::kOk;
-          const DT v = DT(val[k]);
-          finite = finite && std::isfinite(double(v));
-          rep[std::size_t(c) * ntap + ((dim == 3 ? dz + rad : 0) * nl + dy + rad) * nl + dx + rad] = v;
-        }
-        finite = finite && std::isfinite(double(repd[c]));
-      }
-      DevMem drep, drepd, dflag;
-      F3_RC(drep.alloc(sizeof(DT) * rep.size()));
-      F3_RC(drepd.alloc(sizeof(DT) * repd.size()));
-      F3_RC(dflag.alloc(sizeof(int)));
-      F3_CHECK(hipMemcpyAsync(drep.p, rep.data(), sizeof(DT) * rep.size(), hipMemcpyHostToDevice, s));
-      F3_CHECK(hipMemcpyAsync(drepd.p, repd.data(), sizeof(DT) * repd.size(), hipMemcpyHostToDevice, s));
-      F3_CHECK(hipMemsetAsync(dflag.p, 0, sizeof(int), s));
-      lat::k_lattice_check<DT, VT><<<setup_blocks(l.n), 256, 0, s>>>(
-        l.n, m, dim, rad, per, l.A.rp.template as<u32>(), l.A.col.template as<u32>(), l.A.val.template as<VT>(),
-        l.mask.template as<u32>(), l.dinv.template as<DT>(), drep.template as<DT>(), drepd.template as<DT>(), ntap,
-        dflag.template as<int>());
-      F3_RC(rt::check_launch());
-      int flag = 3;
-      F3_CHECK(hipMemcpyAsync(&flag, dflag.p, sizeof(int), hipMemcpyDeviceToHost, s));
-      F3_CHECK(hipStreamSynchronize(s));
-      if(flag & 1) return rt::kOk;
-      if(!finite || (flag & 2))
+      const int nl = 2 * rad + 1, ntap = dim == 3 ? nl * nl * nl : nl * nl, per = rad == 2 ? 2 : 1;
+      std::vector<DT> rep, repd;
+      bool box = false, uniform = false;
+      F3_RC((lattice_rows<DT, VT>(l.A, l.mask, l.dinv.template as<DT>(), dim, rad, m, rep, repd, &box, &uniform)));
+      if(!box) return rt::kOk;
+      if(!uniform)
       {
         // a row per node: 2D Q1
         if(dim != 2 || rad != 1) return rt::kOk;
@@ -2154,27 +2229,15 @@ namespace
       }
       else if(per == 2)
       {
-        std::vector<DT> tab;
-        for(int c = 0; c < 4; ++c)
-        {
-          tab.insert(tab.end(), rep.begin() + c * ntap, rep.begin() + (c + 1) * ntap);
-          tab.push_back(repd[c]);
-        }
-        F3_RC(l.coef.alloc(sizeof(DT) * tab.size()));
-        F3_CHECK(hipMemcpy(l.coef.p, tab.data(), sizeof(DT) * tab.size(), hipMemcpyHostToDevice));
+        F3_RC(class_table(rep, repd, ntap, l.coef));
         l.lat = 4;
       }
       else
       {
         for(int t = 0; t < ntap; ++t) l.k[t] = rep[t];
         l.d = repd[0];
-        l.lat = dim == 2 ? 2 : 0;
-        if(dim == 3 && sizeof(DT) == 4)
-        {
-          bool faces = false;
-          for(int t = 0; t < ntap; ++t) faces = faces || (!((lat::kTapsNoFaces >> t) & 1u) && rep[t] != DT(0));
-          l.lat = faces ? 0 : 1;
-        }
+        l.lat = dim == 2 ? 2 : (sizeof(DT) == 4 && !has_faces(rep) ? 1 : 0);
+        l.cols = dim == 3 && l.n >= kColumnRows;
       }
       l.m = m;
       return with_brick(l.lat, [&](auto b) -> int {
@@ -2184,6 +2247,53 @@ namespace
                                        hipFuncAttributeMaxDynamicSharedMemorySize, B::LDS));
         return rt::kOk;
       });
+    }
+    template<typename T>
+    static bool has_faces(const std::vector<T>& rep)
+    {
+      for(int t = 0; t < 27; ++t)
+        if(!((lat::kTapsNoFaces >> t) & 1u) && rep[t] != T(0)) return true;
+      return false;
+    }
+    // [class][tap..., dinv] on the device
+    template<typename T>
+    int class_table(const std::vector<T>& rep, const std::vector<T>& repd, int ntap, DevMem& out)
+    {
+      std::vector<T> tab;
+      for(std::size_t c = 0; c < repd.size(); ++c)
+      {
+        tab.insert(tab.end(), rep.begin() + c * ntap, rep.begin() + (c + 1) * ntap);
+        tab.push_back(repd[c]);
+      }
+      F3_RC(out.alloc(sizeof(T) * tab.size()));
+      F3_CHECK(hipMemcpy(out.p, tab.data(), sizeof(T) * tab.size(), hipMemcpyHostToDevice));
+      return rt::kOk;
+    }
+
+    template<typename T>
+    static u64 columns_blocks(u64 m)
+    {
+      constexpr u64 CX = lat::ColShape<T>::CX, CZ = lat::ColShape<T>::CZ;
+      return ((m * m + CX - 1) / CX + lat::kColThreads - 1) / lat::kColThreads * ((m + CZ - 1) / CZ);
+    }
+    // one launch of lat::k_columns; returns its block count (the number of partials)
+    template<int OP, typename T>
+    unsigned columns(u32 m, const T* k, T d, bool faces, const T* x, const T* rhs, T* out, double* part, const int* status)
+    {
+      constexpr int CX = lat::ColShape<T>::CX;
+      lat::ColArgs<T> a{};
+      a.m = m;
+      a.mm = m * m;
+      a.groups = (a.mm + CX - 1) / CX;
+      a.gblocks = (a.groups + lat::kColThreads - 1) / lat::kColThreads;
+      a.div = mg::udiv_magic_for(m);
+      a.x = x; a.rhs = rhs; a.out = out; a.partials = part; a.status = status;
+      for(int t = 0; t < 27; ++t) a.k[t] = k[t];
+      a.d = d;
+      const unsigned nb = unsigned(columns_blocks<T>(m));
+      if(faces) lat::k_columns<T, lat::kTapsAll, OP><<<nb, lat::kColThreads, 0, s>>>(a);
+      else lat::k_columns<T, lat::kTapsNoFaces, OP><<<nb, lat::kColThreads, 0, s>>>(a);
+      return nb;
     }
 
     // tile extents, halo and block count of a launch of `sweeps` steps; false: the halo leaves no tile
@@ -2243,9 +2353,11 @@ namespace
       for(std::size_t k = 0; k < cycle_ops.size();)
       {
         const CycleOp c = cycle_ops[k];
-        if(c.lvl >= nl || L[c.lvl]->lat < 0 || c.op == Op::bottom)
+        if(L[c.lvl]->lat < 0 || L[c.lvl]->cols || c.op == Op::bottom)
         {
-          plan.push_back(PlanOp{c, false, 0, 0, false, false});
+          PlanOp o{c, false, 0, 0, false, false};
+          if(c.op == Op::rest_step && L[c.lvl + 1]->lat >= 0 && !L[c.lvl + 1]->cols) { o.c.op = Op::rest; zero[c.lvl + 1] = 1; }
+          plan.push_back(o);
           ++k;
           continue;
         }
@@ -2261,7 +2373,7 @@ namespace
         {
           rest = true;
           step = cycle_ops[k + 1].op == Op::rest_step;
-          if(step && L[i + 1]->lat >= 0) { step = false; zero[i + 1] = 1; }
+          if(step && L[i + 1]->lat >= 0 && !L[i + 1]->cols) { step = false; zero[i + 1] = 1; }
           k += 2;
         }
         // the split: best[s] = least cost of the last s steps (the restriction in the last launch)
@@ -2411,10 +2523,19 @@ namespace
             oth[0] = f.t.template as<DT>();
             break;
           case Op::sweep:
-            F3_RC(sweep(f, cur[i], oth[i], status));
+            if(f.cols)
+              columns<lat::kColSweep, DT>(f.m, f.k, f.d, f.lat == 0, cur[i], f.rhs.template as<DT>(), oth[i], nullptr, status);
+            else
+              F3_RC(sweep(f, cur[i], oth[i], status));
             std::swap(cur[i], oth[i]);
             break;
           case Op::defect:
+            if(f.cols)
+            {
+              columns<lat::kColDefect, DT>(f.m, f.k, f.d, f.lat == 0, cur[i], f.rhs.template as<DT>(), f.def.template as<DT>(), nullptr,
+                                           status);
+              break;
+            }
             F3_RC(with_rows<DT, VT>(f.A, [&](auto A, mg::RowGrid g) {
               mg::k_defect<<<g.blocks, kBlock, 0, s>>>(A, g.per, f.mask.template as<u32>(), f.rhs.template as<DT>(),
                                                        (const DT*)cur[i], f.def.template as<DT>(), status);
@@ -2452,6 +2573,13 @@ namespace
             cur[i] = f.xfinal;
             break;
           case Op::prol:
+            if(f.cols)
+            {
+              const u32 m = f.m, quads = (m + 3) / 4;
+              lat::k_prolong_q1<DT><<<dim3((quads * (m - 2) + 255) / 256, m - 2), 256, 0, s>>>(
+                m, f.P.tmi[0], quads, mg::udiv_magic_for(quads), (const DT*)cur[i + 1], cur[i], status);
+              break;
+            }
             F3_RC(with_transfer_rows<DT, VT>(f.P, [&](auto P, mg::RowGrid g) {
               mg::k_prolong<<<g.blocks, kBlock, 0, s>>>(P, g.per, f.mask.template as<u32>(), (const DT*)cur[i + 1], cur[i],
                                                         status);
@@ -2641,11 +2769,7 @@ namespace
       mg::PcgState* S = st();
       double* part = partials.template as<double>();
       unsigned nb = 0;
-      F3_RC(with_rows<double, double>(outer_matrix(), [&](auto A, mg::RowGrid g) {
-        mg::k_pcg_spmv_dot<<<g.blocks, kBlock, 0, s>>>(A, g.per, mask0_ptr(), p.template as<double>(), q.template as<double>(),
-                                                       S, part);
-        nb = g.blocks;
-      }));
+      F3_RC(outer_product(S, nb));
       fin<mg::kFinAlpha>(nb);
       mg::k_pcg_update_norm<<<stream_blocks(n0), kBlock, 0, s>>>(n0, p.template as<double>(), q.template as<double>(),
                                                                 x_cur, r.template as<double>(), S, part);
@@ -2713,10 +2837,7 @@ namespace
       if(correct)
       {
         unsigned nb = 0;
-        F3_RC(with_rows<double, double>(outer_matrix(), [&](auto A, mg::RowGrid g) {
-          mg::k_pcg_defect_norm<<<g.blocks, kBlock, 0, s>>>(A, g.per, mask0_ptr(), b, (const double*)x, r.template as<double>(), part);
-          nb = g.blocks;
-        }));
+        F3_RC(outer_defect(b, x, nb));
         fin<mg::kFinInitDefect>(nb);
       }
       else
@@ -2825,8 +2946,20 @@ namespace
         {
           switch(which)
           {
-            case 0: F3_RC(sweep(f, f.x.template as<DT>(), f.t.template as<DT>(), nullptr)); break;
+            case 0:
+              if(f.cols)
+                columns<lat::kColSweep, DT>(f.m, f.k, f.d, f.lat == 0, f.x.template as<DT>(), f.rhs.template as<DT>(), f.t.template as<DT>(),
+                                            nullptr, nullptr);
+              else
+                F3_RC(sweep(f, f.x.template as<DT>(), f.t.template as<DT>(), nullptr));
+              break;
             case 1:
+              if(f.cols)
+              {
+                columns<lat::kColDefect, DT>(f.m, f.k, f.d, f.lat == 0, f.x.template as<DT>(), f.rhs.template as<DT>(),
+                                             f.def.template as<DT>(), nullptr, nullptr);
+                break;
+              }
               F3_RC(with_rows<DT, VT>(f.A, [&](auto A, mg::RowGrid g) {
                 mg::k_defect<<<g.blocks, kBlock, 0, s>>>(A, g.per,f.mask.template as<u32>(), f.rhs.template as<DT>(),
                                                              (const DT*)f.x.template as<DT>(), f.def.template as<DT>(), nullptr);
@@ -2843,11 +2976,8 @@ namespace
                 F3_RC(timing_state.alloc(sizeof(mg::PcgState)));
                 F3_CHECK(hipMemcpyAsync(timing_state.p, &h, sizeof(h), hipMemcpyHostToDevice, s));
               }
-              F3_RC(with_rows<double, double>(outer_matrix(), [&](auto A, mg::RowGrid g) {
-                mg::k_pcg_spmv_dot<<<g.blocks, kBlock, 0, s>>>(A, g.per, mask0_ptr(), p.template as<double>(),
-                                                               q.template as<double>(), timing_state.template as<mg::PcgState>(),
-                                                               partials.template as<double>());
-              }));
+              unsigned nb = 0;
+              F3_RC(outer_product(timing_state.template as<mg::PcgState>(), nb));
               break;
             }
             case 3: F3_RC(enqueue_vcycle(r.template as<double>(), nullptr)); break;
@@ -2863,8 +2993,11 @@ namespace
       if(bytes)
       {
         const u64 vb = sizeof(DT);
-        // sweep: matrix + x gathered once + rhs + dinv + x_out; defect: matrix + x + rhs + def (+mask)
-        if(which == 0) *bytes = f.A.matrix_bytes() + f.n * vb * 4;
+        // sweep: matrix + x gathered once + rhs + dinv + x_out; defect: matrix + x + rhs + def (+mask);
+        // by columns: the vectors only (the matrix row is in the launch's arguments)
+        if(f.cols && which <= 1) *bytes = f.n * vb * 3;
+        else if(out_m && which == 2) *bytes = n0 * 8 * 2;
+        else if(which == 0) *bytes = f.A.matrix_bytes() + f.n * vb * 4;
         else if(which == 1) *bytes = f.A.matrix_bytes() + f.n * vb * 3 + (f.n + 31) / 32 * 4;
         else if(which == 2) *bytes = outer_matrix().matrix_bytes() + n0 * 8 * 2 + (n0 + 31) / 32 * 4;
         else *bytes = 0;

@@ -94,3 +94,32 @@ def test_other_formats_agree(torch, fmt, inner):
     b, _ = cycles(torch, H, d, inner, 0, fmt=fmt)
     eps = np.finfo(np.float64 if inner == "f64" else np.float32).eps
     assert np.linalg.norm(a - b) <= 27 * eps * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("inner", ["f64", "f32"])
+def test_columns_are_bitwise_the_steps(torch, inner):
+    """The finest 3D level of 2^20 rows or more takes its steps by columns (129^3 nodes): the cycle bit for
+    bit; the solve, whose dot products are grouped by other blocks, the same iterations and 1e-12."""
+    from feat3_amd.solver import MGPCG
+    levels = pb.hierarchy_device(3, 1, 7, 1)
+    n = levels[0].A.rows
+    b = torch.rand(n, dtype=torch.float64, device="cuda", generator=torch.Generator("cuda").manual_seed(3)) - 0.5
+    b[levels[0].bnd.long()] = 0.0
+    out = []
+    for lattice in (1, 0):
+        s = MGPCG(levels, inner=inner, fmt="banded", options={"lattice": lattice}).init()
+        c = torch.empty_like(b)
+        for _ in range(2):
+            s.vcycle(c, b)
+        x = torch.zeros_like(b)
+        st, it = s.correct(x, b)
+        # from a start other than zero: the initial defect's product
+        y = 0.5 * x
+        st2, it2 = s.correct(y, b)
+        out.append((c.cpu().numpy(), x.cpu().numpy(), y.cpu().numpy(), st, it, st2, it2))
+        s.done()
+    a, e = out
+    assert np.array_equal(a[0], e[0])
+    assert a[3:] == e[3:] and a[3] == a[5] == 2
+    assert np.linalg.norm(a[1] - e[1]) <= 1e-12 * np.linalg.norm(e[1])
+    assert np.linalg.norm(a[2] - e[2]) <= 1e-12 * np.linalg.norm(e[2])

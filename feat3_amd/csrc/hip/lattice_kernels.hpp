@@ -61,6 +61,8 @@ namespace lat
     DT_* rhs_c;
     DT_* x_c;                  // first step of the next level (null: not wanted)
     const DT_* dinv_c;
+    const double* dot_r;       // with it: partials[block] = sum of r x over the tile (the cycle's last launch)
+    double* partials;
     const int* status;
     DT_ k[27];                 // MODE 0
     DT_ d;
@@ -207,6 +209,17 @@ namespace lat
 #pragma unroll
       for(int j = 0; j < CZ; ++j) b[j] = inside(j) ? b[j] : DT(0);
     }
+    double rv[CZ];   // (loaded ahead of the steps: behind them it cost the launch another memory latency)
+    if(a.dot_r)
+    {
+#pragma unroll
+      for(int j = 0; j < CZ; ++j) rv[j] = a.dot_r[at[j]];
+    }
+    else
+    {
+#pragma unroll
+      for(int j = 0; j < CZ; ++j) rv[j] = 0.0;
+    }
     if(a.in == kMem || a.in == kProl)
     {
 #pragma unroll
@@ -350,6 +363,14 @@ namespace lat
       for(int j = 0; j < CZ; ++j)
         if(owned(j)) a.xout[i0 + u32(j) * layer] = xr[j];
     }
+    if(a.dot_r)
+    {
+      double v = 0.0;
+#pragma unroll
+      for(int j = 0; j < CZ; ++j)
+        if(owned(j)) v += rv[j] * double(xr[j]);
+      dev::block_partial(v, a.partials);
+    }
     if(!a.restrict_) return;
     if(needed(B_::RLO, B_::RHI))
     {
@@ -429,7 +450,9 @@ namespace lat
   constexpr int kColThreads = 256;
   template<typename DT_> struct ColShape { static constexpr int CX = sizeof(DT_) == 4 ? 4 : 2, CZ = sizeof(DT_) == 4 ? 2 : 4; };
 
-  enum ColOp : int { kColSweep = 0, kColDefect = 1, kColProduct = 2, kColInit = 3 };
+  // kColZero: a step from the first step's iterate dinv .* rhs, formed where it is read (no x); kColLast: a
+  // step with the partials of r . out; kColProduct commits the new gamma (mg::commit_gamma)
+  enum ColOp : int { kColSweep = 0, kColDefect = 1, kColProduct = 2, kColInit = 3, kColZero = 4, kColLast = 5 };
 
   template<typename DT_>
   struct ColArgs
@@ -439,7 +462,9 @@ namespace lat
     const DT_* x;
     const DT_* rhs;
     DT_* out;
-    double* partials;             // kColProduct: out . x, kColInit: out . out (per block)
+    double* partials;             // per block: kColProduct out . x, kColInit out . out, kColLast r . out
+    const double* r;              // kColLast
+    mg::PcgState* st;             // kColProduct
     const int* status;
     DT_ k[27];
     DT_ d;
@@ -491,8 +516,25 @@ namespace lat
     const int m = int(a.m), mm = int(a.mm), n = mm * m;
     const int z0 = int(zc) * CZ, q0 = int(g) * CX;
     double dot = 0.0;
+    if constexpr(OP_ == kColProduct) mg::commit_gamma(a.st);
     if(g < a.groups)
     {
+      const u32 y0 = mg::udiv_magic(u32(q0), a.div), x0 = u32(q0) - y0 * a.m;
+      // kColZero: dinv at the loaded nodes of an inner plane
+      DT_ dz[3][CX + 2];
+      if constexpr(OP_ == kColZero)
+      {
+#pragma unroll
+        for(int y = 0; y < 3; ++y)
+#pragma unroll
+          for(int k = 0; k < CX + 2; ++k)
+          {
+            int lx = int(x0) + k - 1, ly = int(y0) + y - 1;
+            if(lx < 0) { lx += m; --ly; }
+            if(lx >= m) { lx -= m; ++ly; }
+            dz[y][k] = lx >= 1 && lx + 1 < m && ly >= 1 && ly + 1 < m ? a.d : DT_(0);
+          }
+      }
       DT_ s[CZ][CX], xc[CZ][CX];
 #pragma unroll
       for(int j = 0; j < CZ; ++j)
@@ -505,7 +547,16 @@ namespace lat
         if(z < 0 || z >= m) continue;   // (planes outside: only boundary nodes reach them)
         DT_ v[3][CX + 2];
 #pragma unroll
-        for(int y = 0; y < 3; ++y) load_line<CX + 2>(a.x, z * mm + q0 + (y - 1) * m - 1, n, v[y]);
+        for(int y = 0; y < 3; ++y)
+          load_line<CX + 2>(OP_ == kColZero ? a.rhs : a.x, z * mm + q0 + (y - 1) * m - 1, n, v[y]);
+        if constexpr(OP_ == kColZero)
+        {
+          const bool mid = z >= 1 && z + 1 < m;
+#pragma unroll
+          for(int y = 0; y < 3; ++y)
+#pragma unroll
+            for(int k = 0; k < CX + 2; ++k) v[y][k] = (mid ? dz[y][k] : DT_(0)) * v[y][k];
+        }
         if(pl >= 0 && pl < CZ)
         {
 #pragma unroll
@@ -525,7 +576,6 @@ namespace lat
           }
         }
       }
-      const u32 y0 = mg::udiv_magic(u32(q0), a.div), x0 = u32(q0) - y0 * a.m;
 #pragma unroll
       for(int j = 0; j < CZ; ++j)
       {
@@ -533,18 +583,21 @@ namespace lat
         if(z >= m) continue;
         const int i = z * mm + q0;
         DT_ b[CX], o[CX];
+        double rv[CX];
         if constexpr(OP_ != kColProduct) load_line<CX>(a.rhs, i, n, b);
+        if constexpr(OP_ == kColLast) load_line<CX>(a.r, i, n, rv);
         u32 x = x0, y = y0;
 #pragma unroll
         for(int c = 0; c < CX; ++c)
         {
           const bool mid = x >= 1 && x + 1 < a.m && y >= 1 && y + 1 < a.m && z >= 1 && z + 1 < m;
-          if constexpr(OP_ == kColSweep) o[c] = xc[j][c] + (mid ? a.d : DT_(0)) * (b[c] - s[j][c]);
+          if constexpr(OP_ == kColSweep || OP_ == kColZero || OP_ == kColLast) o[c] = xc[j][c] + (mid ? a.d : DT_(0)) * (b[c] - s[j][c]);
           else if constexpr(OP_ == kColProduct) o[c] = mid ? s[j][c] : DT_(0);
           else o[c] = mid ? b[c] - s[j][c] : DT_(0);
           const bool in = q0 + c < mm;
           if constexpr(OP_ == kColProduct) dot += in ? double(o[c]) * double(xc[j][c]) : 0.0;
           if constexpr(OP_ == kColInit) dot += in ? double(o[c]) * double(o[c]) : 0.0;
+          if constexpr(OP_ == kColLast) dot += in ? rv[c] * double(o[c]) : 0.0;
           ++x;
           if(x == a.m) { x = 0; ++y; }
         }
@@ -564,7 +617,7 @@ namespace lat
         }
       }
     }
-    if constexpr(OP_ == kColProduct || OP_ == kColInit) dev::block_partial(dot, a.partials);
+    if constexpr(OP_ == kColProduct || OP_ == kColInit || OP_ == kColLast) dev::block_partial(dot, a.partials);
   }
 
   // x_f += P x_c on a 3D Q1 lattice: a thread takes four consecutive nodes of a line, whose coarse
@@ -638,14 +691,15 @@ namespace lat
   // nodes other than the lattice's boundary.  Classes: the coordinates' parities (per = 2) or one;
   // rep[class][tap], repd[class] in the arithmetic type (dinv null: not compared).
   template<typename DT_, typename VT_>
-  __global__ void k_lattice_check(u64 n, u32 m, int dim, int rad, int per, const u32* __restrict__ rp, const u32* __restrict__ col,
+  __global__ void k_lattice_check(u64 n, u32 m, u64 div_m, int dim, int rad, int per, const u32* __restrict__ rp, const u32* __restrict__ col,
                                   const VT_* __restrict__ val, const u32* __restrict__ mask, const DT_* __restrict__ dinv,
                                   const DT_* __restrict__ rep, const DT_* __restrict__ repd, int ntap, int* flags)
   {
     const int nl = 2 * rad + 1;
     for(u64 r = u64(blockIdx.x) * blockDim.x + threadIdx.x; r < n; r += u64(gridDim.x) * blockDim.x)
     {
-      const int x = int(r % m), y = int((r / m) % m), z = int(r / (u64(m) * m));
+      const u32 rl = mg::udiv_magic(u32(r), div_m), rz = mg::udiv_magic(rl, div_m);
+      const int x = int(u32(r) - rl * m), y = int(rl - rz * m), z = int(rz);
       const bool edge = x == 0 || y == 0 || (dim == 3 && z == 0) || x == int(m) - 1 || y == int(m) - 1 || (dim == 3 && z == int(m) - 1);
       const bool dir = dev::masked(mask, r);
       int f = dir != edge ? 2 : 0;
@@ -653,8 +707,8 @@ namespace lat
       u32 hit = 0;
       for(u32 k = rp[r]; k < rp[r + 1]; ++k)
       {
-        const u32 c = col[k];
-        const int dx = int(c % m) - x, dy = int((c / m) % m) - y, dz = int(c / (m * m)) - z;
+        const u32 c = col[k], cl = mg::udiv_magic(c, div_m), cz = mg::udiv_magic(cl, div_m);
+        const int dx = int(c - cl * m) - x, dy = int(cl - cz * m) - y, dz = int(cz) - z;
         if(dx < -rad || dx > rad || dy < -rad || dy > rad || dz < -rad || dz > rad || (dim == 2 && dz != 0)) { f |= 3; continue; }
         const int t = ((dim == 3 ? dz + rad : 0) * nl + dy + rad) * nl + dx + rad;
         const DT_ v = dev::ld<DT_>(val, k);

@@ -806,7 +806,7 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
   // ---- V-cycle kernels -------------------------------------------------------------------
 
   // MG entry: rhs = def (converted to the inner precision, convert_precond.hpp:104),
-  // first Richardson step from zero: x = dinv .* rhs
+  // first Richardson step from zero: x = dinv .* rhs (x null: the cycle's first launch forms it)
   template<typename DT_>
   __global__ void k_mg_entry(u64 n, const double* __restrict__ def, DT_* __restrict__ rhs, DT_* __restrict__ x,
                              const DT_* __restrict__ dinv, const int* status)
@@ -816,7 +816,7 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     {
       const DT_ r = DT_(def[i]);
       rhs[i] = r;
-      x[i] = dinv[i] * r;
+      if(x) x[i] = dinv[i] * r;
     }
   }
 
@@ -1198,10 +1198,12 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
 #pragma unroll
       for(u32 k = 0; k < U; ++k)
       {
-        const u32 j = j0 + k * u32(dev::kWave);
-        av[k] = j < n ? a[j] : DT_(0);
-        bv[k] = j < n ? rhs[j] : DT_(0);
+        const u32 j = j0 + k * u32(dev::kWave), i = j < n ? j : n - 1u;   // (no branches between the loads)
+        av[k] = a[i];
+        bv[k] = rhs[i];
       }
+#pragma unroll
+      for(u32 k = 0; k < U; ++k) bv[k] = j0 + k * u32(dev::kWave) < n ? bv[k] : DT_(0);
 #pragma unroll
       for(u32 k = 0; k < U; ++k) s = fmadd(double(av[k]), double(bv[k]), s);
     }
@@ -1231,12 +1233,35 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
   // device-resident PCG scalars and the criteria of IterativeSolver (iterative.hpp:213-237)
   struct PcgState
   {
-    double gamma, alpha, beta, def_init, def_cur, def_prev;
+    double gamma, gamma_new, alpha, beta, def_init, def_cur, def_prev;
     double tol_rel, tol_abs, tol_abs_low, div_rel, div_abs, stag_rate;
     u64 num_iter, min_iter, max_iter, min_stag_iter, num_stag_iter, hist_cap;
     int status;
     int first;   // set with the initial defect: the next beta finalisation starts the recurrence
   };
+
+  // The scalars of an iteration pass from kernel to kernel without launches of their own: a kernel that
+  // needs the sum of its predecessor's nb block partials forms it in every block (the same order,
+  // so the same bits, in each).  Such a kernel must not change what its other blocks still read, so
+  // k_pcg_update_p leaves the new gamma in gamma_new and the product behind it, which reads
+  // neither, moves it to gamma.  With more partials than kFoldPartials (general formats of large
+  // matrices) the sums keep a one-block launch (k_pcg_fin): every block of the reader would read them.
+  // Measured (2D Q1 L6 FP64, 3D Q1 L7 FP32): a k_pcg_fin launch takes 3.5 to 4.8 us, a folded sum adds
+  // below 1 us to its kernel.
+  constexpr unsigned kFoldPartials = 2048;
+  __device__ __forceinline__ void commit_gamma(PcgState* st)
+  {
+    if(blockIdx.x == 0 && threadIdx.x == 0) { st->gamma = st->gamma_new; st->first = 0; }
+  }
+  // the sum of the predecessor's partials, in every thread of the block
+  __device__ __forceinline__ double folded_sum(const double* partials, unsigned nb)
+  {
+    __shared__ double sum_;
+    const double t = dev::sum_partials(partials, nb);
+    if(threadIdx.x == 0) sum_ = t;
+    __syncthreads();
+    return sum_;
+  }
 
   // _set_initial_defect (iterative.hpp:744-766)
   __device__ inline void set_initial_defect(PcgState* st, double* hist, double d)
@@ -1316,28 +1341,13 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     dev::block_partial(v, partials);
   }
 
-  // p = z (correction converted back to FP64, convert_precond.hpp:115), partial sums of r.p
-  template<typename DT_>
-  __global__ __launch_bounds__(256) void k_pcg_p_gamma(u64 n, const DT_* __restrict__ z, const double* __restrict__ r,
-                                                       double* __restrict__ p, const PcgState* st, double* partials)
-  {
-    if(st->status != kProgress) return;
-    double v = 0.0;
-    for(u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += u64(gridDim.x) * blockDim.x)
-    {
-      const double zi = double(z[i]);
-      p[i] = zi;
-      v += r[i] * zi;
-    }
-    dev::block_partial(v, partials);
-  }
-
   // q = filter(A p), partial sums of q.p   (pcg.hpp:236-242)
   template<typename Rows_>
   __global__ __launch_bounds__(256) F3_ROW_ATTR void k_pcg_spmv_dot(Rows_ A, u64 per, const u32* __restrict__ mask, const double* __restrict__ p,
-                                                        double* __restrict__ q, const PcgState* st, double* partials)
+                                                        double* __restrict__ q, PcgState* st, double* partials)
   {
     if(st->status != kProgress) return;
+    commit_gamma(st);
     double v = 0.0;
     for_rows(A, per, p, [&](u64 pos, double s, bool w) {
       const u64 row = A.row(pos);
@@ -1352,13 +1362,24 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     dev::block_partial(v, partials);
   }
 
-  // x += alpha p, r -= alpha q, partial sums of r.r   (pcg.hpp:244-259)
-  static __global__ __launch_bounds__(256) void k_pcg_update_norm(u64 n, const double* __restrict__ p, const double* __restrict__ q,
-                                                           double* __restrict__ x, double* __restrict__ r, const PcgState* st,
-                                                           double* partials)
+  // x += alpha p, r -= alpha q, partial sums of r.r   (pcg.hpp:244-259); alpha = gamma / (q.p) from the
+  // product's nb partials (nb = 0: from the state).  Also the next cycle's entry: rhs = (inner) r
+  // (convert_precond.hpp:104; null: not wanted) and, with dinv, its first smoothing step x0 = dinv .* rhs.
+  template<typename DT_>
+  __global__ __launch_bounds__(256) void k_pcg_update_norm(u64 n, const double* __restrict__ p, const double* __restrict__ q,
+                                                           double* __restrict__ x, double* __restrict__ r, PcgState* st,
+                                                           const double* __restrict__ pq, unsigned nb, double* partials,
+                                                           DT_* __restrict__ rhs, DT_* __restrict__ x0, const DT_* __restrict__ dinv)
   {
     if(st->status != kProgress) return;
-    const double alpha = st->alpha;
+    double alpha;
+    if(nb)
+    {
+      alpha = st->gamma / folded_sum(pq, nb);                          // pcg.hpp:240
+      if(blockIdx.x == 0 && threadIdx.x == 0) st->alpha = alpha;       // (read by no other block)
+    }
+    else
+      alpha = st->alpha;
     // axpy with |alpha| < eps is a copy; written as a negation so that a NaN alpha updates (and the
     // NaN reaches the defect norm) as in dense_vector.hpp:891
     const bool upd = !(fabs(alpha) < 2.220446049250313e-16);
@@ -1373,6 +1394,12 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
         r[i] = ri;
       }
       v += ri * ri;
+      if(rhs)
+      {
+        const DT_ c = DT_(ri);
+        rhs[i] = c;
+        if(x0) x0[i] = dinv[i] * c;
+      }
     }
     dev::block_partial(v, partials);
   }
@@ -1389,50 +1416,64 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     dev::block_partial(v, partials);
   }
 
-  enum : int { kFinInitDefect = 0, kFinAlpha = 1, kFinNewDefect = 2, kFinGamma = 3, kFinBeta = 4 };
+  enum : int { kFinInitDefect = 0, kFinAlpha = 1, kFinNewDefect = 2, kFinGamma = 3, kFinBeta = 4 };   // (kFinGamma: batched)
 
-  // finalisation of one PCG reduction (one block of 256 threads)
+  // Publication of the solver state to the host: publication c of a solve (c counted on the device in
+  // *count) goes to slot c % R of a ring in pinned host memory, and after a system-scope fence its
+  // sequence number c + 1 to seq[c % R], which the host polls.
+  struct PubRing
+  {
+    PcgState* ring;
+    unsigned* seq;
+    unsigned* count;
+    unsigned slots;
+  };
+
+  // finalisation of one PCG reduction (one block of 256 threads); the defects' also publish the
+  // state, whatever the status, so that every publication the host launched arrives
   template<int OP>
-  __global__ __launch_bounds__(256) void k_pcg_fin(const double* __restrict__ partials, unsigned nb, PcgState* st, double* hist)
+  __global__ __launch_bounds__(256) void k_pcg_fin(const double* __restrict__ partials, unsigned nb, PcgState* st, double* hist,
+                                                   PubRing pub)
   {
-    if(OP != kFinInitDefect && st->status != kProgress) return;
-    const double t = dev::sum_partials(partials, nb);
+    constexpr bool publish = OP == kFinInitDefect || OP == kFinNewDefect;
+    const bool run = OP == kFinInitDefect || st->status == kProgress;
+    if(!publish && !run) return;
+    const double t = run ? dev::sum_partials(partials, nb) : 0.0;   // (run is the same in every thread)
     if(threadIdx.x != 0) return;
-    if(OP == kFinInitDefect) set_initial_defect(st, hist, sqrt(t));        // iterative.hpp:744-766
-    else if(OP == kFinAlpha) st->alpha = st->gamma / t;                     // pcg.hpp:240
-    else if(OP == kFinNewDefect) set_new_defect(st, hist, sqrt(t));         // iterative.hpp:848-879
-    else if(OP == kFinGamma) st->gamma = t;                                 // pcg.hpp:229
-    else if(st->first)
+    if(run)
     {
-      // the initial preconditioner application: gamma = r.z, p = z (pcg.hpp:225-231)
-      st->gamma = t;
-      st->beta = 0.0;
-      st->first = 0;
+      if(OP == kFinInitDefect) set_initial_defect(st, hist, sqrt(t));        // iterative.hpp:744-766
+      else if(OP == kFinAlpha) st->alpha = st->gamma / t;                     // pcg.hpp:240
+      else if(OP == kFinNewDefect) set_new_defect(st, hist, sqrt(t));         // iterative.hpp:848-879
+      else { st->beta = st->first ? 0.0 : t / st->gamma; st->gamma_new = t; } // pcg.hpp:225-231,273-279
     }
-    else { const double g2 = st->gamma; st->gamma = t; st->beta = t / g2; } // pcg.hpp:273-279
+    if(publish)
+    {
+      const unsigned c = *pub.count;
+      pub.ring[c % pub.slots] = *st;
+      __threadfence_system();
+      reinterpret_cast<volatile unsigned*>(pub.seq)[c % pub.slots] = c + 1;
+      *pub.count = c + 1;
+    }
   }
 
-  // Publication of the solver state to the host (one thread): publication c of a solve (c counted
-  // on the device in *count) goes to slot c % R of a ring in pinned host memory, and after a
-  // system-scope fence its sequence number c + 1 to seq[c % R], which the host polls.  It runs
-  // whatever the status, so every publication the host launched arrives.
-  template<int R>
-  __global__ void k_publish(const PcgState* __restrict__ st, PcgState* ring, unsigned* seq, unsigned* count)
-  {
-    if(blockIdx.x != 0 || threadIdx.x != 0) return;
-    const unsigned c = *count;
-    ring[c % R] = *st;
-    __threadfence_system();
-    reinterpret_cast<volatile unsigned*>(seq)[c % R] = c + 1;
-    *count = c + 1;
-  }
-
-  // p = beta p + z  (axpy with r == x: r = r*a + y; |beta| < eps: copy)   (pcg.hpp:281-283)
+  // p = beta p + z  (axpy with r == x: r = r*a + y; |beta| < eps: copy)   (pcg.hpp:281-283); beta from
+  // the nb partials of r.z (nb = 0: from the state); the first application has beta = 0, so p = z
+  // (pcg.hpp:225-231)
   template<typename DT_>
-  __global__ void k_pcg_update_p(u64 n, const DT_* __restrict__ z, double* __restrict__ p, const PcgState* st)
+  __global__ __launch_bounds__(256) void k_pcg_update_p(u64 n, const DT_* __restrict__ z, double* __restrict__ p, PcgState* st,
+                                                        const double* __restrict__ rz, unsigned nb)
   {
     if(st->status != kProgress) return;
-    const double beta = st->beta;
+    double beta;
+    if(nb)
+    {
+      const double t = folded_sum(rz, nb);
+      beta = st->first ? 0.0 : t / st->gamma;
+      if(blockIdx.x == 0 && threadIdx.x == 0) { st->beta = beta; st->gamma_new = t; }   // (read by no other block)
+    }
+    else
+      beta = st->beta;
     const bool copy = fabs(beta) < 2.220446049250313e-16;
     for(u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += u64(gridDim.x) * blockDim.x)
       p[i] = copy ? double(z[i]) : p[i] * beta + double(z[i]);

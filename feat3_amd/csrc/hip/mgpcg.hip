@@ -1550,7 +1550,7 @@ namespace
     DevMem ainv;
     // outer FP64 PCG
     DevCsr<double> A64own;
-    DevMem r, p, q, zcg, state, hist, partials;
+    DevMem r, p, q, zcg, state, hist, partials, partials2;
     const DevCsr<double>* A64 = nullptr;
     // the outer product by columns (lat::k_columns): its lattice (0: not) and the matrix row
     u32 out_m = 0;
@@ -1563,7 +1563,7 @@ namespace
     // publication of the state
     hipGraphExec_t gexec = nullptr;
     hipGraph_t graph = nullptr;
-    // published solver states (mg::k_publish): pinned, host-coherent; ring_dev is its device
+    // published solver states (mg::k_pcg_fin): pinned, host-coherent; ring_dev is its device
     // address, pub_count the device's count of publications in the running solve
     static constexpr int kRing = 4;
     struct HostRing
@@ -1749,7 +1749,10 @@ namespace
       // 8192 blocks (mg::row_grid), the streaming ones at most 4096
       u64 max_blocks = 8192;
       if(out_m) max_blocks = std::max<u64>(max_blocks, columns_blocks<double>(out_m));
+      // two buffers: a folding kernel reads its predecessor's partials while it writes its own
+      if(L.front()->lat >= 0) max_blocks = std::max<u64>(max_blocks, last_blocks());
       F3_RC(partials.alloc(sizeof(double) * max_blocks));
+      F3_RC(partials2.alloc(sizeof(double) * max_blocks));
       if(!ring)
       {
         F3_CHECK(hipHostMalloc(reinterpret_cast<void**>(&ring), sizeof(HostRing), hipHostMallocMapped | hipHostMallocCoherent));
@@ -1780,13 +1783,13 @@ namespace
     }
 
     // q = filter(A p) with block partials of q.p; returns the number of partials in nb
-    int outer_product(const mg::PcgState* S, unsigned& nb)
+    int outer_product(mg::PcgState* S, unsigned& nb)
     {
       double* part = partials.template as<double>();
       if(out_m)
       {
         nb = columns<lat::kColProduct, double>(out_m, out_k, 0.0, out_faces, p.template as<double>(), nullptr, q.template as<double>(),
-                                               part, reinterpret_cast<const int*>(&S->status));
+                                               part, reinterpret_cast<const int*>(&S->status), nullptr, S);
         return rt::kOk;
       }
       return with_rows<double, double>(outer_matrix(), [&](auto A, mg::RowGrid g) {
@@ -2183,7 +2186,7 @@ namespace
       F3_CHECK(hipMemcpyAsync(drepd.p, repd.data(), sizeof(T) * repd.size(), hipMemcpyHostToDevice, s));
       F3_CHECK(hipMemsetAsync(dflag.p, 0, sizeof(int), s));
       lat::k_lattice_check<T, V><<<setup_blocks(A.rows), 256, 0, s>>>(
-        A.rows, m, dim, rad, per, A.rp.template as<u32>(), A.col.template as<u32>(), A.val.template as<V>(),
+        A.rows, m, mg::udiv_magic_for(m), dim, rad, per, A.rp.template as<u32>(), A.col.template as<u32>(), A.val.template as<V>(),
         mask.template as<u32>(), dinv, drep.template as<T>(), drepd.template as<T>(), ntap, dflag.template as<int>());
       F3_RC(rt::check_launch());
       int flag = 3;
@@ -2278,7 +2281,8 @@ namespace
     }
     // one launch of lat::k_columns; returns its block count (the number of partials)
     template<int OP, typename T>
-    unsigned columns(u32 m, const T* k, T d, bool faces, const T* x, const T* rhs, T* out, double* part, const int* status)
+    unsigned columns(u32 m, const T* k, T d, bool faces, const T* x, const T* rhs, T* out, double* part, const int* status,
+                     const double* rr = nullptr, mg::PcgState* S = nullptr)
     {
       constexpr int CX = lat::ColShape<T>::CX;
       lat::ColArgs<T> a{};
@@ -2287,7 +2291,7 @@ namespace
       a.groups = (a.mm + CX - 1) / CX;
       a.gblocks = (a.groups + lat::kColThreads - 1) / lat::kColThreads;
       a.div = mg::udiv_magic_for(m);
-      a.x = x; a.rhs = rhs; a.out = out; a.partials = part; a.status = status;
+      a.x = x; a.rhs = rhs; a.out = out; a.partials = part; a.status = status; a.r = rr; a.st = S;
       for(int t = 0; t < 27; ++t) a.k[t] = k[t];
       a.d = d;
       const unsigned nb = unsigned(columns_blocks<T>(m));
@@ -2324,11 +2328,14 @@ namespace
     {
       LatTiles g;
       if(!lat_tiles<B>(m, sweeps, rest, g)) return 1e30;
-      const double reads = double(B::NC) * (B::CZ + 2 * B::RAD) / B::CZ * (sizeof(DT) / 4);
-      const double step = B::PTS / 64.0 * reads * 2.0 / 2400.0;   // LDS cycles of a step
-      const double load = 0.3 + B::PTS * 3e-4 * (sizeof(DT) / 4) * (B::MODE == 2 ? 3 : 1);
-      const double block = load + (sweeps + (rest ? 1 : 0)) * step;
-      return 3.5 + std::max(1.5 * block, double(g.blocks) / 256.0 * block);
+      // instructions of a thread's step: its multiply-adds, its LDS reads (8-byte ones count twice)
+      // and about 25 more; a CU issues one per 4 cycles for each of its four SIMDs' waves.  Measured per
+      // step and block: 2D Q2 FP32 0.65 us, 3D Q1 FP32 0.8 us (one block per CU)
+      const double instr = B::CZ * B::NTAP + B::NC * (B::CZ + 2 * B::RAD) * (sizeof(DT) / 4) + 25;
+      const double step = instr * 4.0 * (B::NT / 256.0) / 2400.0;
+      const double load = 0.3 + B::PTS * 1.5e-4 * (sizeof(DT) / 4) * (B::MODE == 2 ? 3 : 1);
+      const double block = load + (sweeps + (rest ? 1.5 : 0)) * step;
+      return 3.0 + std::max(1.2 + block, double(g.blocks) / 256.0 * block);
     }
 
     // One entry of the cycle as it is launched: an operation, or (lat) the operations of one level
@@ -2339,8 +2346,24 @@ namespace
       bool lat;
       int in, sweeps;
       bool rest, step;   // step: the restriction takes the next level's first step
+      bool last;         // the cycle's last step on the finest level, where it can sum r.z too
     };
     std::vector<PlanOp> plan;
+    bool zero_cols = false;   // the entry writes no iterate: lat::kColZero
+
+    // blocks of the cycle's last launch (the partials of r.z), 0: it sums none
+    u64 last_blocks()
+    {
+      if(plan.empty() || !plan.back().last) return 0;
+      if(!plan.back().lat) return columns_blocks<DT>(L[0]->m);
+      u64 nb = 0;
+      (void)with_brick(L[0]->lat, [&](auto b) -> int {
+        LatTiles g;
+        if(lat_tiles<decltype(b)>(L[0]->m, plan.back().sweeps, false, g)) nb = g.blocks;
+        return 0;
+      });
+      return nb;
+    }
 
     // groups the operations of the lattice levels; a run of steps is split into the launches of the
     // least estimated time (lat_cost): all in one on the small levels, where the launches count, few
@@ -2355,7 +2378,7 @@ namespace
         const CycleOp c = cycle_ops[k];
         if(L[c.lvl]->lat < 0 || L[c.lvl]->cols || c.op == Op::bottom)
         {
-          PlanOp o{c, false, 0, 0, false, false};
+          PlanOp o{c, false, 0, 0, false, false, false};
           if(c.op == Op::rest_step && L[c.lvl + 1]->lat >= 0 && !L[c.lvl + 1]->cols) { o.c.op = Op::rest; zero[c.lvl + 1] = 1; }
           plan.push_back(o);
           ++k;
@@ -2409,13 +2432,20 @@ namespace
             });
             with_rest = t <= t0 + best[0];
           }
-          plan.push_back(PlanOp{CycleOp{Op::sweep, i, 0}, true, in, n, with_rest, with_rest && step});
+          plan.push_back(PlanOp{CycleOp{Op::sweep, i, 0}, true, in, n, with_rest, with_rest && step, false});
           q -= n;
-          if(q == 0 && rest && !with_rest) plan.push_back(PlanOp{CycleOp{Op::sweep, i, 0}, true, lat::kMem, 0, true, step});
+          if(q == 0 && rest && !with_rest) plan.push_back(PlanOp{CycleOp{Op::sweep, i, 0}, true, lat::kMem, 0, true, step, false});
           in = -1;
           if(q > 0) in = lat::kMem;
         }
       }
+      // columns: the first step after the entry forms the entry's iterate itself
+      zero_cols = false;
+      if(L[0]->cols)
+        for(std::size_t k = 0; k + 1 < plan.size(); ++k)
+          if(plan[k].c.op == Op::entry) zero_cols = plan[k + 1].c.op == Op::sweep && plan[k + 1].c.lvl == 0;
+      plan.back().last = plan.back().c.lvl == 0 && !plan.back().rest &&
+                         (plan.back().lat || (L[0]->cols && plan.back().c.op == Op::sweep));
       // the buffer in which the top level's iterate ends is the one the PCG reads
       if(tail0 > 0 || tail0 + 1 >= nl)
       {
@@ -2432,7 +2462,8 @@ namespace
       }
     }
 
-    int launch_lattice(std::size_t i, const PlanOp& o, const double* def, std::vector<DT*>& cur, std::vector<DT*>& oth, const int* status)
+    int launch_lattice(std::size_t i, const PlanOp& o, const double* def, const double* dot_r, std::vector<DT*>& cur, std::vector<DT*>& oth,
+                       const int* status)
     {
       Level<DT, VT>& f = *L[i];
       return with_brick(f.lat, [&](auto b) -> int {
@@ -2444,7 +2475,8 @@ namespace
         a.nbx = g.nb[0]; a.nby = g.nb[1];
         for(int k = 0; k < 3; ++k) a.t[k] = g.t[k];
         a.hl = g.hl;
-        a.in = o.in;
+        a.in = o.in == lat::kEntry && !def ? lat::kZero : o.in;   // no def: rhs is written already
+        if(o.last && dot_r) { a.dot_r = dot_r; a.partials = partials2.template as<double>(); }
         a.sweeps = o.sweeps;
         a.restrict_ = o.rest ? 1 : 0;
         a.rhs = f.rhs.template as<DT>();
@@ -2496,12 +2528,16 @@ namespace
     // evs (statistics only): an event is recorded before every operation k with span_start[k]
     // set (span_start[0] is) and one after the last operation, so that each span of operations
     // lies between two consecutive events
+    // def: the defect to start from; null: the entry (rhs, and the iterate unless the first launch forms
+    // it) was written by the kernel before.  dot_r: the cycle's last launch also leaves the partials
+    // of dot_r . z (last_blocks() of them, where it can)
     int enqueue_vcycle(const double* def, const int* status, const std::vector<hipEvent_t>* evs = nullptr,
-                       const std::vector<char>* span_start = nullptr)
+                       const std::vector<char>* span_start = nullptr, const double* dot_r = nullptr)
     {
       const std::size_t nl = L.size();
       std::vector<DT*> cur(nl, nullptr), oth(nl, nullptr);
       std::size_t k = 0, e = 0;
+      bool fresh = true;   // before the finest level's first step
       for(const PlanOp& o : plan)
       {
         const CycleOp& c = o.c;
@@ -2511,22 +2547,29 @@ namespace
         ++k;
         if(o.lat)
         {
-          F3_RC(launch_lattice(i, o, def, cur, oth, status));
+          F3_RC(launch_lattice(i, o, def, dot_r, cur, oth, status));
           continue;
         }
         switch(c.op)
         {
           case Op::entry:
-            mg::k_mg_entry<DT><<<stream_blocks(f.n), kBlock, 0, s>>>(f.n, def, f.rhs.template as<DT>(), f.x.template as<DT>(),
-                                                                    f.dinv.template as<DT>(), status);
+            if(def)
+              mg::k_mg_entry<DT><<<stream_blocks(f.n), kBlock, 0, s>>>(f.n, def, f.rhs.template as<DT>(), entry_x(),
+                                                                      f.dinv.template as<DT>(), status);
             cur[0] = f.x.template as<DT>();
             oth[0] = f.t.template as<DT>();
             break;
           case Op::sweep:
-            if(f.cols)
+            if(f.cols && i == 0 && zero_cols && fresh)
+              columns<lat::kColZero, DT>(f.m, f.k, f.d, f.lat == 0, nullptr, f.rhs.template as<DT>(), oth[i], nullptr, status);
+            else if(f.cols && o.last && dot_r)
+              columns<lat::kColLast, DT>(f.m, f.k, f.d, f.lat == 0, cur[i], f.rhs.template as<DT>(), oth[i], partials2.template as<double>(),
+                                         status, dot_r);
+            else if(f.cols)
               columns<lat::kColSweep, DT>(f.m, f.k, f.d, f.lat == 0, cur[i], f.rhs.template as<DT>(), oth[i], nullptr, status);
             else
               F3_RC(sweep(f, cur[i], oth[i], status));
+            if(i == 0) fresh = false;
             std::swap(cur[i], oth[i]);
             break;
           case Op::defect:
@@ -2725,6 +2768,9 @@ namespace
     }
 
     const DT* z_ptr() const { return L.front()->xfinal; }
+    // where the cycle's entry writes the first iterate (null: its first launch forms it)
+    DT* entry_x() const { return zero_cols || (!plan.empty() && plan.front().lat) ? nullptr : L.front()->x.template as<DT>(); }
+    bool entry_is_op() const { return !plan.empty() && (plan.front().lat ? plan.front().in == lat::kEntry : plan.front().c.op == Op::entry); }
 
     int vcycle(double* cor, const double* def) override
     {
@@ -2737,14 +2783,6 @@ namespace
     }
 
     // ---- PCG ------------------------------------------------------------------------------
-    int enqueue_precond(const int* status)
-    {
-      if(cfg.precond == 0)
-        return enqueue_vcycle(r.template as<double>(), status);
-      mg::k_copy_filter<<<stream_blocks(n0), kBlock, 0, s>>>(n0, r.template as<double>(), mask0_ptr(), zcg.template as<double>(),
-                                                            status);
-      return rt::check_launch();
-    }
     const u32* mask0_ptr() const { return L.front()->mask.template as<u32>(); }
 
     template<typename F>
@@ -2757,23 +2795,34 @@ namespace
 
     // one-block finalisation of a reduction whose producing kernel ran with nb blocks
     template<int OP>
-    void fin(unsigned nb)
+    void fin(unsigned nb, const DevMem& part)
     {
-      mg::k_pcg_fin<OP><<<1, kBlock, 0, s>>>(partials.template as<double>(), nb, st(), hist.template as<double>());
+      mg::k_pcg_fin<OP><<<1, kBlock, 0, s>>>(part.template as<double>(), nb, st(), hist.template as<double>(),
+                                             mg::PubRing{ring_dev->st, ring_dev->seq, pub_count.template as<unsigned>(), unsigned(kRing)});
     }
 
+    // Blocks of the kernels that fold their predecessor's nb partials: a quarter of the streaming
+    // grid, since every block reads the partials (FP64 sums of 2.1 M rows: the same time)
+    static unsigned fold_blocks(u64 n) { return std::min(stream_blocks(n), 1024u); }
+
+    // the preconditioner reads the cycle's entry from rhs (and x): written with every new r
+    bool entered() const { return cfg.precond == 0 && entry_is_op(); }
+
     // outer half of a PCG iteration (pcg.hpp:236-262): q = A p, alpha, x += alpha p,
-    // r -= alpha q, the new defect and the stopping criterion
+    // r -= alpha q, the new defect, the stopping criterion and the publication of the state
     int enqueue_outer_half()
     {
       mg::PcgState* S = st();
-      double* part = partials.template as<double>();
       unsigned nb = 0;
       F3_RC(outer_product(S, nb));
-      fin<mg::kFinAlpha>(nb);
-      mg::k_pcg_update_norm<<<stream_blocks(n0), kBlock, 0, s>>>(n0, p.template as<double>(), q.template as<double>(),
-                                                                x_cur, r.template as<double>(), S, part);
-      fin<mg::kFinNewDefect>(stream_blocks(n0));
+      if(nb > mg::kFoldPartials) { fin<mg::kFinAlpha>(nb, partials); nb = 0; }
+      const unsigned ub = nb ? fold_blocks(n0) : stream_blocks(n0);
+      Level<DT, VT>& f = *L.front();
+      DT* rhs = entered() ? f.rhs.template as<DT>() : nullptr;
+      mg::k_pcg_update_norm<DT><<<ub, kBlock, 0, s>>>(n0, p.template as<double>(), q.template as<double>(), x_cur, r.template as<double>(),
+                                                     S, partials.template as<double>(), nb, partials2.template as<double>(), rhs,
+                                                     rhs ? entry_x() : nullptr, f.dinv.template as<DT>());
+      fin<mg::kFinNewDefect>(ub, partials2);
       return rt::check_launch();
     }
 
@@ -2781,31 +2830,50 @@ namespace
     int enqueue_precond_half()
     {
       mg::PcgState* S = st();
-      double* part = partials.template as<double>();
-      F3_RC(enqueue_precond(cfg.vcycle_status ? status_ptr() : nullptr));
+      const int* status = cfg.vcycle_status ? status_ptr() : nullptr;
+      const double* rr = r.template as<double>();
+      unsigned nb = 0;
+      if(cfg.precond == 0)
+      {
+        F3_RC(enqueue_vcycle(entered() ? nullptr : rr, status, nullptr, nullptr, rr));
+        nb = unsigned(last_blocks());
+      }
+      else
+      {
+        mg::k_copy_filter<<<stream_blocks(n0), kBlock, 0, s>>>(n0, rr, mask0_ptr(), zcg.template as<double>(), status);
+        F3_RC(rt::check_launch());
+      }
       F3_RC(with_z([&](auto z) {
-        mg::k_pcg_gamma_beta<<<stream_blocks(n0), kBlock, 0, s>>>(n0, z, r.template as<double>(), S, part);
-        fin<mg::kFinBeta>(stream_blocks(n0));
-        mg::k_pcg_update_p<<<stream_blocks(n0), kBlock, 0, s>>>(n0, z, p.template as<double>(), S);
+        if(nb == 0)
+        {
+          nb = fold_blocks(n0);
+          mg::k_pcg_gamma_beta<<<nb, kBlock, 0, s>>>(n0, z, rr, S, partials2.template as<double>());
+        }
+        if(nb > mg::kFoldPartials) { fin<mg::kFinBeta>(nb, partials2); nb = 0; }
+        mg::k_pcg_update_p<<<nb ? fold_blocks(n0) : stream_blocks(n0), kBlock, 0, s>>>(n0, z, p.template as<double>(), S,
+                                                                                   partials2.template as<double>(), nb);
       }));
+      return rt::check_launch();
+    }
+    // the cycle's entry for the r of the initial defect
+    int enqueue_entry()
+    {
+      if(!entered()) return rt::kOk;
+      Level<DT, VT>& f = *L.front();
+      mg::k_mg_entry<DT><<<stream_blocks(f.n), kBlock, 0, s>>>(f.n, r.template as<double>(), f.rhs.template as<DT>(), entry_x(),
+                                                              f.dinv.template as<DT>(), status_ptr());
       return rt::check_launch();
     }
 
     double* x_cur = nullptr;   // the solution vector of the running solve
     double* x_graph = nullptr; // the one the captured graph was built for
 
-    // the preconditioner half of iteration k, the outer half of iteration k + 1 and the
-    // publication of its state: one graph
+    // the preconditioner half of iteration k and the outer half of iteration k + 1, which publishes its
+    // state: one graph
     int enqueue_iteration()
     {
       F3_RC(enqueue_precond_half());
-      F3_RC(enqueue_outer_half());
-      return enqueue_publish();
-    }
-    int enqueue_publish()
-    {
-      mg::k_publish<kRing><<<1, 64, 0, s>>>(st(), ring_dev->st, ring_dev->seq, pub_count.template as<unsigned>());
-      return rt::check_launch();
+      return enqueue_outer_half();
     }
 
     int solve(double* x, const double* b, bool correct, int* status, u64* iters,
@@ -2838,17 +2906,17 @@ namespace
       {
         unsigned nb = 0;
         F3_RC(outer_defect(b, x, nb));
-        fin<mg::kFinInitDefect>(nb);
+        fin<mg::kFinInitDefect>(nb, partials);   // publication 1: the initial defect
       }
       else
       {
         // apply(cor, def): r = def, cor = 0
         F3_CHECK(hipMemsetAsync(x, 0, sizeof(double) * n0, s));
         mg::k_pcg_copy_norm<<<stream_blocks(n0), kBlock, 0, s>>>(n0, b, r.template as<double>(), part);
-        fin<mg::kFinInitDefect>(stream_blocks(n0));
+        fin<mg::kFinInitDefect>(stream_blocks(n0), partials);   // publication 1: the initial defect
       }
       F3_RC(rt::check_launch());
-      F3_RC(enqueue_publish());   // publication 1: the initial defect
+      F3_RC(enqueue_entry());
 
       // publications launched and read (in order); the host reads publication j from slot
       // (j - 1) % kRing once its sequence number reads j

@@ -1238,6 +1238,8 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     u64 num_iter, min_iter, max_iter, min_stag_iter, num_stag_iter, hist_cap;
     int status;
     int first;   // set with the initial defect: the next beta finalisation starts the recurrence
+    unsigned pub;  // publications of this solve
+    double* x;     // the solution vector (here and not in the launches, so that a captured iteration serves every x)
   };
 
   // The scalars of an iteration pass from kernel to kernel without launches of their own: a kernel that
@@ -1367,11 +1369,12 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
   // (convert_precond.hpp:104; null: not wanted) and, with dinv, its first smoothing step x0 = dinv .* rhs.
   template<typename DT_>
   __global__ __launch_bounds__(256) void k_pcg_update_norm(u64 n, const double* __restrict__ p, const double* __restrict__ q,
-                                                           double* __restrict__ x, double* __restrict__ r, PcgState* st,
+                                                           double* __restrict__ r, PcgState* st,
                                                            const double* __restrict__ pq, unsigned nb, double* partials,
                                                            DT_* __restrict__ rhs, DT_* __restrict__ x0, const DT_* __restrict__ dinv)
   {
     if(st->status != kProgress) return;
+    double* __restrict__ const x = st->x;
     double alpha;
     if(nb)
     {
@@ -1416,45 +1419,54 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     dev::block_partial(v, partials);
   }
 
-  enum : int { kFinInitDefect = 0, kFinAlpha = 1, kFinNewDefect = 2, kFinGamma = 3, kFinBeta = 4 };   // (kFinGamma: batched)
+  enum : int { kFinInitDefect = 0, kFinAlpha = 1, kFinNewDefect = 2, kFinGamma = 3, kFinBeta = 4 };   // (0 and 3: batched)
 
-  // Publication of the solver state to the host: publication c of a solve (c counted on the device in
-  // *count) goes to slot c % R of a ring in pinned host memory, and after a system-scope fence its
-  // sequence number c + 1 to seq[c % R], which the host polls.
+  // Publication of the solver state to the host: publication c of a solve (counted in the state) goes
+  // to slot c % R of a ring in pinned host memory, and after a system-scope fence its sequence number
+  // c + 1 to seq[c % R], which the host polls (and clears before a solve, when the stream is idle).
   struct PubRing
   {
     PcgState* ring;
     unsigned* seq;
-    unsigned* count;
     unsigned slots;
   };
+  __device__ __forceinline__ void publish_state(PcgState* st, const PubRing& pub)
+  {
+    const unsigned c = st->pub++;
+    pub.ring[c % pub.slots] = *st;
+    __threadfence_system();
+    reinterpret_cast<volatile unsigned*>(pub.seq)[c % pub.slots] = c + 1;
+  }
 
-  // finalisation of one PCG reduction (one block of 256 threads); the defects' also publish the
+  // the start of a solve (one block of 256 threads): the state from the host's record h, the initial
+  // defect from its partials, and the first publication
+  static __global__ __launch_bounds__(256) void k_pcg_begin(const double* __restrict__ partials, unsigned nb, PcgState h, PcgState* st,
+                                                            double* hist, PubRing pub)
+  {
+    const double t = dev::sum_partials(partials, nb);
+    if(threadIdx.x != 0) return;
+    *st = h;
+    set_initial_defect(st, hist, sqrt(t));        // iterative.hpp:744-766
+    publish_state(st, pub);
+  }
+
+  // finalisation of one PCG reduction (one block of 256 threads); the new defect's also publishes the
   // state, whatever the status, so that every publication the host launched arrives
   template<int OP>
   __global__ __launch_bounds__(256) void k_pcg_fin(const double* __restrict__ partials, unsigned nb, PcgState* st, double* hist,
                                                    PubRing pub)
   {
-    constexpr bool publish = OP == kFinInitDefect || OP == kFinNewDefect;
-    const bool run = OP == kFinInitDefect || st->status == kProgress;
-    if(!publish && !run) return;
-    const double t = run ? dev::sum_partials(partials, nb) : 0.0;   // (run is the same in every thread)
+    const bool run = st->status == kProgress;                               // (the same in every thread)
+    if(OP != kFinNewDefect && !run) return;
+    const double t = run ? dev::sum_partials(partials, nb) : 0.0;
     if(threadIdx.x != 0) return;
     if(run)
     {
-      if(OP == kFinInitDefect) set_initial_defect(st, hist, sqrt(t));        // iterative.hpp:744-766
-      else if(OP == kFinAlpha) st->alpha = st->gamma / t;                     // pcg.hpp:240
+      if(OP == kFinAlpha) st->alpha = st->gamma / t;                          // pcg.hpp:240
       else if(OP == kFinNewDefect) set_new_defect(st, hist, sqrt(t));         // iterative.hpp:848-879
       else { st->beta = st->first ? 0.0 : t / st->gamma; st->gamma_new = t; } // pcg.hpp:225-231,273-279
     }
-    if(publish)
-    {
-      const unsigned c = *pub.count;
-      pub.ring[c % pub.slots] = *st;
-      __threadfence_system();
-      reinterpret_cast<volatile unsigned*>(pub.seq)[c % pub.slots] = c + 1;
-      *pub.count = c + 1;
-    }
+    if(OP == kFinNewDefect) publish_state(st, pub);
   }
 
   // p = beta p + z  (axpy with r == x: r = r*a + y; |beta| < eps: copy)   (pcg.hpp:281-283); beta from

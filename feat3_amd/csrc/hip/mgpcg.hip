@@ -1563,8 +1563,7 @@ namespace
     // publication of the state
     hipGraphExec_t gexec = nullptr;
     hipGraph_t graph = nullptr;
-    // published solver states (mg::k_pcg_fin): pinned, host-coherent; ring_dev is its device
-    // address, pub_count the device's count of publications in the running solve
+    // published solver states (mg::publish_state): pinned, host-coherent; ring_dev is its device address
     static constexpr int kRing = 4;
     struct HostRing
     {
@@ -1573,7 +1572,6 @@ namespace
     };
     HostRing* ring = nullptr;
     HostRing* ring_dev = nullptr;
-    DevMem pub_count;
     hipEvent_t t0 = nullptr, t1 = nullptr;
     DevMem timing_state;   // solver state "in progress" for timing the outer product alone
 
@@ -1759,7 +1757,6 @@ namespace
         std::memset(ring, 0, sizeof(HostRing));
         F3_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&ring_dev), ring, 0));
       }
-      F3_RC(pub_count.alloc(sizeof(unsigned)));
       if(!t0) F3_CHECK(hipEventCreate(&t0));
       if(!t1) F3_CHECK(hipEventCreate(&t1));
       F3_CHECK(hipStreamSynchronize(s));
@@ -1772,6 +1769,14 @@ namespace
       out_m = 0;
       const Level<DT, VT>& f = *L.front();
       if(!f.cols) return rt::kOk;
+      if constexpr(std::is_same<VT, double>::value)
+      {
+        // the finest level's matrix, whose rows were compared for it
+        for(int t = 0; t < 27; ++t) out_k[t] = f.k[t];
+        out_faces = f.lat == 0;
+        out_m = f.m;
+        return rt::kOk;
+      }
       std::vector<double> rep, repd;
       bool box = false, uniform = false;
       F3_RC((lattice_rows<double, double>(*A64, f.mask, nullptr, 3, 1, f.m, rep, repd, &box, &uniform)));
@@ -2797,9 +2802,9 @@ namespace
     template<int OP>
     void fin(unsigned nb, const DevMem& part)
     {
-      mg::k_pcg_fin<OP><<<1, kBlock, 0, s>>>(part.template as<double>(), nb, st(), hist.template as<double>(),
-                                             mg::PubRing{ring_dev->st, ring_dev->seq, pub_count.template as<unsigned>(), unsigned(kRing)});
+      mg::k_pcg_fin<OP><<<1, kBlock, 0, s>>>(part.template as<double>(), nb, st(), hist.template as<double>(), pub_ring());
     }
+    mg::PubRing pub_ring() const { return mg::PubRing{ring_dev->st, ring_dev->seq, unsigned(kRing)}; }
 
     // Blocks of the kernels that fold their predecessor's nb partials: a quarter of the streaming
     // grid, since every block reads the partials (FP64 sums of 2.1 M rows: the same time)
@@ -2819,7 +2824,7 @@ namespace
       const unsigned ub = nb ? fold_blocks(n0) : stream_blocks(n0);
       Level<DT, VT>& f = *L.front();
       DT* rhs = entered() ? f.rhs.template as<DT>() : nullptr;
-      mg::k_pcg_update_norm<DT><<<ub, kBlock, 0, s>>>(n0, p.template as<double>(), q.template as<double>(), x_cur, r.template as<double>(),
+      mg::k_pcg_update_norm<DT><<<ub, kBlock, 0, s>>>(n0, p.template as<double>(), q.template as<double>(), r.template as<double>(),
                                                      S, partials.template as<double>(), nb, partials2.template as<double>(), rhs,
                                                      rhs ? entry_x() : nullptr, f.dinv.template as<DT>());
       fin<mg::kFinNewDefect>(ub, partials2);
@@ -2865,9 +2870,6 @@ namespace
       return rt::check_launch();
     }
 
-    double* x_cur = nullptr;   // the solution vector of the running solve
-    double* x_graph = nullptr; // the one the captured graph was built for
-
     // the preconditioner half of iteration k and the outer half of iteration k + 1, which publishes its
     // state: one graph
     int enqueue_iteration()
@@ -2885,13 +2887,14 @@ namespace
       h.div_rel = cfg.div_rel; h.div_abs = cfg.div_abs; h.stag_rate = cfg.stag_rate;
       h.min_iter = cfg.min_iter; h.max_iter = cfg.max_iter; h.min_stag_iter = cfg.min_stag_iter;
       h.hist_cap = hist_cap; h.status = mg::kUndefined;
-      F3_CHECK(hipMemcpyAsync(state.p, &h, sizeof(h), hipMemcpyHostToDevice, s));
-      F3_CHECK(hipMemsetAsync(pub_count.p, 0, sizeof(unsigned), s));
-      double* part = partials.template as<double>();
-      x_cur = x;
-      if(cfg.use_graph && (gexec == nullptr || x_graph != x))
+      h.x = x;
+      // no publication of an earlier solve is on its way: a solve drains the stream before it returns,
+      // unless an error ended it
+      if(running) F3_CHECK(hipStreamSynchronize(s));
+      running = true;
+      for(unsigned& q : ring->seq) __atomic_store_n(&q, 0u, __ATOMIC_RELEASE);
+      if(cfg.use_graph && gexec == nullptr)
       {
-        drop_graphs();
         F3_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         const int rc = enqueue_iteration();
         hipGraph_t g = nullptr;
@@ -2900,21 +2903,19 @@ namespace
         if(e != hipSuccess) return rt::kErrRuntime;
         graph = g;
         F3_CHECK(hipGraphInstantiate(&gexec, graph, nullptr, nullptr, 0));
-        x_graph = x;
       }
+      unsigned nb = 0;
       if(correct)
-      {
-        unsigned nb = 0;
         F3_RC(outer_defect(b, x, nb));
-        fin<mg::kFinInitDefect>(nb, partials);   // publication 1: the initial defect
-      }
       else
       {
         // apply(cor, def): r = def, cor = 0
         F3_CHECK(hipMemsetAsync(x, 0, sizeof(double) * n0, s));
-        mg::k_pcg_copy_norm<<<stream_blocks(n0), kBlock, 0, s>>>(n0, b, r.template as<double>(), part);
-        fin<mg::kFinInitDefect>(stream_blocks(n0), partials);   // publication 1: the initial defect
+        nb = stream_blocks(n0);
+        mg::k_pcg_copy_norm<<<nb, kBlock, 0, s>>>(n0, b, r.template as<double>(), partials.template as<double>());
       }
+      // publication 1: the initial defect
+      mg::k_pcg_begin<<<1, kBlock, 0, s>>>(partials.template as<double>(), nb, h, st(), hist.template as<double>(), pub_ring());
       F3_RC(rt::check_launch());
       F3_RC(enqueue_entry());
 
@@ -2982,6 +2983,7 @@ namespace
       if(epilogue) F3_RC((*epilogue)());
       while(read < launched) F3_RC(read_state());   // the last publication is the final state
       F3_CHECK(hipStreamSynchronize(s));
+      running = false;
       if(status) *status = last.status;
       if(iters) *iters = last.num_iter;
       last_hist_len = std::min<u64>(last.num_iter + 1, hist_cap);
@@ -2989,6 +2991,7 @@ namespace
     }
 
     u64 last_hist_len = 0;
+    bool running = false;   // a solve has begun and not drained the stream
 
     int history(double* out, u64 cap, u64* len) override
     {

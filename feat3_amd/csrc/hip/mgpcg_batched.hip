@@ -13,6 +13,7 @@
 // zeros); node Dirichlet bitmask; per-system PCG scalars (SysState[K]).
 
 #include "batch_kernels.hpp"
+#include "batch_lattice.hpp"
 #include "device_common.hpp"
 #include "mg_kernels.hpp"
 #include "runtime.hpp"
@@ -86,6 +87,9 @@ namespace
     // shared values: the levels of at most this many nodes (below the finest) run in one
     // LDS-resident workgroup per system (batch::k_tail_sys); 0 = every level keeps its launches
     u64 tail_nodes = 1000;
+    // 3D lattice levels whose inner rows are all alike take their steps by lines along z
+    // (batch_lattice.hpp); 0: the row kernels on every level
+    bool lattice = true;
   };
 
   // drop stored exact zeros of a scalar graph (the transfers' structural zeros)
@@ -303,6 +307,10 @@ namespace
       DevMem ea_col, ea_val, ep_col, ep_val, er_col, er_val;
       u32 aw = 0, pw = 0, rw = 0;
       DT* xfinal = nullptr;
+      // 3D lattice with one row for every inner node: nodes per axis (0: not), the row, dinv
+      u32 m = 0;
+      bool faces = false;
+      DT k[27] = {}, d = DT(0);
       const u32* order() const { return ord.p ? ord.template as<u32>() : nullptr; }
     };
     Config cfg;
@@ -312,6 +320,9 @@ namespace
     std::vector<std::unique_ptr<Level>> L;
     DevMem ainv, a64, r, p, q, st, cr, hist, partials, sums, any;
     DevMem orp, ocol;   // the outer product's graph where level 0's inner graph is thinned
+    u32 out_m = 0;      // the outer product by lines: its lattice (0: not) and row
+    bool out_faces = false;
+    double out_k[27] = {};
     u64 m0 = 0, hist_cap = 0, ncoarse_rows = 0;
     // coarse tail: levels tail0..nl-1 run in k_tail_sys when tail0 + 1 < nl (shared values);
     // tail_lds bytes of LDS hold one system's vectors on them
@@ -402,6 +413,122 @@ namespace
               L[0]->order()};
     }
 
+    // The row of a 3D lattice matrix (scalar values, or blocks that are multiples of the identity) when
+    // every inner node has the same one bit for bit, finite, on the 27 nodes of its box or on those
+    // but the six face neighbours (lat::kTapsNoFaces), and the Dirichlet nodes are exactly the
+    // lattice's boundary; returns the nodes per axis (0: not so).
+    // val holds per values per entry (1, B: diagonals, B * B: blocks), taken as the row kernels read them.
+    template<typename T, typename V>
+    u32 lattice_row(u64 nodes, const std::vector<u32>& rp, const std::vector<u32>& col, const std::vector<double>& val, u64 per,
+                    const std::vector<u32>& mask, T (&k)[27], bool& faces) const
+    {
+      const u32 m = u32(std::lround(std::cbrt(double(nodes))));
+      if(m < 3 || u64(m) * m * m != nodes || !SHARED || !cfg.lattice || cfg.tile_rows > 1) return 0;
+      for(T& v : k) v = T(0);
+      u32 taps = 0;
+      std::int64_t off[27];
+      u64 r = 0;
+      for(u32 z = 0; z < m; ++z)
+        for(u32 y = 0; y < m; ++y)
+          for(u32 x = 0; x < m; ++x, ++r)
+          {
+            const bool edge = x == 0 || y == 0 || z == 0 || x + 1 == m || y + 1 == m || z + 1 == m;
+            const bool dir = (mask[r >> 5] >> (r & 31u)) & 1u;
+            if(dir != edge) return 0;
+            if(edge) continue;
+            const u32 e0 = rp[r], count = rp[r + 1] - e0;
+            if(taps == 0)
+            {
+              // the first inner row gives the taps; their offsets ascend, so the entries must too
+              if(count == 0 || count > 27) return 0;
+              for(u32 i = 0, t = 0; i < count; ++i, ++t)
+              {
+                const std::int64_t o = std::int64_t(col[e0 + i]) - std::int64_t(r);
+                auto at = [m](u32 q) {
+                  return (std::int64_t(q / 9) - 1) * m * m + (std::int64_t(q / 3 % 3) - 1) * m + std::int64_t(q % 3) - 1;
+                };
+                while(t < 27 && at(t) != o) ++t;
+                if(t == 27) return 0;
+                taps |= 1u << t;
+                off[i] = o;
+                k[t] = T(to_storage<V>(val[u64(e0 + i) * per]));
+                if(!std::isfinite(double(k[t]))) return 0;
+              }
+              if(taps != lat::kTapsAll && taps != lat::kTapsNoFaces) return 0;
+            }
+            if(count != (taps == lat::kTapsAll ? 27u : 21u)) return 0;
+            u32 t = 0;
+            for(u32 i = 0; i < count; ++i, ++t)
+            {
+              while(!((taps >> t) & 1u)) ++t;
+              if(std::int64_t(col[e0 + i]) - std::int64_t(r) != off[i]) return 0;
+              const double* v = val.data() + u64(e0 + i) * per;
+              for(u64 h = 0; h < per; ++h)
+                if(per > u64(B) && h % u64(B + 1) != 0 ? v[h] != 0.0 : T(to_storage<V>(v[h])) != k[t]) return 0;
+            }
+          }
+      faces = taps == lat::kTapsAll;
+      return m;
+    }
+
+    // Grid of batch::k_lat_lines on a lattice of m nodes per axis (vectors of type T); wide: 16-byte
+    // accesses.  A block takes 8 threads per node -- 128 bytes of its values, one cache line -- and up
+    // to 32 lines, so that the tile's nodes and halo (6 x 5 lines: 7 KB a plane) stay in the L1 beside
+    // those of the CU's other blocks; the node's other columns go to other blocks.  Measured, 65^3
+    // nodes of 96 values, FP32 sweep / FP64 product: whole nodes in blocks of 768 threads 88 / 173 us,
+    // 256 threads 89 / 163 us; 8 threads a node in blocks of 256 83 / 142 us, 512 91 / 155 us, 1024
+    // 102 / 164 us; 4 threads a node (half lines) 120 / 200 us.
+    template<typename T>
+    batch::LatArgs<T> line_grid(u32 m, bool& wide, unsigned& nb) const
+    {
+      constexpr u32 SV = u32(16 / sizeof(T));
+      batch::LatArgs<T> a{};
+      a.m = m; a.ncol = u32(B * K); a.K = u32(K);
+      wide = a.ncol % SV == 0;
+      a.lanes = a.ncol / (wide ? SV : 1);
+      a.groups = (a.lanes + 7) / 8;
+      a.lanes = std::min<u32>(a.lanes, 8);
+      // the tile of at most 256 threads with the smallest halo
+      const u32 most = 256 / a.lanes;
+      a.nx = a.ny = 1;
+      for(u32 ny = 1; ny <= std::min<u32>(16, most); ++ny)
+      {
+        const u32 nx = std::min<u32>(16, most / ny);
+        if(u64(nx + 2) * (ny + 2) * a.nx * a.ny < u64(a.nx + 2) * (a.ny + 2) * nx * ny) { a.nx = nx; a.ny = ny; }
+      }
+      a.bx = (m + a.nx - 1) / a.nx;
+      a.by = (m + a.ny - 1) / a.ny;
+      // planes per block: about 1500 blocks (six a CU), at least 4 planes (each block reads two more)
+      const u32 lines = a.bx * a.by * a.groups;
+      const u32 chunks = std::max<u32>(1, std::min<u32>((1500 + lines - 1) / lines, m / 4));
+      a.zlen = (m + chunks - 1) / chunks;
+      nb = lines * ((m + a.zlen - 1) / a.zlen);
+      return a;
+    }
+
+    // one launch of batch::k_lat_lines; returns its block count (the number of partials)
+    template<int OP, typename T>
+    unsigned lines(u32 m, const T (&k)[27], T d, bool faces, const T* x, const T* rhs, T* out, const int* any_)
+    {
+      constexpr int SV = int(16 / sizeof(T));
+      bool wide = false;
+      unsigned nb = 0;
+      batch::LatArgs<T> a = line_grid<T>(m, wide, nb);
+      a.x = x; a.rhs = rhs; a.out = out; a.any = any_;
+      a.partials = partials.template as<double>();
+      for(int t = 0; t < 27; ++t) a.k[t] = k[t];
+      a.d = d;
+      const unsigned nt = (a.lanes * a.nx * a.ny + 63) / 64 * 64;
+      const unsigned lds = OP == batch::kLatProduct || OP == batch::kLatInit ? unsigned(sizeof(double)) * a.nx * a.ny * a.lanes * (wide ? SV : 1) : 0u;
+      auto go = [&](auto ch) {
+        constexpr int C = decltype(ch)::value;
+        if(faces) batch::k_lat_lines<T, C, lat::kTapsAll, OP><<<nb, nt, lds, s>>>(a);
+        else batch::k_lat_lines<T, C, lat::kTapsNoFaces, OP><<<nb, nt, lds, s>>>(a);
+      };
+      if(wide) go(ic<SV>()); else go(ic<1>());
+      return nb;
+    }
+
     int init(const std::vector<HostLevel>& lv, const Config& c, hipStream_t stream) override
     {
       cfg = c;
@@ -413,6 +540,8 @@ namespace
         const HostLevel& h = lv[i];
         std::unique_ptr<Level> l(new Level());
         l->nodes = h.nodes;
+        std::vector<u32> m((h.nodes + 31) / 32 + 1, 0u);
+        for(u32 f : h.fidx) m[f >> 5] |= 1u << (f & 31u);
         if(SHARED && sizeof(VT) < 8)
         {
           const HostGraph T = thin_graph(h.A, vpe(), B);
@@ -420,7 +549,9 @@ namespace
           l->nnz = T.rp[h.nodes];
           F3_RC(l->arp.put(T.rp, s));
           F3_RC(l->acol.put(T.col, s));
-          F3_RC(l->aval.put(conv<VT>(stored(T.val)), s));
+          const std::vector<double> tv = stored(T.val);
+          F3_RC(l->aval.put(conv<VT>(tv), s));
+          l->m = lattice_row<DT, VT>(h.nodes, T.rp, T.col, tv, svpe(), m, l->k, l->faces);
           F3_CHECK(hipStreamSynchronize(s));   // T leaves scope
         }
         else
@@ -428,7 +559,9 @@ namespace
           l->nnz = h.A.rp[h.nodes];
           F3_RC(l->arp.put(h.A.rp, s));
           F3_RC(l->acol.put(h.A.col, s));
-          F3_RC(l->aval.put(conv<VT>(stored(h.A.val)), s));
+          const std::vector<double> av = stored(h.A.val);
+          F3_RC(l->aval.put(conv<VT>(av), s));
+          l->m = lattice_row<DT, VT>(h.nodes, h.A.rp, h.A.col, av, svpe(), m, l->k, l->faces);
         }
         if(i + 1 < lv.size())
         {
@@ -437,8 +570,6 @@ namespace
           F3_RC(l->prp.put(P.rp, s)); F3_RC(l->pcol.put(P.col, s)); F3_RC(l->pval.put(conv<VT>(P.val), s));
           F3_RC(l->rrp.put(R.rp, s)); F3_RC(l->rcol.put(R.col, s)); F3_RC(l->rval.put(conv<VT>(R.val), s));
         }
-        std::vector<u32> m((h.nodes + 31) / 32 + 1, 0u);
-        for(u32 f : h.fidx) m[f >> 5] |= 1u << (f & 31u);
         F3_RC(l->mask.put(m, s));
         if(cfg.tile_rows > 1 && h.nodes > cfg.tile_rows)
         {
@@ -463,6 +594,12 @@ namespace
                 }
         }
         F3_RC(l->dinv.put(dinv, s));
+        if(l->m)
+        {
+          // the rows are alike, so is dinv (an inner node: 1 + m + m^2)
+          l->d = dinv[(1 + u64(l->m) + u64(l->m) * l->m) * B * kv];
+          if(!std::isfinite(double(l->d))) l->m = 0;
+        }
         const u64 nv = h.nodes * B * u64(K);
         F3_RC(l->rhs.alloc(sizeof(DT) * nv)); F3_RC(l->x.alloc(sizeof(DT) * nv));
         F3_RC(l->t.alloc(sizeof(DT) * nv)); F3_RC(l->def.alloc(sizeof(DT) * nv));
@@ -607,7 +744,15 @@ namespace
     {
       // outer FP64
       m0 = l0.nodes * B;
-      F3_RC(a64.put(stored(l0.A.val), s));
+      const std::vector<double> ov = stored(l0.A.val);
+      F3_RC(a64.put(ov, s));
+      out_m = 0;
+      if(L[0]->m)
+      {
+        std::vector<u32> m((l0.nodes + 31) / 32 + 1, 0u);
+        for(u32 f : l0.fidx) m[f >> 5] |= 1u << (f & 31u);
+        out_m = lattice_row<double, double>(l0.nodes, l0.A.rp, l0.A.col, ov, svpe(), m, out_k, out_faces);
+      }
       if(L[0]->thinned)
       {
         F3_RC(orp.put(l0.A.rp, s));
@@ -619,7 +764,15 @@ namespace
       F3_RC(cr.alloc(sizeof(batch::Criteria)));
       hist_cap = cfg.max_iter + 2;
       F3_RC(hist.alloc(sizeof(double) * hist_cap * K));
-      F3_RC(partials.alloc(sizeof(double) * 8192 * u64(K)));
+      u64 np = 8192;
+      if(out_m)
+      {
+        bool wide = false;
+        unsigned nb = 0;
+        (void)line_grid<double>(out_m, wide, nb);
+        np = std::max<u64>(np, nb);
+      }
+      F3_RC(partials.alloc(sizeof(double) * np * u64(K)));
       F3_RC(sums.alloc(sizeof(double) * u64(K)));
       F3_RC(any.alloc(64));
       if(!ring)
@@ -648,6 +801,11 @@ namespace
 
     int sweep(Level& f, DT* xin, DT* xout, const int* a)
     {
+      if(f.m)
+      {
+        lines<batch::kLatSweep, DT>(f.m, f.k, f.d, f.faces, xin, f.rhs.template as<DT>(), xout, a);
+        return rt::kOk;
+      }
       return with_layout<DT>(GV, S, [&](auto gv, auto sv) {
         constexpr int Gc = decltype(gv)::value, Sc = decltype(sv)::value;
         const mg::RowGrid g = vcycle_grid(f.nodes, Gc);
@@ -658,6 +816,11 @@ namespace
 
     int defect(Level& f, const DT* x, const int* a)
     {
+      if(f.m)
+      {
+        lines<batch::kLatDefect, DT>(f.m, f.k, f.d, f.faces, x, f.rhs.template as<DT>(), f.def.template as<DT>(), a);
+        return rt::kOk;
+      }
       return with_layout<DT>(GV, S, [&](auto gv, auto sv) {
         constexpr int Gc = decltype(gv)::value, Sc = decltype(sv)::value;
         const mg::RowGrid g = vcycle_grid(f.nodes, Gc);
@@ -744,6 +907,11 @@ namespace
     // outer q = filter(A p) with partials of q.p; returns the number of blocks (the partial count)
     int outer_spmv_dot(unsigned& nb)
     {
+      if(out_m)
+      {
+        nb = lines<batch::kLatProduct, double>(out_m, out_k, 0.0, out_faces, p.template as<double>(), nullptr, q.template as<double>(), anyp());
+        return rt::kOk;
+      }
       return with_layout<double>(GO, SO, [&](auto gv, auto sv) {
         constexpr int Gc = decltype(gv)::value, Sc = decltype(sv)::value;
         const mg::RowGrid g = mg::row_grid(L[0]->nodes, Gc);
@@ -757,6 +925,11 @@ namespace
 
     int outer_defect(const double* b, const double* x, unsigned& nb)
     {
+      if(out_m)
+      {
+        nb = lines<batch::kLatInit, double>(out_m, out_k, 0.0, out_faces, x, b, r.template as<double>(), nullptr);
+        return rt::kOk;
+      }
       return with_layout<double>(GO, SO, [&](auto gv, auto sv) {
         constexpr int Gc = decltype(gv)::value, Sc = decltype(sv)::value;
         const mg::RowGrid g = mg::row_grid(L[0]->nodes, Gc);
@@ -962,6 +1135,13 @@ namespace
       // a thinned graph or the block-diagonal storage was chosen for the values given at init;
       // other values need a new solver
       if(l.thinned || DIAG) return rt::kErrState;
+      // the new values' rows need not be alike
+      if(l.m || (level == 0 && out_m))
+      {
+        l.m = 0;
+        if(level == 0) out_m = 0;
+        drop_graphs();
+      }
       const u64 nval = l.nnz * vals_per_entry();
       const unsigned nb = unsigned(std::max<u64>(1, std::min<u64>((nval + 255) / 256, 65536)));
       k_to_storage<VT><<<nb, 256, 0, s>>>(nval, dv, l.aval.template as<VT>());
@@ -1023,7 +1203,9 @@ namespace
         // algorithmic: values + column indices + row pointers, x once, and the row-wise vectors
         // (sweep: rhs, x_out, dinv; outer: p read for the dot is the x read, q written)
         const u64 nvk = f.nodes * B * u64(K);
-        if(which == 2)
+        if(which == 2 ? out_m : f.m)   // one row for all nodes: the vectors alone
+          *bytes = which == 2 ? nvk * 8 * 2 : nvk * sizeof(DT) * 3;
+        else if(which == 2)
           *bytes = f.nnz * (vals_per_entry() * 8 + 4) + (f.nodes + 1) * 4 + nvk * 8 * 2;
         else
           *bytes = f.nnz * (vals_per_entry() * sizeof(VT) + 4) + (f.nodes + 1) * 4 + nvk * sizeof(DT) * 3 +
@@ -1158,6 +1340,7 @@ int feat3_batch_set_option(feat3_batch* h, const char* name, double value)
   if(n == "tile_rows" && value >= 0) h->cfg.tile_rows = u64(value);
   else if(n == "diag_blocks") h->cfg.diag_blocks = value != 0.0;
   else if(n == "tail_max_n" && value >= 0) h->cfg.tail_nodes = u64(value);
+  else if(n == "lattice") h->cfg.lattice = value != 0.0;
   else return rt::kErrArg;
   h->eng.reset();
   return rt::kOk;

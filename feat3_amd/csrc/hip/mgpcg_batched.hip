@@ -14,6 +14,7 @@
 
 #include "batch_kernels.hpp"
 #include "batch_lattice.hpp"
+#include "batch_rows.hpp"
 #include "device_common.hpp"
 #include "mg_kernels.hpp"
 #include "runtime.hpp"
@@ -88,7 +89,8 @@ namespace
     // LDS-resident workgroup per system (batch::k_tail_sys); 0 = every level keeps its launches
     u64 tail_nodes = 1000;
     // 3D lattice levels whose inner rows are all alike take their steps by lines along z
-    // (batch_lattice.hpp); 0: the row kernels on every level
+    // (batch_lattice.hpp), 2D lattice levels with one matrix per system several steps a pass
+    // (batch_rows.hpp); 0: the row kernels on every level
     bool lattice = true;
   };
 
@@ -311,6 +313,7 @@ namespace
       u32 m = 0;
       bool faces = false;
       DT k[27] = {}, d = DT(0);
+      u32 fm = 0;             // 2D 9-point lattice with values per system: nodes per axis (0: not)
       const u32* order() const { return ord.p ? ord.template as<u32>() : nullptr; }
     };
     Config cfg;
@@ -529,6 +532,102 @@ namespace
       return nb;
     }
 
+    // A level with values per system whose graph is the 9-point lattice of m x m nodes (rows and
+    // columns ascending, m >= kFieldNodes), with the boundary as its Dirichlet nodes: m, else 0.  The
+    // graph is all that matters, so values may change (set_values).
+    u32 field_lattice(u64 nodes, const std::vector<u32>& rp, const std::vector<u32>& col, const std::vector<u32>& mask) const
+    {
+      const u32 m = u32(std::lround(std::sqrt(double(nodes))));
+      if(SHARED || B != 1 || m < kFieldNodes || u64(m) * m != nodes || !cfg.lattice || cfg.tile_rows > 1) return 0;
+      u64 r = 0;
+      for(u32 y = 0; y < m; ++y)
+        for(u32 x = 0; x < m; ++x, ++r)
+        {
+          const bool edge = x == 0 || y == 0 || x + 1 == m || y + 1 == m;
+          if(bool((mask[r >> 5] >> (r & 31u)) & 1u) != edge) return 0;
+          if(edge) continue;
+          const u64 e = batch::field_entry(m, x, y);
+          if(rp[r] != e || rp[r + 1] != e + 9) return 0;
+          for(u32 t = 0; t < 9; ++t)
+            if(u64(col[e + t]) != r + u64(t / 3) * m + t % 3 - m - 1) return 0;
+        }
+      return m;
+    }
+
+    // Steps of one pass at most (batch::k_field_rows): the registers of 1024 threads (128 each) hold the
+    // rows of four FP32 steps, of three with binary16 values (converted at each use) or two FP64 ones.
+    static constexpr int kFieldSteps = sizeof(DT) == 8 ? 2 : sizeof(VT) == 2 ? 3 : 4;
+    static constexpr u32 kFieldNodes = 100;
+
+    // the next pass of `left` steps on level f: its number of steps (1: the row kernels)
+    static int field_pass(const Level& f, int left)
+    {
+      if(!f.fm || left < 2) return 1;
+      const int n = std::min(left, kFieldSteps);
+      return left - n == 1 && n > 2 ? n - 1 : n;
+    }
+
+    template<int NS, bool DEF>
+    int field_rows(Level& f, const DT* xin, DT* xout, const int* any_)
+    {
+      if constexpr(!SHARED && B == 1 && NS <= kFieldSteps)
+      {
+        batch::FieldArgs<DT, VT> a{};
+        a.m = f.fm; a.K = u32(K);
+        a.groups = (a.K + 15) / 16;
+        a.lanes = (a.K + a.groups - 1) / a.groups;
+        a.nx = batch::kFieldThreads / a.lanes;
+        const u32 wide = a.nx - 2 * NS;
+        a.bx = (a.m + wide - 1) / wide;
+        // one block per CU: as many chunks of rows as make about 256 blocks, none shorter than NS rows
+        const u32 chunks = std::max<u32>(1, std::min<u32>(256 / (a.bx * a.groups), a.m / NS));
+        a.ylen = (a.m + chunks - 1) / chunks;
+        const unsigned nb = a.groups * a.bx * ((a.m + a.ylen - 1) / a.ylen);
+        a.val = f.aval.template as<VT>();
+        a.dinv = f.dinv.template as<DT>();
+        a.rhs = f.rhs.template as<DT>();
+        a.x = xin; a.out = xout; a.def = f.def.template as<DT>();
+        a.any = any_;
+        batch::k_field_rows<DT, VT, NS, DEF><<<nb, batch::kFieldThreads, 0, s>>>(a);
+        return rt::kOk;
+      }
+      (void)f; (void)xin; (void)xout; (void)any_;
+      return rt::kErrState;
+    }
+
+    // n smoothing steps of level f from cur (oth: the other iterate), then its defect if asked for
+    int smooth(Level& f, DT*& cur, DT*& oth, int n, bool def, const int* a)
+    {
+      for(int left = n + (def ? 1 : 0); left > 0;)
+      {
+        const int ns = field_pass(f, left);
+        left -= ns;
+        const bool d = def && left == 0;
+        if(ns == 1)
+        {
+          if(d) { F3_RC(defect(f, cur, a)); continue; }
+          F3_RC(sweep(f, cur, oth, a));
+        }
+        else if(ns == 2) F3_RC(d ? field_rows<2, true>(f, cur, oth, a) : field_rows<2, false>(f, cur, oth, a));
+        else if(ns == 3) F3_RC(d ? field_rows<3, true>(f, cur, oth, a) : field_rows<3, false>(f, cur, oth, a));
+        else F3_RC(d ? field_rows<4, true>(f, cur, oth, a) : field_rows<4, false>(f, cur, oth, a));
+        std::swap(cur, oth);
+      }
+      return rt::kOk;
+    }
+    // how often smooth() swaps the iterates
+    static int swaps(const Level& f, int n, bool def)
+    {
+      int k = 0;
+      for(int left = n + (def ? 1 : 0); left > 0;)
+      {
+        const int ns = field_pass(f, left);
+        left -= ns;
+        k += ns > 1 || !(def && left == 0);
+      }
+      return k;
+    }
+
     int init(const std::vector<HostLevel>& lv, const Config& c, hipStream_t stream) override
     {
       cfg = c;
@@ -562,6 +661,7 @@ namespace
           const std::vector<double> av = stored(h.A.val);
           F3_RC(l->aval.put(conv<VT>(av), s));
           l->m = lattice_row<DT, VT>(h.nodes, h.A.rp, h.A.col, av, svpe(), m, l->k, l->faces);
+          l->fm = field_lattice(h.nodes, h.A.rp, h.A.col, m);
         }
         if(i + 1 < lv.size())
         {
@@ -609,7 +709,7 @@ namespace
       coarse_host = lv.back();
       F3_RC(coarse_inverses(coarse_host.A.val));
       for(std::size_t i = 0; i + 1 < L.size(); ++i)
-        L[i]->xfinal = ((cfg.pre - 1 + cfg.post) % 2 == 0) ? L[i]->x.template as<DT>() : L[i]->t.template as<DT>();
+        L[i]->xfinal = ((swaps(*L[i], cfg.pre - 1, true) + swaps(*L[i], cfg.post, false)) % 2 == 0) ? L[i]->x.template as<DT>() : L[i]->t.template as<DT>();
       L.back()->xfinal = L.back()->x.template as<DT>();
       F3_RC(setup_tail());
       return init_outer(lv[0]);
@@ -866,8 +966,7 @@ namespace
         Level& c = *L[i + 1];
         cur[i] = f.x.template as<DT>();
         oth[i] = f.t.template as<DT>();
-        for(int k = 1; k < cfg.pre; ++k) { F3_RC(sweep(f, cur[i], oth[i], a)); std::swap(cur[i], oth[i]); }
-        F3_RC(defect(f, cur[i], a));
+        F3_RC(smooth(f, cur[i], oth[i], cfg.pre - 1, true, a));
         F3_RC(restrict_to(f, c, (i + 1 < tail0) ? c.x.template as<DT>() : nullptr, a));
       }
       if constexpr(SHARED)
@@ -888,7 +987,7 @@ namespace
         Level& f = *L[i];
         Level& c = *L[i + 1];
         F3_RC(prolong(f, c.xfinal, cur[i], a));
-        for(int k = 0; k < cfg.post; ++k) { F3_RC(sweep(f, cur[i], oth[i], a)); std::swap(cur[i], oth[i]); }
+        F3_RC(smooth(f, cur[i], oth[i], cfg.post, false, a));
         if(cur[i] != f.xfinal) return rt::kErrState;
       }
       return rt::check_launch();

@@ -498,7 +498,7 @@ namespace batch
     }
   }
 
-  // ---- coarse tail of the shared-values solver: one workgroup per system ----------------------
+  // ---- coarse tail: one workgroup per system --------------------------------------------------
   //
   // Below about a thousand nodes a level step is a launch of 5-7 us that moves a few hundred KB.
   // k_tail_sys runs the V-cycle's part on the levels tail[0] (entered from the restriction above,
@@ -506,7 +506,8 @@ namespace batch
   // kTailSysThreads per system, with barriers between the steps.  The system's vectors on these
   // levels live in LDS ([node][h]: x0, x1, rhs, def, dinv; 5 * nodes * B values per level); the
   // shared matrices are read from global memory in ELL order (TailSysEll: the entries of a wave's
-  // rows coalesced), where the K workgroups keep them L2-resident.
+  // rows coalesced), where the K workgroups keep them L2-resident.  With values per system (PER_)
+  // every workgroup has an ELL copy of its own.
   // A thread takes a node and its B components.  Every step sums a row's terms in the order of
   // k_sweep / k_defect / k_restrict / k_prolong / k_coarse with the same expressions, so the
   // results are bit for bit those of the per-level launches.
@@ -531,8 +532,25 @@ namespace batch
     u32 nodes, off;                // nodes; offset of the level's vectors in LDS (DT_ elements)
     TailSysEll<VT_> A, P, R;       // P: rows = this level's nodes; R: rows = the next coarser level's
     const u32* mask;
-    const DT_* dinv;               // [node][h]
+    const DT_* dinv;               // [node][h], [node][k] with values per system
   };
+
+  // the same for values per system (val [entry][k]): one ELL copy [k][entry of the row][row] per system
+  template<typename VT_>
+  __global__ void k_tail_ell_sys(u32 rows, u32 w, u32 K, const u32* __restrict__ rp, const u32* __restrict__ col,
+                                 const VT_* __restrict__ val, u32* __restrict__ ecol, VT_* __restrict__ eval)
+  {
+    const u64 n = u64(rows) * w * K;
+    for(u64 i = u64(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += u64(gridDim.x) * blockDim.x)
+    {
+      const u32 k = u32(i % K);
+      const u64 j = i / K;
+      const u32 t = u32(j % w), r = u32(j / w), e = rp[r] + t;
+      const bool in = e < rp[r + 1];
+      if(k == 0) ecol[u64(t) * rows + r] = in ? col[e] : 0u;
+      eval[(u64(k) * w + t) * rows + r] = in ? val[u64(e) * K + k] : VT_(0.0f);
+    }
+  }
 
   // ELL copy of a CSR matrix with V values per entry (TailSysEll), one thread per (row, k)
   template<typename VT_>
@@ -648,7 +666,7 @@ namespace batch
   // grid: K workgroups of kTailSysThreads (workgroup k = system k); dynamic LDS: the levels'
   // vectors.  Level li's iterate alternates between its buffers x0 and x1; the coarsest level's
   // solution is x0.
-  template<typename DT_, typename VT_, int B_, bool DIAG_>
+  template<typename DT_, typename VT_, int B_, bool DIAG_, bool PER_ = false>
   __global__ __launch_bounds__(kTailSysThreads) void k_tail_sys(TailSysDesc<DT_, VT_> d, int K, const int* any)
   {
     if(idle(any)) return;
@@ -656,6 +674,12 @@ namespace batch
     DT_* arena = reinterpret_cast<DT_*>(tail_sys_arena_);
     const u32 tid = threadIdx.x;
     const u64 k = blockIdx.x;
+    // level l's matrix as this system sees it
+    auto mat = [&](const TailSysLevel<DT_, VT_>& l) {
+      TailSysEll<VT_> A = l.A;
+      if constexpr(PER_) A.val += k * u64(A.w) * A.rows;
+      return A;
+    };
     // dinv of every level; tail[0]'s right-hand side and first smoothing step x0 = dinv rhs
     for(int i = 0; i < d.nlev; ++i)
     {
@@ -664,7 +688,7 @@ namespace batch
       DT_* v = arena + l.off;
       for(u32 r = tid; r < n; r += kTailSysThreads)
       {
-        const DT_ di = l.dinv[r];
+        const DT_ di = l.dinv[PER_ ? u64(r) * u64(K) + k : u64(r)];
         v[4 * n + r] = di;
         if(i == 0)
         {
@@ -688,7 +712,7 @@ namespace batch
       for(u32 p = tid; p < l.nodes; p += kTailSysThreads)
       {
         DT_ s[B_];
-        tail_sys_block_row<DT_, VT_, B_, DIAG_>(l.A, p, xi, s);
+        tail_sys_block_row<DT_, VT_, B_, DIAG_>(mat(l), p, xi, s);
 #pragma unroll
         for(int h = 0; h < B_; ++h)
         {
@@ -711,7 +735,7 @@ namespace batch
       for(u32 p = tid; p < f.nodes; p += kTailSysThreads)
       {
         DT_ s[B_];
-        tail_sys_block_row<DT_, VT_, B_, DIAG_>(f.A, p, fv + cur(li) * n, s);
+        tail_sys_block_row<DT_, VT_, B_, DIAG_>(mat(f), p, fv + cur(li) * n, s);
         const bool m = masked(f.mask, p);
 #pragma unroll
         for(int h = 0; h < B_; ++h)
@@ -746,7 +770,7 @@ namespace batch
       const u32 m = d.ncoarse;
       for(u32 i = tid; i < m; i += kTailSysThreads)
       {
-        const double* a = d.ainv + u64(i) * m;
+        const double* a = d.ainv + (PER_ ? k * m * m : 0) + u64(i) * m;
         double s = 0.0;
 #pragma unroll 8
         for(u32 j = 0; j < m; ++j) s += a[j] * double(cv[2 * m + j]);

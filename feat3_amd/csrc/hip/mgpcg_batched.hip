@@ -88,6 +88,9 @@ namespace
     // shared values: the levels of at most this many nodes (below the finest) run in one
     // LDS-resident workgroup per system (batch::k_tail_sys); 0 = every level keeps its launches
     u64 tail_nodes = 1000;
+    // the same limit with values per system.  Forward, adjoint and gradient of 16 fields at 2D level 10:
+    // no tail 33.0 ms, from 17^2 nodes 31.6, 33^2 31.4, 65^2 32.0 (16 workgroups on 256 CUs)
+    u64 tail_fields = 1100;
     // 3D lattice levels whose inner rows are all alike take their steps by lines along z
     // (batch_lattice.hpp), 2D lattice levels with one matrix per system several steps a pass
     // (batch_rows.hpp); 0: the row kernels on every level
@@ -557,7 +560,7 @@ namespace
     // Steps of one pass at most (batch::k_field_rows): the registers of 1024 threads (128 each) hold the
     // rows of four FP32 steps, of three with binary16 values (converted at each use) or two FP64 ones.
     static constexpr int kFieldSteps = sizeof(DT) == 8 ? 2 : sizeof(VT) == 2 ? 3 : 4;
-    static constexpr u32 kFieldNodes = 100;
+    static constexpr u32 kFieldNodes = 100;   // 129^2: 17 us a pass against 4 x 4.9 us; 65^2: 4 x 4.3 us
 
     // the next pass of `left` steps on level f: its number of steps (1: the row kernels)
     static int field_pass(const Level& f, int left)
@@ -722,7 +725,8 @@ namespace
       const std::size_t nl = L.size();
       tail0 = nl - 1;
       tail_lds = 0;
-      if(!SHARED || cfg.tail_nodes == 0) return rt::kOk;
+      const u64 most = SHARED ? cfg.tail_nodes : cfg.tail_fields;
+      if(most == 0) return rt::kOk;
       int dev = 0, cap = 65536;
       if(hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cap, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
       auto bytes = [&](std::size_t t0) {
@@ -730,7 +734,7 @@ namespace
         for(std::size_t i = t0; i < nl; ++i) b += 5 * L[i]->nodes * u64(B) * sizeof(DT);
         return b;
       };
-      while(tail0 > 0 && L[tail0 - 1]->nodes <= cfg.tail_nodes && nl - (tail0 - 1) <= std::size_t(batch::kTailSysMax) &&
+      while(tail0 > 0 && L[tail0 - 1]->nodes <= most && nl - (tail0 - 1) <= std::size_t(batch::kTailSysMax) &&
             bytes(tail0 - 1) <= u64(cap))
         --tail0;
       if(tail0 + 1 >= nl) return rt::kOk;
@@ -738,7 +742,7 @@ namespace
       for(std::size_t i = tail0; i < nl; ++i)
       {
         Level& l = *L[i];
-        F3_RC(tail_ell(l.arp, l.acol, l.aval, l.nodes, u32(svpe()), l.ea_col, l.ea_val, l.aw));
+        F3_RC(tail_ell(l.arp, l.acol, l.aval, l.nodes, u32(svpe()), l.ea_col, l.ea_val, l.aw, !SHARED));
         if(i + 1 < nl)
         {
           F3_RC(tail_ell(l.prp, l.pcol, l.pval, l.nodes, 1u, l.ep_col, l.ep_val, l.pw));
@@ -746,30 +750,35 @@ namespace
         }
       }
       F3_CHECK(hipStreamSynchronize(s));
-      if constexpr(SHARED)
-      {
-        if(tail_lds > 65536)
-          F3_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&batch::k_tail_sys<DT, VT, B, DIAG>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(tail_lds)));
-      }
+      if(tail_lds > 65536)
+        F3_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&batch::k_tail_sys<DT, VT, B, DIAG, !SHARED>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(tail_lds)));
       return rt::kOk;
     }
 
     // ELL copy (batch::TailSysEll) of a device CSR matrix of `rows` rows with V values per
-    // entry; w = its longest row.  Rebuilt from the CSR values when they change (set_values).
-    int tail_ell(const DevMem& rp, const DevMem& col, const DevMem& val, u64 rows, u32 V, DevMem& ecol, DevMem& eval, u32& w)
+    // entry (sys: one value per system and entry); w = its longest row.  Rebuilt from the CSR values when they change (set_values).
+    int tail_ell(const DevMem& rp, const DevMem& col, const DevMem& val, u64 rows, u32 V, DevMem& ecol, DevMem& eval, u32& w,
+                 bool sys = false)
     {
-      std::vector<u32> h(rows + 1);
-      F3_CHECK(hipMemcpyAsync(h.data(), rp.p, sizeof(u32) * (rows + 1), hipMemcpyDeviceToHost, s));
-      F3_CHECK(hipStreamSynchronize(s));
-      w = 0;
-      for(u64 r = 0; r < rows; ++r) w = std::max(w, h[r + 1] - h[r]);
-      if(w == 0) w = 1;
-      if(!ecol.p) F3_RC(ecol.alloc(sizeof(u32) * rows * w));
-      if(!eval.p) F3_RC(eval.alloc(sizeof(VT) * rows * w * V));
-      const u64 n = rows * w;
+      if(!ecol.p)   // the graph stays when values change
+      {
+        std::vector<u32> h(rows + 1);
+        F3_CHECK(hipMemcpyAsync(h.data(), rp.p, sizeof(u32) * (rows + 1), hipMemcpyDeviceToHost, s));
+        F3_CHECK(hipStreamSynchronize(s));
+        w = 0;
+        for(u64 r = 0; r < rows; ++r) w = std::max(w, h[r + 1] - h[r]);
+        if(w == 0) w = 1;
+        F3_RC(ecol.alloc(sizeof(u32) * rows * w));
+        F3_RC(eval.alloc(sizeof(VT) * rows * w * (sys ? u64(K) : V)));
+      }
+      const u64 n = rows * w * (sys ? u64(K) : 1);
       const unsigned nb = unsigned(std::max<u64>(1, std::min<u64>((n + 255) / 256, 65536)));
-      batch::k_tail_ell<VT><<<nb, 256, 0, s>>>(u32(rows), w, V, rp.template as<u32>(), col.template as<u32>(),
+      if(sys)
+        batch::k_tail_ell_sys<VT><<<nb, 256, 0, s>>>(u32(rows), w, u32(K), rp.template as<u32>(), col.template as<u32>(),
+                                                     val.template as<VT>(), ecol.template as<u32>(), eval.template as<VT>());
+      else
+        batch::k_tail_ell<VT><<<nb, 256, 0, s>>>(u32(rows), w, V, rp.template as<u32>(), col.template as<u32>(),
                                                val.template as<VT>(), ecol.template as<u32>(), eval.template as<VT>());
       return rt::check_launch();
     }
@@ -969,11 +978,8 @@ namespace
         F3_RC(smooth(f, cur[i], oth[i], cfg.pre - 1, true, a));
         F3_RC(restrict_to(f, c, (i + 1 < tail0) ? c.x.template as<DT>() : nullptr, a));
       }
-      if constexpr(SHARED)
-      {
-        if(tail0 + 1 < nl)
-          batch::k_tail_sys<DT, VT, B, DIAG><<<unsigned(K), batch::kTailSysThreads, tail_lds, s>>>(tail_desc(), K, a);
-      }
+      if(tail0 + 1 < nl)
+        batch::k_tail_sys<DT, VT, B, DIAG, !SHARED><<<unsigned(K), batch::kTailSysThreads, tail_lds, s>>>(tail_desc(), K, a);
       if(tail0 + 1 >= nl)
       {
         Level& cl = *L.back();
@@ -1252,7 +1258,7 @@ namespace
                                                    l.dinv.template as<DT>());
       F3_RC(rt::check_launch());
       if(tail0 + 1 < L.size() && std::size_t(level) >= tail0)
-        F3_RC(tail_ell(l.arp, l.acol, l.aval, l.nodes, u32(svpe()), l.ea_col, l.ea_val, l.aw));
+        F3_RC(tail_ell(l.arp, l.acol, l.aval, l.nodes, u32(svpe()), l.ea_col, l.ea_val, l.aw, !SHARED));
       if(level == 0) F3_CHECK(hipMemcpyAsync(a64.p, dv, sizeof(double) * nval, hipMemcpyDeviceToDevice, s));
       if(level + 1 == int(L.size()))
       {
@@ -1438,7 +1444,7 @@ int feat3_batch_set_option(feat3_batch* h, const char* name, double value)
   const std::string n(name);
   if(n == "tile_rows" && value >= 0) h->cfg.tile_rows = u64(value);
   else if(n == "diag_blocks") h->cfg.diag_blocks = value != 0.0;
-  else if(n == "tail_max_n" && value >= 0) h->cfg.tail_nodes = u64(value);
+  else if(n == "tail_max_n" && value >= 0) h->cfg.tail_nodes = h->cfg.tail_fields = u64(value);
   else if(n == "lattice") h->cfg.lattice = value != 0.0;
   else return rt::kErrArg;
   h->eng.reset();

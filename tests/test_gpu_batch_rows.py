@@ -38,3 +38,37 @@ def test_rows_match_single_steps(torch_cuda, inner, level, nsys, pre, post):
     assert np.isfinite(out[1][0]).all()
     assert np.array_equal(out[0][1], out[1][1])
     assert np.array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("inner", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("dim,level,nsys,tail", [(2, 4, 1, 300), (2, 5, 16, 1100), (2, 6, 5, 1100), (2, 6, 16, 4300), (3, 3, 3, 800),
+                                                 (2, 3, 40, 5000)])
+def test_field_tail_is_identical(torch_cuda, inner, dim, level, nsys, tail):
+    """One matrix per system: the levels of at most tail_max_n nodes in one workgroup per system against
+    the per-level launches (tail_max_n 0), bit for bit; also after new values (every level's copies)."""
+    import ctypes
+    from feat3_amd import capi
+    from feat3_amd.batch import BatchMGPCG
+    torch = torch_cuda
+    print(f"case field tail {inner} {dim}D L{level} K={nsys} tail {tail}", flush=True)
+    H = pb.hierarchy(dim, 1, level, 1)
+    rng = np.random.default_rng(level * 10 + nsys)
+    sets = [[np.ascontiguousarray(np.asarray(L.A.val)[:, None] * rng.uniform(0.5, 2.0, nsys)) for L in H.levels] for _ in range(2)]
+    B = torch.from_numpy(np.ascontiguousarray(pb.random_rhs(H.n, 1, nsys, H.levels[0].bnd, seed=5))).cuda()
+    out = []
+    for t in (tail, 0):
+        s = BatchMGPCG(H, nsys, values=sets[0], shared=False, inner=inner, options={"tail_max_n": t}).init()
+        res = []
+        for new in (False, True):
+            if new:
+                dev = [torch.from_numpy(v).cuda() for v in sets[1]]
+                for i, v in enumerate(dev):
+                    capi.call("feat3_batch_set_values", s._h, i, ctypes.c_void_p(v.data_ptr()))
+            x = torch.zeros(s.shape, dtype=torch.float64, device="cuda")
+            st, it = s.correct(x, B)
+            assert (st == 2).all()
+            res += [x.cpu().numpy(), it, np.concatenate([s.history(k) for k in range(nsys)])]
+        out.append(res)
+        s.done()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)

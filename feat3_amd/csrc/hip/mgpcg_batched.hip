@@ -317,6 +317,8 @@ namespace
       bool faces = false;
       DT k[27] = {}, d = DT(0);
       u32 fm = 0;             // 2D 9-point lattice with values per system: nodes per axis (0: not)
+      int pdim = 0;           // dimension of the lattice whose Q1 prolongation P is (0: not), and
+      u32 pm = 0;             // its nodes per axis: they stay when values change
       const u32* order() const { return ord.p ? ord.template as<u32>() : nullptr; }
     };
     Config cfg;
@@ -512,6 +514,29 @@ namespace
       return a;
     }
 
+    // P (without stored zeros) is the Q1 prolongation of a lattice of m nodes per axis from every other one,
+    // rows in ascending column order: its dimension, else 0.  m is a level's l.m or l.fm, so its Dirichlet nodes are the
+    // boundary.
+    static int q1_prolongation(u32 m, u64 nodes, u64 nc, const HostGraph& P)
+    {
+      const int dim = nodes == u64(m) * m ? 2 : nodes == u64(m) * m * m ? 3 : 0;
+      const u64 mc = (u64(m) + 1) / 2;
+      if(!dim || m < 3 || m % 2 == 0 || m > 65535 || nc != (dim == 2 ? mc * mc : mc * mc * mc)) return 0;
+      for(u64 r = 0; r < nodes; ++r)
+      {
+        const u64 x = r % m, y = r / m % m, z = r / m / m;
+        u32 e = P.rp[r];
+        const u64 ox = x & 1u, oy = y & 1u, oz = z & 1u;
+        if(P.rp[r + 1] - e != (ox + 1) * (oy + 1) * (oz + 1)) return 0;
+        const double w = (ox ? 0.5 : 1.0) * (oy ? 0.5 : 1.0) * (oz ? 0.5 : 1.0);
+        for(u64 c = 0; c <= oz; ++c)
+          for(u64 b = 0; b <= oy; ++b)
+            for(u64 a = 0; a <= ox; ++a, ++e)
+              if(u64(P.col[e]) != ((z / 2 + c) * mc + y / 2 + b) * mc + x / 2 + a || P.val[e] != w) return 0;
+      }
+      return dim;
+    }
+
     // one launch of batch::k_lat_lines; returns its block count (the number of partials)
     template<int OP, typename T>
     unsigned lines(u32 m, const T (&k)[27], T d, bool faces, const T* x, const T* rhs, T* out, const int* any_)
@@ -670,6 +695,8 @@ namespace
         {
           const HostGraph P = compact(h.P), R = compact(h.R);
           l->nc = lv[i + 1].nodes;
+          l->pm = l->m ? l->m : l->fm;
+          if(l->pm) l->pdim = q1_prolongation(l->pm, h.nodes, l->nc, P);
           F3_RC(l->prp.put(P.rp, s)); F3_RC(l->pcol.put(P.col, s)); F3_RC(l->pval.put(conv<VT>(P.val), s));
           F3_RC(l->rrp.put(R.rp, s)); F3_RC(l->rcol.put(R.col, s)); F3_RC(l->rval.put(conv<VT>(R.val), s));
         }
@@ -951,6 +978,19 @@ namespace
 
     int prolong(Level& f, const DT* xc, DT* xf, const int* a)
     {
+      if(f.pdim)
+      {
+        constexpr int SV = int(16 / sizeof(DT));
+        const u32 m = f.pm, ncol = u32(B * K);
+        auto go = [&](auto ch) {
+          constexpr int C = decltype(ch)::value;
+          const dim3 grid(unsigned((u64(m) * (ncol / u32(C)) + 255) / 256), m, f.pdim == 3 ? m : 1);
+          if(f.pdim == 3) batch::k_lat_prolong<DT, C, 3><<<grid, 256, 0, s>>>(m, ncol, xc, xf, a);
+          else batch::k_lat_prolong<DT, C, 2><<<grid, 256, 0, s>>>(m, ncol, xc, xf, a);
+        };
+        if(ncol % u32(SV) == 0) go(ic<SV>()); else go(ic<1>());
+        return rt::kOk;
+      }
       return with_layout<DT>(GV, S, [&](auto gv, auto sv) {
         constexpr int Gc = decltype(gv)::value, Sc = decltype(sv)::value;
         const mg::RowGrid g = vcycle_grid(f.nodes, Gc);

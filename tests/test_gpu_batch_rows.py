@@ -72,3 +72,28 @@ def test_field_tail_is_identical(torch_cuda, inner, dim, level, nsys, tail):
         s.done()
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("case", ["q1", "weight"])
+def test_lattice_prolongation_is_identical(torch_cuda, case):
+    """The prolongation by its closed form against the stored matrix, bit for bit; a matrix with one other
+    weight keeps the stored one (7 systems: one value per thread, 8: four)."""
+    from feat3_amd.batch import BatchMGPCG
+    torch = torch_cuda
+    for nsys in (7, 8):
+        print(f"case lattice prolongation {case} K={nsys}", flush=True)
+        H = pb.hierarchy(2, 1, 7, 1)
+        if case == "weight":
+            H.levels[0].P.val = np.array(H.levels[0].P.val)
+            H.levels[0].P.val[int(H.levels[0].P.row_ptr[64 * 129 + 65])] = 0.375
+        vals = [np.ascontiguousarray(np.repeat(np.asarray(L.A.val)[:, None], nsys, axis=1)) for L in H.levels]
+        B = torch.from_numpy(np.ascontiguousarray(pb.random_rhs(H.n, 1, nsys, H.levels[0].bnd, seed=5))).cuda()
+        out = []
+        for lattice in (1, 0):
+            s = BatchMGPCG(H, nsys, values=vals, shared=False, inner="f32", tol_rel=0.0, min_iter=2, max_iter=2,
+                           options={"lattice": lattice}).init()
+            x = torch.zeros(s.shape, dtype=torch.float64, device="cuda")
+            s.correct(x, B)
+            out.append(x.cpu().numpy())
+            s.done()
+        assert np.isfinite(out[1]).all() and np.array_equal(out[0], out[1])

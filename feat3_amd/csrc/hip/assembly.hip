@@ -6,7 +6,7 @@
 // Structured Q1/Q2 Lagrange space on the refined unit square/cube, lexicographic node and cell
 // numbering.  Entry (i, j) of A(k) is h^(d-2) * sum over the cells c holding both nodes of
 // k_c * K_ref[loc_c(i)][loc_c(j)].  The graph (row_ptr, col_ind) is the host setup's; one thread
-// per (row, field) walks its row.  The cells are summed in the host's order (z, y, x ascending)
+// per (row, field) walks its row (Q1 in the plane: by tiles, k_assemble_q1_2d).  The cells are summed in the host's order (z, y, x ascending)
 // with separate multiply and add (no contraction), so the values are bit-identical to the host
 // assembly.  Fields are [field][cell]; values are written [entry][field], the layout of the
 // batched solver's per-system values.

@@ -13,8 +13,8 @@
 //
 // What bounds them: the vectors, with the tiles' halos read again.  Measured on 65^3 nodes of 3 x 32
 // values, from the row kernels: FP32 sweep 169 -> 83 us (3.8 TB/s of its three vectors; a large copy
-// reaches 5.1), defect 158 -> 82 us, FP64 product with its dot 387 -> 142 us, initial defect 450 ->
-// 190 us.  Without the loads ahead of the sums the sweep takes 101 us.
+// reaches 5.1), defect 158 -> 82 us, FP64 product with its dot 387 -> 142 us.
+// Without the loads ahead of the sums the sweep takes 101 us.
 #pragma once
 
 #include "batch_kernels.hpp"

@@ -1644,7 +1644,10 @@ namespace
           }
           l->P.rows_per_block = cfg.transfer_rows_per_block;
           l->R.rows_per_block = cfg.transfer_rows_per_block;
-          if(cfg.tensor_transfer) F3_RC((build_tensor_pair<DT, VT>(l->P, l->R, s)));
+          F3_RC((build_tensor_pair<DT, VT>(l->P, l->R, s)));
+          // without the option the row kernels keep the stored matrices; whether a level is a lattice
+          // (P.tdeg) does not depend on it
+          if(!cfg.tensor_transfer) l->P.tensor = l->R.tensor = false;
         }
         const std::vector<u32> m = make_mask(l->n, h.fidx);
         F3_RC(l->mask.alloc(sizeof(u32) * m.size()));
@@ -2213,7 +2216,7 @@ namespace
     int setup_lattice(Level<DT, VT>& l)
     {
       l.lat = -1;
-      if(!l.P.tensor || l.P.tdeg == 0 || l.n >= (u64(1) << 31)) return rt::kOk;
+      if(l.P.tdeg == 0 || l.n >= (u64(1) << 31)) return rt::kOk;
       const int dim = l.P.tmo[2] > 1 ? 3 : 2, rad = l.P.tdeg;
       const u32 m = l.P.tmo[0];
       if((dim == 3 && rad != 1) || m < 9) return rt::kOk;

@@ -123,3 +123,24 @@ def test_columns_are_bitwise_the_steps(torch, inner):
     assert a[3:] == e[3:] and a[3] == a[5] == 2
     assert np.linalg.norm(a[1] - e[1]) <= 1e-12 * np.linalg.norm(e[1])
     assert np.linalg.norm(a[2] - e[2]) <= 1e-12 * np.linalg.norm(e[2])
+
+
+@pytest.mark.parametrize("dim,deg,lvl", [(2, 1, 6), (2, 2, 5), (3, 1, 5)])
+@pytest.mark.parametrize("inner", ["f64", "f32"])
+def test_row_kernels_with_and_without_tensor_transfers(torch_cuda, dim, deg, lvl, inner):
+    """Without the lattice kernels (lattice = 0) the tensor transfers and the stored ones give the same
+    solve bit for bit; with them the option changes nothing either."""
+    from feat3_amd.solver import MGPCG
+    torch = torch_cuda
+    print(f"case transfers {dim}D Q{deg} L{lvl} {inner}", flush=True)
+    H = pb.hierarchy(dim, deg, lvl, 1)
+    b = torch.from_numpy(pb.filtered_rhs(H, 0)).cuda()
+    for lattice in (0, 1):
+        out = []
+        for tensor in (1, 0):
+            s = MGPCG(H, inner=inner, fmt="banded", options={"lattice": lattice, "tensor_transfer": tensor}).init()
+            x = torch.zeros_like(b)
+            st, it = s.correct(x, b)
+            out.append((st, it, x.cpu().numpy()))
+            s.done()
+        assert out[0][:2] == out[1][:2] and np.array_equal(out[0][2], out[1][2])

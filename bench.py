@@ -25,13 +25,13 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, public spec
 
 # HBM bytes per launch of the finest-level sweep, measured with rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE (separate runs of this script) and scaled by the same counters on a plain 512 MiB
-# device copy (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0); profiles/k_sweep_3d_q1_l7_f32.md,
-# profiles/solve_kernels_2d_q2_l9.md and profiles/batch_k_sweep_vector32_f32.md hold the commands
-# and raw values (the two scalar workloads' bands are value-coded).  Keyed by (workload, level, inner, format); absent -> null.
+# device copy (FETCH_SIZE x 2.0, WRITE_SIZE x 1.0); profiles/lattice_kernels.md and
+# profiles/solve_kernels_2d_q2_l9.md hold the commands and raw values (3D: the step without a matrix
+# stream; 2D Q2: the value-coded band).  Keyed by (workload, level, inner, format); absent -> null.
 MEASURED_SWEEP_TRAFFIC = {
-    ("poisson3d", 7, "f32", "banded"): (2 * 25674.4 + 8385.5) * 1024,
+    ("poisson3d", 7, "f32", "banded"): (2 * 8920.1 + 8386.0) * 1024,
     ("poisson2d", 9, "f32", "banded"): (2 * 14486.4 + 4104.0) * 1024,
-    ("vector32", 6, "f32", "banded"): (2 * 288738.1 + 102984.4) * 1024,
+    ("vector32", 6, "f32", "banded"): (2 * 124146.9 + 102984.4) * 1024,
 }
 
 
@@ -178,7 +178,7 @@ def bench_vector32(args):
     roof = {"bound": "hbm", "achieved": head["sweep_GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": head["sweep_GBs"] / HBM_PEAK_GBS,
             "traffic": MEASURED_SWEEP_TRAFFIC.get(("vector32", lvl, args.inner, "banded")),
-            "kernel": "batch k_sweep<B=3>, finest level (fused damped-Jacobi step, 32 systems)",
+            "kernel": "batch k_lat_lines, finest level (fused damped-Jacobi step, 32 systems)",
             "bytes_per_launch": head["sweep_bytes"], "avg_launch_us": head["sweep_us"]}
     cfg = {"workload": f"3D vector Laplacian Q1 level {lvl}, 3x3 BCSR ({nodes} block rows, {nnzb} blocks), "
                        f"32 right-hand sides in one batched PCG(FP64) + MG V(4,4), {args.inner} V-cycle, rel. tol 1e-8",
@@ -605,7 +605,7 @@ def main():
         log(f"cpu baseline: {cpu}")
 
     achieved = head["sweep_GBs"]
-    # measured with the value-coded band (the default)
+    # measured with the default formats
     traffic = MEASURED_SWEEP_TRAFFIC.get((args.workload, args.level, args.inner, args.fmt)) if args.band_dict else None
     out = {
         "metric": "time to rel. residual 1e-8 & DOF·iter/s, FP32-inner vs FP64; SpMV GB/s",
@@ -629,7 +629,7 @@ def main():
         "iterations": float(np.mean(iters)),
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": "k_sweep, finest level (fused damped-Jacobi step)",
+                     "kernel": ("k_columns" if dim == 3 and args.level >= 7 else "k_sweep") + ", finest level (fused damped-Jacobi step)",
                      "bytes_per_launch": head["sweep_bytes"], "avg_launch_us": head["sweep_us"]},
         "headline": head,
         "variants": {k: v[0] for k, v in variants.items()},

@@ -871,7 +871,9 @@ namespace
         if(!invert_dense(a, mc)) return rt::kErrNumeric;
         std::copy(a.begin(), a.end(), inv_all.begin() + k * mc * mc);
       }
-      F3_RC(ainv.put(inv_all, s));
+      // new values keep the buffer (its size depends on the graph alone): captured iterations hold its address
+      if(!ainv.p) F3_RC(ainv.alloc(sizeof(double) * inv_all.size()));
+      F3_CHECK(hipMemcpyAsync(ainv.p, inv_all.data(), sizeof(double) * inv_all.size(), hipMemcpyHostToDevice, s));
       F3_CHECK(hipStreamSynchronize(s));   // inv_all goes out of scope
       return rt::kOk;
     }

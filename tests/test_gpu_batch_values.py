@@ -1,0 +1,50 @@
+"""New values of every level (feat3_batch_set_values) between two solves into the SAME solution vector.
+
+The second solve replays the iterations captured by the first one, whose launches hold device addresses;
+what they read (the coarse inverses among it) is refreshed in place.  The solution has to be, bit for
+bit, that of a solver built for the new values.  Allocations made in between take whatever memory the
+refresh would have given back."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from feat3_amd import problems as pb
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("inner", ["f64", "f32"])
+@pytest.mark.parametrize("nsys,shared,tail", [(3, False, 1100), (16, False, 0), (4, True, 1000), (4, True, 0)])
+def test_replayed_iterations_take_the_new_values(torch_cuda, inner, nsys, shared, tail):
+    from feat3_amd import capi
+    from feat3_amd.batch import BatchMGPCG
+    torch = torch_cuda
+    print(f"case new values {inner} K={nsys} shared={shared} tail {tail}", flush=True)
+    H = pb.hierarchy(2, 1, 5, 1)
+    rng = np.random.default_rng(nsys)
+    f = [rng.uniform(0.5, 2.0, 1 if shared else nsys) for _ in range(3)]
+    sets = [[np.ascontiguousarray(np.asarray(L.A.val)[:, None] * w) for L in H.levels] for w in f]
+    B = torch.from_numpy(np.ascontiguousarray(pb.random_rhs(H.n, 1, nsys, H.levels[0].bnd, seed=5))).cuda()
+
+    def make(vals):
+        return BatchMGPCG(H, nsys, values=vals, shared=shared, inner=inner, options={"tail_max_n": tail}).init()
+
+    s = make(sets[0])
+    x = torch.zeros(s.shape, dtype=torch.float64, device="cuda")
+    s.correct(x, B)
+    held = []
+    for vals in sets[1:] + sets[:1]:
+        for i, v in enumerate(vals):
+            dv = torch.from_numpy(v).cuda()
+            capi.call("feat3_batch_set_values", s._h, i, ctypes.c_void_p(dv.data_ptr()))
+            held += [dv, torch.full((1 << 16,), float("nan"), dtype=torch.float64, device="cuda")]
+        x.zero_()
+        st, it = s.correct(x, B)
+        e = make(vals)
+        y = torch.zeros_like(x)
+        se, ie = e.correct(y, B)
+        e.done()
+        assert (st == 2).all() and (se == 2).all() and (it == ie).all()
+        assert torch.equal(x, y)
+    s.done()

@@ -686,7 +686,8 @@ namespace lat
 
   // ---- setup ---------------------------------------------------------------------------------
 
-  // Flags raised: 1 an entry outside the box of RAD nodes around its row's node; 2 an inner row that
+  // Flags raised: 1 an entry outside the box of RAD nodes around its row's node, or a second one of the
+  // same column (the general formats add both; the lattice kernels have one value per neighbour); 2 an inner row that
   // differs (any value or its dinv, as bit patterns) from its class's row in rep, or Dirichlet
   // nodes other than the lattice's boundary.  Classes: the coordinates' parities (per = 2) or one;
   // rep[class][tap], repd[class] in the arithmetic type (dinv null: not compared).
@@ -712,6 +713,7 @@ namespace lat
         if(dx < -rad || dx > rad || dy < -rad || dy > rad || dz < -rad || dz > rad || (dim == 2 && dz != 0)) { f |= 3; continue; }
         const int t = ((dim == 3 ? dz + rad : 0) * nl + dy + rad) * nl + dx + rad;
         const DT_ v = dev::ld<DT_>(val, k);
+        if((hit >> t) & 1u) f |= 3;
         hit |= 1u << t;
         if(!dir && !(v == rep[cls * ntap + t])) f |= 2;
       }

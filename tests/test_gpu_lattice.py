@@ -83,6 +83,39 @@ def test_changed_rows_are_not_taken_as_uniform(torch, dim, deg, lvl):
     assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("inner", ["f64", "f32"])
+@pytest.mark.parametrize("dim,deg,lvl", [(2, 1, 6), (2, 2, 5), (3, 1, 4)])
+@pytest.mark.parametrize("where", ["all", "one"])
+def test_two_entries_of_one_column_are_added(torch, dim, deg, lvl, inner, where):
+    """An entry stored as two halves (exact) of one column, in every inner row or in one: the general formats
+    add them, so such a level is no lattice.  The cycles agree with the whole entry's to the rounding of a
+    row sum (25 or 27 terms); with bands on the other levels they are those of lattice = 0 bit for bit."""
+    H = pb.hierarchy(dim, deg, lvl, 1)
+    A = H.levels[0].A
+    rows = np.repeat(np.arange(A.rows), np.diff(A.row_ptr.astype(np.int64)))
+    inner_row = np.ones(A.rows, bool)
+    inner_row[H.levels[0].bnd] = False
+    pick = np.flatnonzero((A.col_ind == rows + 1) & inner_row[rows] & inner_row[np.minimum(rows + 1, A.rows - 1)])
+    if where == "one":
+        pick = pick[pick.size // 2:][:1]
+    d = defect(H)
+    whole, _ = cycles(torch, H, d, inner, 0, fmt="csr")
+    times = np.ones(A.nnz, np.int64)
+    times[pick] = 2
+    ends = np.cumsum(times)
+    val = np.repeat(A.val, times)
+    val[ends[pick] - 1] *= 0.5
+    val[ends[pick] - 2] *= 0.5
+    rp = np.concatenate([[0], ends])[A.row_ptr.astype(np.int64)].astype(np.uint32)
+    H.levels[0].A = pb.Csr(A.rows, A.cols, rp, np.repeat(A.col_ind, times), val)
+    eps = np.finfo(np.float64 if inner == "f64" else np.float32).eps
+    for fmt in ("csr", "banded"):
+        a, _ = cycles(torch, H, d, inner, 1, fmt=fmt)
+        b, _ = cycles(torch, H, d, inner, 0, fmt=fmt)
+        assert fmt == "csr" or np.array_equal(a, b), np.abs(a - b).max()
+        assert np.linalg.norm(a - whole) <= 27 * eps * np.linalg.norm(whole)
+
+
 @pytest.mark.parametrize("fmt", ["csr", "sell"])
 @pytest.mark.parametrize("inner", ["f64", "f32"])
 def test_other_formats_agree(torch, fmt, inner):

@@ -82,12 +82,18 @@ namespace batch
       for(int e = 0; e < 3; ++e) win[s][0][e] = win[s][1][e] = DT_(0);
 
     const int t0 = y0 - NS_ > 0 ? y0 - NS_ : 0, t1 = y1 + NS_;
-    DT_ next = on ? a.x[u64(t0) * rowv + at] : DT_(0);
+    // row t of x; on the boundary plus dinv, which is 0 there or, in a row that is not finite, NaN
+    auto load_x = [&](int t) {
+      DT_ v = a.x[u64(t) * rowv + at];
+      if(!mid || t == 0 || t + 1 == m) v += a.dinv[u64(t) * rowv + at];
+      return v;
+    };
+    DT_ next = on ? load_x(t0) : DT_(0);
     // turn t: row t of x arrives; step s completes row t - 1 - s from its input's rows t - 2 - s .. t - s
     auto turn = [&](int t, auto phase) {
       constexpr int P = decltype(phase)::value;
       DT_ cur = next;
-      if(on && t + 1 < m) next = a.x[u64(t + 1) * rowv + at];
+      if(on && t + 1 < m) next = load_x(t + 1);
       if(mid && t >= 1 && t + 1 < m)
       {
         const VT_* v = a.val + field_entry(u64(m), u64(x), u64(t)) * K + k;

@@ -688,8 +688,9 @@ namespace lat
 
   // Flags raised: 1 an entry outside the box of RAD nodes around its row's node, or a second one of the
   // same column (the general formats add both; the lattice kernels have one value per neighbour); 2 an inner row that
-  // differs (any value or its dinv, as bit patterns) from its class's row in rep, or Dirichlet
-  // nodes other than the lattice's boundary.  Classes: the coordinates' parities (per = 2) or one;
+  // differs (any value or its dinv, as bit patterns) from its class's row in rep, a Dirichlet row with a
+  // value that is not finite (the row kernels carry it into the cycle, and the solve reports it: such a
+  // level keeps them, or its own table of values), or Dirichlet nodes other than the lattice's boundary.  Classes: the coordinates' parities (per = 2) or one;
   // rep[class][tap], repd[class] in the arithmetic type (dinv null: not compared).
   template<typename DT_, typename VT_>
   __global__ void k_lattice_check(u64 n, u32 m, u64 div_m, int dim, int rad, int per, const u32* __restrict__ rp, const u32* __restrict__ col,
@@ -715,7 +716,7 @@ namespace lat
         const DT_ v = dev::ld<DT_>(val, k);
         if((hit >> t) & 1u) f |= 3;
         hit |= 1u << t;
-        if(!dir && !(v == rep[cls * ntap + t])) f |= 2;
+        if(dir ? !isfinite(v) : !(v == rep[cls * ntap + t])) f |= 2;
       }
       if(!dir)
         for(int t = 0; t < ntap; ++t)

@@ -235,7 +235,20 @@ namespace
           else d = DT(VT(float(v)));
           break;
         }
-      dinv[t] = dev::masked(mask, node) ? DT(0) : omega_r * (omega_j / d);
+      dinv[t] = omega_r * (omega_j / d);
+      if(dev::masked(mask, node))
+      {
+        // 0 times the row: NaN if a value is not finite, also where a kernel does not read the row
+        d = DT(0);
+        for(u32 e = rp[node]; e < rp[node + 1]; ++e)
+          for(int ww = 0; ww < B; ++ww)
+          {
+            const double v = val[(u64(e) * u64(B * B) + hh * u64(B) + u64(ww)) * kv + k];
+            if constexpr(sizeof(VT) == 8) d += DT(0) * DT(v);
+            else d += DT(0) * DT(VT(float(v)));
+          }
+        dinv[t] = d;
+      }
     }
   }
 
@@ -443,7 +456,13 @@ namespace
             const bool edge = x == 0 || y == 0 || z == 0 || x + 1 == m || y + 1 == m || z + 1 == m;
             const bool dir = (mask[r >> 5] >> (r & 31u)) & 1u;
             if(dir != edge) return 0;
-            if(edge) continue;
+            if(edge)
+            {
+              // (the row kernels carry a value that is not finite into the cycle, and the solve reports it)
+              for(u64 e = rp[r] * per; e < rp[r + 1] * per; ++e)
+                if(!std::isfinite(double(T(to_storage<V>(val[e]))))) return 0;
+              continue;
+            }
             const u32 e0 = rp[r], count = rp[r + 1] - e0;
             if(taps == 0)
             {
@@ -722,6 +741,10 @@ namespace
                   const DT d = DT(to_storage<VT>(h.A.val[(u64(e) * vpe() + u64(hh) * B + u64(hh)) * kv + k]));
                   dinv[(node * B + u64(hh)) * kv + k] = dir ? DT(0) : DT(cfg.omega_r) * (DT(cfg.omega_j) / d);
                 }
+          // 0 times a Dirichlet row (k_batch_dinv)
+          for(u32 e = h.A.rp[node]; dir && e < h.A.rp[node + 1]; ++e)
+            for(u64 i = 0; i < vpe() * kv; ++i)
+              dinv[(node * B + i / kv / B % B) * kv + i % kv] += DT(0) * DT(to_storage<VT>(h.A.val[u64(e) * vpe() * kv + i]));
         }
         F3_RC(l->dinv.put(dinv, s));
         if(l->m)

@@ -116,6 +116,26 @@ def test_two_entries_of_one_column_are_added(torch, dim, deg, lvl, inner, where)
         assert np.linalg.norm(a - whole) <= 27 * eps * np.linalg.norm(whole)
 
 
+@pytest.mark.parametrize("inner", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("dim,deg,lvl,coef", [(2, 1, 7, False), (2, 1, 7, True), (2, 2, 6, False), (3, 1, 5, False)])
+def test_dirichlet_rows_that_are_not_finite(torch, dim, deg, lvl, coef, inner):
+    """A NaN or an infinity in the matrix row of a Dirichlet node of the finest or the next level: the cycle
+    carries it and the solve ends with status aborted, as with the row kernels (lattice = 0)."""
+    from feat3_amd.solver import MGPCG
+    k = np.exp(np.random.default_rng(7).uniform(-1.0, 1.0, 1 << (2 * lvl))) if coef else None
+    for level, bad in ((0, np.nan), (0, np.inf), (1, np.nan)):
+        H = pb.hierarchy(dim, deg, lvl, 1, kcell=k)
+        L = H.levels[level]
+        L.A.val[int(L.A.row_ptr[int(L.bnd[L.bnd.size // 3])])] = bad
+        b = torch.from_numpy(pb.filtered_rhs(H, 0)).cuda()
+        out = []
+        for lattice in (1, 0):
+            s = MGPCG(H, inner=inner, options={"lattice": lattice}).init()
+            out.append(s.correct(torch.zeros_like(b), b))
+            s.done()
+        assert out[0] == out[1] and out[0][0] == 3, (level, bad, out)
+
+
 @pytest.mark.parametrize("fmt", ["csr", "sell"])
 @pytest.mark.parametrize("inner", ["f64", "f32"])
 def test_other_formats_agree(torch, fmt, inner):

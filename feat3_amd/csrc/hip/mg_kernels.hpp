@@ -1075,12 +1075,10 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     return s;
   }
 
-  // ops[0, nops): the segment's steps; out_buf: the buffer of tail[0]'s iterate at the end.
-  // UNIT_: block j takes the j-th unit vector as the right-hand side and writes column j of the
-  // segment's matrix mat (row-major, n x n) instead of an iterate (see k_tail_apply).
-  template<typename DT_, typename VT_, bool UNIT_ = false>
+  // ops[0, nops): the segment's steps; out_buf: the buffer of tail[0]'s iterate at the end
+  template<typename DT_, typename VT_>
   __global__ __launch_bounds__(kTailThreads) void k_tail(TailDesc<DT_, VT_> d, const u32* __restrict__ ops, u32 nops,
-                                                         u32 out_buf, const int* status, DT_* __restrict__ mat = nullptr)
+                                                         u32 out_buf, const int* status)
   {
     if(stopped(status)) return;
     extern __shared__ double tail_arena_[];
@@ -1098,7 +1096,7 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
         if(i == 0)
         {
           // the first smoothing step from x = 0 (as the restriction above writes it)
-          const DT_ b = UNIT_ ? DT_(r == blockIdx.x ? 1 : 0) : d.rhs_in[r];
+          const DT_ b = d.rhs_in[r];
           v[2 * l.n + r] = b;
           v[r] = di * b;
         }
@@ -1167,47 +1165,217 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
     }
     const TailLevel<DT_, VT_>& t = d.lv[0];
     const DT_* xf = arena + t.off + out_buf * t.n;
-    for(u32 r = tid; r < t.n; r += kTailThreads)
-    {
-      if constexpr(UNIT_) mat[u64(r) * t.n + blockIdx.x] = xf[r];
-      else d.x_out[r] = xf[r];
-    }
+    for(u32 r = tid; r < t.n; r += kTailThreads) d.x_out[r] = xf[r];
   }
 
   // A segment of the cycle on the coarse tail is a linear map from tail[0]'s right-hand side to its
   // iterate, fixed once the levels and the smoothers are: init forms its matrix column by column
-  // (k_tail with UNIT_, the arithmetic of the cycle) and the cycle applies it with one product, one
-  // wave per row.  k_tail itself is a chain of 20 to 40 dependent steps of 0.7 to 1.6 us on one CU,
-  // whatever the levels' sizes; the product reads at most 9.5 MB (1089 rows in FP64), which the L2s
-  // hold, over the whole chip.
-  constexpr u64 kTailMatRows = 2048;   // levels of at most this many rows (a 33 MB matrix in FP64)
+  // (k_tail_columns) and the cycle applies it with one product, one wave per row (k_tail_apply).
+  // k_tail itself is a chain of 20 to 40 dependent steps of 0.7 to 1.6 us on one CU, whatever the
+  // levels' sizes; the product reads one matrix (1089 rows, the most by default: 9.5 MB, 19 MB in
+  // FP64), which the L2s hold, over the whole chip.
+  //
+  // Precision: an entry's error counts against |M| |b| and not against |M b|, so it does not shrink with
+  // the result as the steps' errors do (2D Q1, 33 x 33 nodes, checkerboard b: |M| |b| is 100 times M b).
+  // So M is formed and kept with twice the digits of the cycle's arithmetic -- FP64 for FP32 cycles, an
+  // unevaluated sum of two FP64 values (Dd) for FP64 ones -- and the product is summed alike: its
+  // result is M b rounded once.  Relative error there, steps -> matrix: FP32 5e-8 -> 2.4e-8, FP64
+  // 7e-17 -> 6e-17 (with entries of the cycle's own precision 1.3e-6 and 7e-15).
+  constexpr u64 kTailMatRows = 2048;   // levels of at most this many rows (a 67 MB matrix in FP64)
+
+  struct Dd
+  {
+    double h, l;
+  };
+  __device__ __forceinline__ Dd two_sum(double a, double b)   // a + b exactly (Knuth)
+  {
+#pragma clang fp contract(off)
+    const double s = a + b, t = s - a;
+    return {s, (a - (s - t)) + (b - t)};
+  }
+  __device__ __forceinline__ Dd two_prod(double a, double b)
+  {
+    const double p = a * b;
+    return {p, __builtin_fma(a, b, -p)};
+  }
+  __device__ __forceinline__ Dd dd_fast(double h, double l)   // |h| >= |l| or h = 0
+  {
+#pragma clang fp contract(off)
+    const double s = h + l;
+    return {s, l - (s - h)};
+  }
+  // the arithmetic of k_tail_columns: value conversion, a + b, a - b, s + a x
+  template<typename C_> __device__ __forceinline__ C_ tail_cast(double v);
+  template<> __device__ __forceinline__ double tail_cast<double>(double v) { return v; }
+  template<> __device__ __forceinline__ Dd tail_cast<Dd>(double v) { return {v, 0.0}; }
+  __device__ __forceinline__ double tail_sub(double a, double b) { return a - b; }
+  __device__ __forceinline__ double tail_add(double a, double b) { return a + b; }
+  __device__ __forceinline__ double tail_mac(double a, double x, double s) { return __builtin_fma(a, x, s); }
+  __device__ __forceinline__ Dd tail_add(Dd a, Dd b)
+  {
+    const Dd s = two_sum(a.h, b.h);
+    return dd_fast(s.h, s.l + (a.l + b.l));
+  }
+  __device__ __forceinline__ Dd tail_sub(Dd a, Dd b) { return tail_add(a, Dd{-b.h, -b.l}); }
+  __device__ __forceinline__ Dd tail_mac(double a, Dd x, Dd s)
+  {
+    const Dd p = two_prod(a, x.h);
+    return tail_add(s, dd_fast(p.h, __builtin_fma(a, x.l, p.l)));
+  }
+
+  // Columns of a segment's matrix (row-major, hi plus lo): block j runs the segment's steps on the j-th
+  // unit vector with the arithmetic of C_ (double, Dd) and the operands of k_tail.  LDS: x0, x1, rhs and
+  // def of the tail's levels in C_.
+  template<typename C_, typename DT_, typename VT_>
+  __global__ __launch_bounds__(kTailThreads) void k_tail_columns(TailDesc<DT_, VT_> d, const u32* __restrict__ ops, u32 nops,
+                                                                 u32 out_buf, double* __restrict__ hi, double* __restrict__ lo)
+  {
+    extern __shared__ double tail_arena_[];
+    C_* arena = reinterpret_cast<C_*>(tail_arena_);
+    const u32 tid = threadIdx.x;
+    auto vec = [&](u32 li) { return arena + d.lv[li].off / 5u * 4u; };
+    auto row = [](const TailEll<VT_>& M, u32 r, const C_* xs) {
+      C_ s = tail_cast<C_>(0.0);
+#pragma unroll 9
+      for(u32 k = 0; k < M.w; ++k)
+      {
+        const u64 at = u64(k) * M.n + r;
+        s = tail_mac(dev::ld<double>(M.val, at), xs[M.col[at]], s);
+      }
+      return s;
+    };
+    const C_ zero = tail_cast<C_>(0.0);
+    for(u32 r = tid; r < d.lv[0].n; r += kTailThreads)
+    {
+      C_* v = vec(0);
+      const C_ b = tail_cast<C_>(r == blockIdx.x ? 1.0 : 0.0);
+      v[2 * d.lv[0].n + r] = b;
+      v[r] = tail_mac(double(d.lv[0].dinv[r]), b, zero);
+    }
+    __syncthreads();
+    for(u32 o = 0; o < nops; ++o)
+    {
+      const u32 op = ops[o];
+      const u32 kind = op & 15u, li = (op >> 4) & 15u, a = (op >> 8) & 1u, b = (op >> 9) & 1u;
+      const TailLevel<DT_, VT_>& f = d.lv[li];
+      C_* fv = vec(li);
+      const u32 n = f.n;
+      C_* xi = fv + a * n;
+      if(kind == kTailSweep)
+      {
+        C_* xo = fv + (a ^ 1u) * n;
+        for(u32 r = tid; r < n; r += kTailThreads) xo[r] = tail_mac(double(f.dinv[r]), tail_sub(fv[2 * n + r], row(f.A, r, xi)), xi[r]);
+      }
+      else if(kind == kTailDefect)
+      {
+        for(u32 r = tid; r < n; r += kTailThreads)
+        {
+          const C_ s = row(f.A, r, xi);
+          fv[3 * n + r] = dev::masked(f.mask, r) ? zero : tail_sub(fv[2 * n + r], s);
+        }
+      }
+      else if(kind == kTailRest)
+      {
+        const TailLevel<DT_, VT_>& c = d.lv[li + 1];
+        C_* cv = vec(li + 1);
+        const bool first_step = ((op >> 10) & 1u) != 0u;
+        for(u32 r = tid; r < c.n; r += kTailThreads)
+        {
+          const C_ s = row(f.R, r, fv + 3 * n);
+          const C_ v = dev::masked(c.mask, r) ? zero : s;
+          cv[2 * c.n + r] = v;
+          if(first_step) cv[r] = tail_mac(double(c.dinv[r]), v, zero);
+        }
+      }
+      else if(kind == kTailCoarse)
+      {
+        for(u32 i = tid; i < d.ncoarse; i += kTailThreads)
+        {
+          C_ s = zero;
+          for(u32 j = 0; j < d.ncoarse; ++j) s = tail_mac(d.ainv[u64(i) * d.ncoarse + j], fv[2 * n + j], s);
+          fv[i] = dev::masked(f.mask, i) ? zero : s;
+        }
+      }
+      else
+      {
+        const C_* xc = vec(li + 1) + b * d.lv[li + 1].n;
+        for(u32 r = tid; r < n; r += kTailThreads)
+        {
+          const C_ s = row(f.P, r, xc);
+          if(!dev::masked(f.mask, r)) xi[r] = tail_add(xi[r], s);
+        }
+      }
+      __syncthreads();
+    }
+    const u32 n = d.lv[0].n;
+    const C_* xf = vec(0) + out_buf * n;
+    for(u32 r = tid; r < n; r += kTailThreads)
+    {
+      if constexpr(std::is_same<C_, Dd>::value)
+      {
+        hi[u64(r) * n + blockIdx.x] = xf[r].h;
+        lo[u64(r) * n + blockIdx.x] = xf[r].l;
+      }
+      else
+        hi[u64(r) * n + blockIdx.x] = xf[r];
+    }
+  }
+
+  // x = M rhs (lo: FP64 cycles only)
   template<typename DT_>
-  __global__ __launch_bounds__(256) void k_tail_apply(u32 n, const DT_* __restrict__ mat, const DT_* __restrict__ rhs,
-                                                      DT_* __restrict__ x, const int* status)
+  __global__ __launch_bounds__(256) void k_tail_apply(u32 n, const double* __restrict__ hi, const double* __restrict__ lo,
+                                                      const DT_* __restrict__ rhs, DT_* __restrict__ x, const int* status)
   {
     if(stopped(status)) return;
+    constexpr bool DD = sizeof(DT_) == 8;
     const u32 lane = threadIdx.x % u32(dev::kWave);
     const u32 r = blockIdx.x * 4u + threadIdx.x / u32(dev::kWave);
     if(r >= n) return;
-    const DT_* a = mat + u64(r) * n;
+    const double* a = hi + u64(r) * n;
+    const double* al = lo + u64(r) * n;
     constexpr u32 U = 6;   // loads of a lane in flight (of each operand)
-    double s = 0.0;   // (costs nothing here, and the FP32 product then adds only its entries' rounding)
+    double s = 0.0, sl = 0.0;
     for(u32 j0 = lane; j0 < n; j0 += U * u32(dev::kWave))
     {
-      DT_ av[U], bv[U];
+      double av[U], lv[U];
+      DT_ bv[U];
 #pragma unroll
       for(u32 k = 0; k < U; ++k)
       {
         const u32 j = j0 + k * u32(dev::kWave), i = j < n ? j : n - 1u;   // (no branches between the loads)
         av[k] = a[i];
+        if constexpr(DD) lv[k] = al[i];
         bv[k] = rhs[i];
       }
 #pragma unroll
       for(u32 k = 0; k < U; ++k) bv[k] = j0 + k * u32(dev::kWave) < n ? bv[k] : DT_(0);
 #pragma unroll
-      for(u32 k = 0; k < U; ++k) s = fmadd(double(av[k]), double(bv[k]), s);
+      for(u32 k = 0; k < U; ++k)
+      {
+        if constexpr(DD)
+        {
+          const Dd p = two_prod(av[k], bv[k]);
+          const Dd t = two_sum(s, p.h);
+          s = t.h;
+          sl += t.l + __builtin_fma(lv[k], bv[k], p.l);
+        }
+        else
+          s = fmadd(av[k], double(bv[k]), s);
+      }
     }
-    s = dev::wave_sum(s);
+    if constexpr(DD)
+    {
+#pragma unroll
+      for(int off = dev::kWave / 2; off > 0; off >>= 1)
+      {
+        const Dd t = two_sum(s, __shfl_xor(s, off, dev::kWave));
+        sl = sl + __shfl_xor(sl, off, dev::kWave) + t.l;
+        s = t.h;
+      }
+      s += sl;
+    }
+    else
+      s = dev::wave_sum(s);
     if(lane == 0u) x[r] = DT_(s);
   }
 

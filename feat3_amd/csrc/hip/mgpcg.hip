@@ -1835,7 +1835,7 @@ namespace
     // tail_lds bytes of LDS hold their vectors
     std::size_t tail0 = 0;
     mg::TailDesc<DT, VT> tail{};
-    u64 tail_lds = 0;
+    u64 tail_lds = 0, tail_cap = 0;   // LDS bytes of k_tail, the device's limit per workgroup
     std::vector<std::unique_ptr<DevMem>> tail_mem;
 
     // ELL copy for the tail kernel: 16-bit columns, the entries band_keeps(v, row diagonal, thin)
@@ -1890,6 +1890,7 @@ namespace
       tail_mem.clear();
       int dev = 0, cap = 65536;
       if(hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cap, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+      tail_cap = u64(cap);
       auto arena = [&](std::size_t t0) {
         u64 b = 0;
         for(std::size_t i = t0; i < nl; ++i) b += 5 * L[i]->n * sizeof(DT);
@@ -1946,24 +1947,26 @@ namespace
     std::vector<std::unique_ptr<DevMem>> tail_mats;
 
     // The matrices of the tail's segments (mg::k_tail_apply), one for all segments with the same
-    // steps (a V-cycle has one segment, a W-cycle many of a few kinds).  Measured per segment (3D Q1
-    // L7 / 2D Q2 L9 in FP32, 2D Q1 L6 / 3D Q1 L7 in FP64): 4.7 / 4.1 / 4.4 / 4.8 us, with k_tail 34 /
-    // 55 / 67 / 99 us; forming a matrix takes 0.1 ms (729 rows, FP32) to 0.4 ms.  Tails of more than
-    // kTailMatRows rows (option tail_max_n; 4225 rows in FP32 would read 71 MB per segment, as long as
-    // k_tail takes) and further kinds beyond eight run k_tail.
+    // steps (a V-cycle has one segment, a W-cycle many of a few kinds).  Kernel times in a trace,
+    // k_tail -> the product: 3D Q1 (729 rows) FP32 34 -> 3.5, FP64 99 -> 4.1 us; 2D (1089 rows) Q2 FP32
+    // 55 -> 3.6, Q1 FP64 67 -> 6.0 us.  Forming a matrix takes 0.15 and 0.41, 0.51 and 0.56 ms there.
+    // Tails of more than kTailMatRows rows (option tail_max_n; 4225 rows would read 143 MB per
+    // segment, longer than k_tail takes), whose vectors do not fit the LDS with twice the digits, and further
+    // kinds beyond eight run k_tail.
     int build_tail_mats(const std::vector<u32>& ops)
     {
+      typedef typename std::conditional<sizeof(DT) == 8, mg::Dd, double>::type C;
       tail_mats.clear();
-      const u64 n = L[tail0]->n;
-      if(n > mg::kTailMatRows) return rt::kOk;
+      const u64 n = L[tail0]->n, lds = tail_lds / sizeof(DT) / 5 * 4 * sizeof(C);
+      if(n > mg::kTailMatRows || lds > tail_cap) return rt::kOk;
       std::vector<const TailSeg*> kinds;
       auto same = [&](const TailSeg& a, const TailSeg& b) {
         return a.count == b.count && a.out_buf == b.out_buf &&
                std::equal(ops.begin() + a.first, ops.begin() + a.first + a.count, ops.begin() + b.first);
       };
-      if(tail_lds > 65536)
-        F3_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&mg::k_tail<DT, VT, true>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(tail_lds)));
+      if(lds > 65536)
+        F3_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&mg::k_tail_columns<C, DT, VT>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
       for(TailSeg& g : tail_segs)
       {
         std::size_t k = 0;
@@ -1972,9 +1975,10 @@ namespace
         {
           if(k == 8) continue;
           std::unique_ptr<DevMem> m(new DevMem());
-          F3_RC(m->alloc(sizeof(DT) * n * n));
-          mg::k_tail<DT, VT, true><<<unsigned(n), mg::kTailThreads, tail_lds, s>>>(tail, tail_ops.template as<u32>() + g.first,
-                                                                                   g.count, g.out_buf, nullptr, m->template as<DT>());
+          F3_RC(m->alloc(sizeof(C) * n * n));
+          double* hi = m->template as<double>();
+          mg::k_tail_columns<C, DT, VT><<<unsigned(n), mg::kTailThreads, lds, s>>>(tail, tail_ops.template as<u32>() + g.first, g.count,
+                                                                                   g.out_buf, hi, hi + n * n);
           F3_RC(rt::check_launch());
           tail_mats.push_back(std::move(m));
           kinds.push_back(&g);
@@ -2610,8 +2614,11 @@ namespace
           }
           case Op::bottom:
             if(tail0 + 1 < nl && tail_segs[c.seg].mat >= 0)
-              mg::k_tail_apply<DT><<<unsigned((f.n + 3) / 4), kBlock, 0, s>>>(u32(f.n), tail_mats[tail_segs[c.seg].mat]->template as<DT>(),
-                                                                             f.rhs.template as<DT>(), f.xfinal, status);
+            {
+              const double* hi = tail_mats[tail_segs[c.seg].mat]->template as<double>();
+              mg::k_tail_apply<DT><<<unsigned((f.n + 3) / 4), kBlock, 0, s>>>(u32(f.n), hi, hi + f.n * f.n, f.rhs.template as<DT>(),
+                                                                             f.xfinal, status);
+            }
             else if(tail0 + 1 < nl)
             {
               const TailSeg& g = tail_segs[c.seg];

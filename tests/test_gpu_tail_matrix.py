@@ -42,3 +42,65 @@ def test_tail_matrix_matches_the_steps(torch, dim, deg, lvl, cycle, inner):
     err = np.linalg.norm(out[0] - out[1]) / np.linalg.norm(out[1])
     print(f"  {dim}D Q{deg} level {lvl} {cycle} {inner}: {err:.2e}", flush=True)
     assert err <= (1e-12 if inner == "f64" else 64 * np.finfo(np.float32).eps)
+
+
+def exact_cycle(H, d, L=0):
+    """The V(4,4) cycle in extended precision (np.longdouble), sparse matrices as they are."""
+    T = np.longdouble
+
+    def mul(M, v):
+        out = np.zeros(M.rows, T)
+        rows = np.repeat(np.arange(M.rows), np.diff(M.row_ptr.astype(np.int64)))
+        np.add.at(out, rows, M.val.astype(T) * v[M.col_ind.astype(np.int64)])
+        return out
+    A, bnd = H.levels[L].A, H.levels[L].bnd
+    rows = np.repeat(np.arange(A.rows), np.diff(A.row_ptr.astype(np.int64)))
+    diag = A.val[A.col_ind == rows].astype(T)
+    dinv = T(0.5) / diag
+    dinv[bnd] = 0
+    if H.levels[L].P is None:      # one inner node
+        return d * dinv * 2
+    x = dinv * d
+    for _ in range(3):
+        x = x + dinv * (d - mul(A, x))
+    r = d - mul(A, x)
+    r[bnd] = 0
+    r = mul(H.levels[L].R, r)
+    r[H.levels[L + 1].bnd] = 0
+    c = mul(H.levels[L].P, exact_cycle(H, r, L + 1))
+    c[bnd] = 0
+    x = x + c
+    for _ in range(4):
+        x = x + dinv * (d - mul(A, x))
+    return x
+
+
+@pytest.mark.parametrize("inner", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("dim,lvl", [(2, 2), (2, 4), (2, 5), (3, 2), (3, 3)])
+def test_tail_matrix_rounds_once(torch, dim, lvl, inner):
+    """Oscillatory, random and smooth right-hand sides, whose cycle on the tail is up to 100 times smaller
+    than |M| |b|: the product is that of the exact linear map, rounded once per value, so its relative
+    error (2-norm) is at most the unit roundoff u of the cycle's arithmetic.  The matrices are scaled to
+    whole numbers (2D 8 and -1, 3D 32, 0, -2 and -1), which every storage holds exactly, as it does dinv
+    and the coarse inverse.  Matrices of the cycle's own precision: up to 22 u."""
+    from feat3_amd.solver import MGPCG
+    H = pb.hierarchy(dim, 1, lvl, 1)
+    for i, L in enumerate(H.levels):
+        L.A.val = np.rint(L.A.val * (3.0 if dim == 2 else 12.0 * 2 ** (lvl - i)))
+    m = 2 ** lvl + 1
+    g = np.indices([m] * dim)
+    cases = {"checkerboard": np.where(g.sum(0) % 2 == 0, 1.0, -1.0).ravel(), "lines": np.where(g[-1] % 2 == 0, 1.0, -1.0).ravel(),
+             "random": np.random.default_rng(5).integers(-1000, 1000, m ** dim).astype(np.float64),
+             "smooth": np.rint(1000 * np.prod(np.sin(np.pi * g / (m - 1)), axis=0)).ravel()}
+    s = MGPCG(H, inner=inner).init()
+    assert s.info()["tail_levels"] == lvl
+    u = 2.0 ** -53 if inner == "f64" else 2.0 ** -24
+    for name, d in cases.items():
+        d[H.levels[0].bnd] = 0.0
+        c = torch.empty(m ** dim, dtype=torch.float64, device="cuda")
+        s.vcycle(c, torch.from_numpy(d).cuda())
+        e = exact_cycle(H, d.astype(np.longdouble))
+        err = float(np.linalg.norm((c.cpu().numpy() - e).astype(np.float64)) / np.linalg.norm(e.astype(np.float64)))
+        print(f"  {dim}D level {lvl} {inner} {name}: {err / u:.3f} u", flush=True)
+        assert err <= 1.001 * u
+    s.done()

@@ -2361,6 +2361,7 @@ namespace
       bool last;         // the cycle's last step on the finest level, where it can sum r.z too
     };
     std::vector<PlanOp> plan;
+    std::vector<PlanOp> steps;   // the cycle's operations one by one (statistics)
     bool zero_cols = false;   // the entry writes no iterate: lat::kColZero
 
     // blocks of the cycle's last launch (the partials of r.z), 0: it sums none
@@ -2383,6 +2384,8 @@ namespace
     void build_plan()
     {
       plan.clear();
+      steps.clear();
+      for(const CycleOp& c : cycle_ops) steps.push_back(PlanOp{c, false, 0, 0, false, false, false});
       const std::size_t nl = L.size();
       std::vector<char> zero(nl, 0);   // the level's first step from zero is left to its first launch
       for(std::size_t k = 0; k < cycle_ops.size();)
@@ -2537,20 +2540,20 @@ namespace
       });
     }
 
-    // evs (statistics only): an event is recorded before every operation k with span_start[k]
-    // set (span_start[0] is) and one after the last operation, so that each span of operations
-    // lies between two consecutive events
+    // one_by_one (statistics only): the operations of `steps` instead of the plan's; evs: an event is
+    // recorded before every operation k with span_start[k] set (span_start[0] is) and one after the last
+    // operation, so that each span of operations lies between two consecutive events
     // def: the defect to start from; null: the entry (rhs, and the iterate unless the first launch forms
     // it) was written by the kernel before.  dot_r: the cycle's last launch also leaves the partials
     // of dot_r . z (last_blocks() of them, where it can)
     int enqueue_vcycle(const double* def, const int* status, const std::vector<hipEvent_t>* evs = nullptr,
-                       const std::vector<char>* span_start = nullptr, const double* dot_r = nullptr)
+                       const std::vector<char>* span_start = nullptr, const double* dot_r = nullptr, bool one_by_one = false)
     {
       const std::size_t nl = L.size();
       std::vector<DT*> cur(nl, nullptr), oth(nl, nullptr);
       std::size_t k = 0, e = 0;
       bool fresh = true;   // before the finest level's first step
-      for(const PlanOp& o : plan)
+      for(const PlanOp& o : one_by_one ? steps : plan)
       {
         const CycleOp& c = o.c;
         const std::size_t i = c.lvl;
@@ -2566,7 +2569,8 @@ namespace
         {
           case Op::entry:
             if(def)
-              mg::k_mg_entry<DT><<<stream_blocks(f.n), kBlock, 0, s>>>(f.n, def, f.rhs.template as<DT>(), entry_x(),
+              mg::k_mg_entry<DT><<<stream_blocks(f.n), kBlock, 0, s>>>(f.n, def, f.rhs.template as<DT>(),
+                                                                      one_by_one && !zero_cols ? f.x.template as<DT>() : entry_x(),
                                                                       f.dinv.template as<DT>(), status);
             cur[0] = f.x.template as<DT>();
             oth[0] = f.t.template as<DT>();
@@ -2646,7 +2650,7 @@ namespace
         }
       }
       if(evs) F3_CHECK(hipEventRecord((*evs)[e], s));
-      if(cur[0] != L[0]->xfinal) return rt::kErrState;
+      if(cur[0] != L[0]->xfinal && !one_by_one) return rt::kErrState;
       return rt::check_launch();
     }
 
@@ -2655,20 +2659,23 @@ namespace
     // on the finer level as the reference does) and coarse solve per cycle, the number of each
     // operation per cycle, and the cycle's algorithmic bytes and flops on that level.  Fused
     // operations count where their main work is: the entry (conversion + first step) as smoothing
-    // on level 0, a brick launch (lattice_kernels.hpp) with the transfers and the defect in it as
-    // smoothing of its level, a restriction with the next level's first smoothing step as
+    // on level 0, a restriction with the next level's first smoothing step as
     // transfer (its step is counted as a smoothing step of the coarser level), and a segment of
-    // the single-workgroup coarse tail as the coarse solve of the tail's top level (one kernel:
+    // the coarse tail as the coarse solve of the tail's top level (one kernel:
     // the levels inside it report counts, bytes and flops, their time is that of the segment).
-    // Cycles are launched operation by operation, with an event wherever the level or the
+    // A level smoothed in bricks (lattice_kernels.hpp) takes its transfers, defects and steps in the
+    // same launches: its time is that of its launches, divided among the three as the operations share
+    // the level's time when they are launched one by one on its format (`steps`).
+    // Cycles are launched with an event wherever the level or the
     // category changes (a run of smoothing steps on one level is one span): an event costs the
     // stream a few microseconds, as much as a small level's operation, so one per operation
-    // would inflate the coarse levels' times.  The span times are scaled to the duration of the
+    // would inflate the coarse levels' times.  The times are scaled to the duration of the
     // cycle without events.  The solve itself is not touched (its graphs record no events).
     std::vector<hipEvent_t> stat_ev;
-    static int op_category(Op op)
+    static int op_category(const PlanOp& o)
     {
-      switch(op)
+      if(o.lat) return 4;   // several at once
+      switch(o.c.op)
       {
         case Op::entry: case Op::sweep: return 0;   // smoothing
         case Op::defect: return 1;
@@ -2677,17 +2684,16 @@ namespace
       }
       return 0;
     }
-    int statistics(int reps, double* out, int cap) override
+    // t[5 * level + category] += ms of `reps` cycles with events, of the plan or operation by operation
+    int time_spans(int reps, bool one_by_one, std::vector<double>& t)
     {
-      const std::size_t nl = L.size(), nops = plan.size();
-      const int need = 3 + 10 * int(nl);
-      if(reps < 1 || !out || cap < need) return rt::kErrArg;
+      const std::vector<PlanOp>& ops = one_by_one ? steps : plan;
       // spans: maximal runs of operations with the same level and category
-      std::vector<char> span_start(nops, 0);
-      std::vector<std::size_t> span_slot;   // 4 * level + category of each span
-      for(std::size_t k = 0; k < nops; ++k)
+      std::vector<char> span_start(ops.size(), 0);
+      std::vector<std::size_t> span_slot;   // 5 * level + category of each span
+      for(std::size_t k = 0; k < ops.size(); ++k)
       {
-        const std::size_t slot = 4 * plan[k].c.lvl + std::size_t(op_category(plan[k].c.op));
+        const std::size_t slot = 5 * ops[k].c.lvl + std::size_t(op_category(ops[k]));
         if(k == 0 || slot != span_slot.back())
         {
           span_start[k] = 1;
@@ -2695,20 +2701,57 @@ namespace
         }
       }
       const std::size_t nspan = span_slot.size();
-      // timing-only events: without the system-scope fence (a cache writeback and invalidation
-      // at every record) an event costs the stream less; the host synchronises the stream
-      // before it reads the times
       while(stat_ev.size() < nspan + 1)
       {
         hipEvent_t e = nullptr;
+        // without the system-scope release of the default event, which writes the L2s back at
+        // every recording: the spans are timed with the kernels' caches as the solve leaves them
+        // (3D Q1 L7 FP32 cycle: 0.54 with, 0.45 without the release, 0.39 ms untimed)
         F3_CHECK(hipEventCreateWithFlags(&e, hipEventDisableSystemFence));
         stat_ev.push_back(e);
       }
-      std::vector<double> t(4 * nl, 0.0), cnt(4 * nl, 0.0), by(nl, 0.0), fl(nl, 0.0);
-      F3_RC(enqueue_vcycle(r.template as<double>(), nullptr));   // warm-up
+      F3_RC(enqueue_vcycle(r.template as<double>(), nullptr, nullptr, nullptr, nullptr, one_by_one));   // warm-up
       F3_CHECK(hipStreamSynchronize(s));
-      // the cycle as it runs, and then with the events; the spans' times are scaled to the former, so
-      // that they add up to the cycle without the events' own cost
+      for(int rep = 0; rep < reps; ++rep)
+      {
+        F3_RC(enqueue_vcycle(r.template as<double>(), nullptr, &stat_ev, &span_start, nullptr, one_by_one));
+        F3_CHECK(hipStreamSynchronize(s));
+        for(std::size_t k = 0; k < nspan; ++k)
+        {
+          float ms = 0.f;
+          F3_CHECK(hipEventElapsedTime(&ms, stat_ev[k], stat_ev[k + 1]));
+          t[span_slot[k]] += double(ms);
+        }
+      }
+      return rt::kOk;
+    }
+    int statistics(int reps, double* out, int cap) override
+    {
+      const std::size_t nl = L.size();
+      const int need = 3 + 10 * int(nl);
+      if(reps < 1 || !out || cap < need) return rt::kErrArg;
+      std::vector<double> t5(5 * nl, 0.0), t(4 * nl, 0.0), cnt(4 * nl, 0.0), by(nl, 0.0), fl(nl, 0.0);
+      F3_RC(time_spans(reps, false, t5));
+      bool lattice = false;
+      double with_events = 0.0;
+      for(std::size_t i = 0; i < nl; ++i)
+      {
+        for(int q = 0; q < 5; ++q) with_events += t5[5 * i + q];
+        for(int q = 0; q < 4; ++q) t[4 * i + q] = t5[5 * i + q];
+        lattice = lattice || t5[5 * i + 4] > 0.0;
+      }
+      if(lattice)
+      {
+        std::vector<double> u(5 * nl, 0.0);
+        F3_RC(time_spans(reps, true, u));
+        for(std::size_t i = 0; i < nl; ++i)
+        {
+          const double all = u[5 * i] + u[5 * i + 1] + u[5 * i + 2];
+          for(int q = 0; q < 3; ++q) t[4 * i + q] += all > 0.0 ? t5[5 * i + 4] * u[5 * i + q] / all : (q == 0 ? t5[5 * i + 4] : 0.0);
+        }
+      }
+      // the cycle as it runs; the times are scaled to it, so that they add up to it without the
+      // events' own cost
       float plain = 0.f;
       F3_CHECK(hipEventRecord(t0, s));
       for(int rep = 0; rep < reps; ++rep) F3_RC(enqueue_vcycle(r.template as<double>(), nullptr));
@@ -2716,19 +2759,6 @@ namespace
       F3_CHECK(hipStreamSynchronize(s));
       F3_CHECK(hipEventElapsedTime(&plain, t0, t1));
       const double total = double(plain);
-      double with_events = 0.0;
-      for(int rep = 0; rep < reps; ++rep)
-      {
-        F3_RC(enqueue_vcycle(r.template as<double>(), nullptr, &stat_ev, &span_start));
-        F3_CHECK(hipStreamSynchronize(s));
-        float ms = 0.f;
-        for(std::size_t k = 0; k < nspan; ++k)
-        {
-          F3_CHECK(hipEventElapsedTime(&ms, stat_ev[k], stat_ev[k + 1]));
-          t[span_slot[k]] += double(ms);
-          with_events += double(ms);
-        }
-      }
       if(with_events > 0.0)
         for(double& v : t) v *= total / with_events;
       // counts, bytes and flops of the cycle's mathematical operations (the full schedule, tail
@@ -2763,7 +2793,7 @@ namespace
       }
       out[0] = double(nl);
       out[1] = total / reps;
-      out[2] = double(nops);
+      out[2] = double(steps.size());
       for(std::size_t i = 0; i < nl; ++i)
       {
         double* o = out + 3 + 10 * i;

@@ -398,14 +398,17 @@ int feat3_mgpcg_time_kernel(feat3_mgpcg* h, int which, int reps, double* avg_ms,
 int feat3_mgpcg_info(feat3_mgpcg* h, uint64_t* out, int cap);
 /* Per-level statistics of the multigrid cycle (MultiGridHierarchy::get_time_smooth/_defect/
  * _transfer/_coarse, multigrid.hpp:858-956, and the flop counter of Statistics,
- * util/statistics.hpp:206-230): `reps` cycles launched operation by operation on the solver's
- * stream with an event wherever the level or the category changes (the solve's own graphs are
- * untouched).  out[0] levels L, out[1] ms per cycle (first to last event), out[2] operations
- * per cycle; then for each level
+ * util/statistics.hpp:206-230): `reps` cycles launched on the solver's stream with an event
+ * wherever the level or the category changes (the solve's own graphs are untouched).  out[0]
+ * levels L, out[1] ms per cycle as it runs, without events (the levels' times are scaled to add up to
+ * it), out[2] operations per cycle; then for each level
  * (finest first) 10 values: ms per cycle in smoothing, defect, grid transfer (restriction and
  * prolongation, on the finer level as the reference counts them), coarse solve; the number of
  * smoothing steps, defects, transfers and coarse solves per cycle; algorithmic bytes and flops
- * per cycle.  A segment of the single-workgroup coarse tail counts as the coarse solve of its
+ * per cycle of these operations on the level's format.  A level smoothed in bricks (option "lattice")
+ * takes the first three in the same launches: the time of its launches is divided among them as they
+ * share the level's time when launched one by one on its format.  A segment of the coarse tail
+ * counts as the coarse solve of its
  * top level (its levels report counts, bytes and flops; their time is the segment's).
  * cap >= 3 + 10 L.  Creates its events at the first call. */
 int feat3_mgpcg_statistics(feat3_mgpcg* h, int reps, double* out, int cap);

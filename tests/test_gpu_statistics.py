@@ -86,3 +86,31 @@ def test_wcycle_coarse_solves(torch):
     for i in range(nl - 1):
         assert st["num_smooth"][i] >= (2 ** i) * 8
     s.done()
+
+
+@pytest.mark.parametrize("dim,deg,lvl,inner,cycle", [(3, 1, 6, "f32", "v"), (2, 2, 7, "f32", "f"), (2, 1, 7, "f64", "v"),
+                                                     (3, 1, 5, "f16", "w")])
+def test_every_category_has_its_time(torch, dim, deg, lvl, inner, cycle):
+    """Levels smoothed in bricks take their steps, defects and transfers in the same launches; each category
+    still has its share of the level's time wherever it has operations, the shares add up to the cycle,
+    and a solve behind the statistics is the one before them."""
+    from feat3_amd.solver import MGPCG
+    print(f"case statistics categories {dim}D Q{deg} L{lvl} {inner} {cycle}", flush=True)
+    H = pb.hierarchy(dim, deg, lvl, 1)
+    b = torch.from_numpy(pb.filtered_rhs(H, 0)).cuda()
+    x, y = torch.zeros_like(b), torch.zeros_like(b)
+    s = MGPCG(H, inner=inner, cycle=cycle).init()
+    ref = s.correct(x, b)
+    for _ in range(2):
+        st = s.statistics(5)
+        info = s.info()
+        upper = info["levels"] - info["tail_levels"]      # the tail's time is its first level's
+        assert upper >= 1 and info["kernels_per_vcycle"] < st["operations"]
+        times = np.stack([st["time_smooth"], st["time_defect"], st["time_transfer"], st["time_coarse"]])
+        nums = np.stack([st["num_smooth"], st["num_defect"], st["num_transfer"], st["num_coarse"]])
+        assert ((times[:3, :upper] > 0) == (nums[:3, :upper] > 0)).all(), times
+        assert (nums[:3, :upper] > 0).all() and times[3, upper] > 0
+        assert (times[:3, upper:] == 0).all() and (times[3, :upper] == 0).all()
+        assert abs(float(times.sum()) - st["ms_per_cycle"]) <= 1e-6 * st["ms_per_cycle"]
+    assert s.correct(y, b) == ref and torch.equal(x, y)
+    s.done()

@@ -76,6 +76,20 @@ def sweep_algorithmic_bytes(info, n, nnz, nchunks):
     return nnz * (s_v + 4) + 4 * (n + 1) + n * s_x * 4
 
 
+def launch_bytes(info, counted, by_values):
+    """Bytes of the finest sweep that time_kernel(0) launches: the solver's own count where it reads 4-bit
+    codes or, by columns, no matrix at all; else the format's (sweep_algorithmic_bytes)."""
+    return counted if info["banded"] == 3 or info["finest_lattice"] == 2 else by_values
+
+
+def sweep_kernel_name(finest_lattice):
+    """The kernel behind sweep_us (time_kernel(0)) for info()["finest_lattice"]."""
+    return {0: "k_sweep, finest level (fused damped-Jacobi step)",
+            1: "k_sweep, finest level (fused damped-Jacobi step) on its format; the cycle smooths this level in bricks "
+               "(k_lattice, several steps per launch) and does not launch it",
+            2: "k_columns, finest level (fused damped-Jacobi step)"}[finest_lattice]
+
+
 def _timed(fn, steps, warmup):
     import torch
     for _ in range(warmup):
@@ -271,7 +285,8 @@ def bench_coeff16(args):
                          f"{dt:.2f} s solve phase)"}
     roof = {"bound": "hbm", "achieved": head["sweep_GBs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": head["sweep_GBs"] / HBM_PEAK_GBS, "traffic": None,
-            "kernel": "batch k_sweep<B=1, per-system values>, finest level (16 fields)",
+            "kernel": "batch k_sweep<B=1, per-system values>, finest level (16 fields), one step of its own" +
+                      (f" (the cycle takes up to {steps} in one pass, k_field_rows)" if (steps := s.info()["steps_per_pass"]) else ""),
             "bytes_per_launch": head["sweep_bytes"], "avg_launch_us": head["sweep_us"]}
     cfg = {"workload": f"2D variable-coefficient diffusion Q1 level {lvl} ({prob.nodes} DOF), 16 coefficient fields: "
                        f"differentiable solve (device assembly, forward + adjoint batched PCG(FP64) + MG V(4,4), "
@@ -530,13 +545,15 @@ def main():
         sb_values = sweep_algorithmic_bytes(dict(info, banded=1) if info["banded"] == 3 else info, n,
                                             band_nnz(H.levels[0].A, inner, upper=info["banded"] == 2),
                                             info["sell_chunks"])
-        sb = sweep_stored_bytes if info["banded"] == 3 else sb_values
+        sb = launch_bytes(info, sweep_stored_bytes, sb_values)
+        by_columns = info["finest_lattice"] == 2      # no matrix stream: no value-stored equivalent of the step
         r = dict(ms_per_solve=ms, ms_min=1e3 * min(times), iterations=iters,
                  dof_iter_per_s=n * sum(iters) / sum(times), final_rel_residual=float(hist[-1] / hist[0]),
                  sweep_us=sweep_ms * 1e3, sweep_bytes=sb, sweep_GBs=sb / (sweep_ms * 1e-3) / 1e9,
                  level_format={0: "csr/sell", 1: "band", 2: "symmetric band", 3: "value-coded band"}[info["banded"]],
-                 sweep_value_bytes=sb_values, sweep_value_GBs=sb_values / (sweep_ms * 1e-3) / 1e9,
-                 vcycle_ms=vc_ms, kernels_per_vcycle=info["kernels_per_vcycle"],
+                 sweep_value_bytes=None if by_columns else sb_values,
+                 sweep_value_GBs=None if by_columns else sb_values / (sweep_ms * 1e-3) / 1e9,
+                 vcycle_ms=vc_ms, kernels_per_vcycle=info["kernels_per_vcycle"], finest_lattice=info["finest_lattice"],
                  outer_product_us=outer_ms * 1e3, outer_product_bytes=outer_bytes,
                  outer_product_GBs=outer_bytes / (outer_ms * 1e-3) / 1e9)
         log(f"{inner}/{fmt}/{cycle}: {ms:.3f} ms/solve, it {iters}, rel.res {r['final_rel_residual']:.2e}, "
@@ -629,7 +646,7 @@ def main():
         "iterations": float(np.mean(iters)),
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                     "kernel": ("k_columns" if dim == 3 and args.level >= 7 else "k_sweep") + ", finest level (fused damped-Jacobi step)",
+                     "kernel": sweep_kernel_name(head["finest_lattice"]),
                      "bytes_per_launch": head["sweep_bytes"], "avg_launch_us": head["sweep_us"]},
         "headline": head,
         "variants": {k: v[0] for k, v in variants.items()},

@@ -92,6 +92,12 @@ class BatchMGPCG:
         capi.call("feat3_batch_time_kernel", self._h, which, reps, ctypes.byref(ms), ctypes.byref(nb))
         return ms.value, nb.value
 
+    def info(self) -> dict:
+        out = np.zeros(7, np.uint64)
+        capi.call("feat3_batch_info", self._h, _ptr(out), out.size)
+        keys = ["levels", "tail_levels", "line_levels", "pass_levels", "steps_per_pass", "lattice_prolongations", "outer_lines"]
+        return {k: int(v) for k, v in zip(keys, out)}
+
     def done(self) -> None:
         if getattr(self, "_h", None) is not None and self._h.value:
             capi.lib.feat3_batch_destroy(self._h)

@@ -3121,32 +3121,54 @@ namespace
     // iteration excluding the V-cycle, [8] sizeof inner DT, [9] sizeof VT
     int info(u64* out, int cap) override
     {
-      std::vector<u64> v(17, 0);
+      std::vector<u64> v(22, 0);
       v[0] = L.size();
       v[1] = L.front()->n;
       v[2] = L.front()->A.nnz;
       v[3] = u64(L.front()->A.lanes);
       v[4] = L.front()->A.sell_size;
+      // what the launches of the cycle move: matrices in their formats, vectors once per launch
       u64 bytes = 0;
       const u64 vb = sizeof(DT);
-      for(const CycleOp& c : cycle_ops)
+      bool fresh = true;
+      for(const PlanOp& o : plan)
       {
+        const CycleOp& c = o.c;
         const Level<DT, VT>& f = *L[c.lvl];
         const u64 nc = c.lvl + 1 < L.size() ? L[c.lvl + 1]->n : 0;
+        if(o.lat)
+        {
+          const bool mem = o.in == lat::kMem || o.in == lat::kProl;
+          if(f.lat == 3) bytes += f.n * vb * 10 + (f.n + 31) / 32 * 4;   // values of the nine neighbours, dinv, mask
+          bytes += o.in == lat::kEntry ? f.n * (8 + vb) : f.n * vb;
+          bytes += mem ? f.n * vb : 0;
+          bytes += o.in == lat::kProl ? nc * vb : 0;
+          bytes += !mem || o.sweeps > 0 || o.in == lat::kProl ? f.n * vb : 0;
+          bytes += o.rest ? nc * vb * (o.step ? 3 : 1) : 0;
+          continue;
+        }
         switch(c.op)
         {
-          case Op::entry: bytes += f.n * (8 + vb * 3); break;
-          case Op::sweep: bytes += f.A.matrix_bytes() + f.n * vb * 4; break;
-          case Op::defect: bytes += f.A.matrix_bytes() + f.n * vb * 3; break;
+          case Op::entry: bytes += f.n * (8 + vb) + (entry_x() ? f.n * vb * 2 : 0); break;
+          case Op::sweep:
+            bytes += f.cols ? f.n * vb * (c.lvl == 0 && zero_cols && fresh ? 2 : 3) : f.A.matrix_bytes() + f.n * vb * 4;
+            fresh = fresh && c.lvl != 0;
+            break;
+          case Op::defect: bytes += (f.cols ? 0 : f.A.matrix_bytes()) + f.n * vb * 3; break;
           case Op::rest: bytes += f.R.matrix_bytes() + f.n * vb + nc * vb * 2; break;
           case Op::rest_step: bytes += f.R.matrix_bytes() + f.n * vb + nc * vb * 4; break;
-          case Op::bottom: bytes += ncoarse * ncoarse * 8 + ncoarse * vb * 2; break;
-          case Op::prol: bytes += f.P.matrix_bytes() + nc * vb + f.n * vb * 2; break;
+          case Op::bottom:
+            if(tail0 + 1 < L.size() && tail_segs[c.seg].mat >= 0) bytes += f.n * f.n * (vb == 8 ? 16 : 8) + f.n * vb * 2;
+            else bytes += ncoarse * ncoarse * 8 + ncoarse * vb * 2;
+            break;
+          case Op::prol: bytes += (f.cols ? 0 : f.P.matrix_bytes()) + nc * vb + f.n * vb * 2; break;
         }
       }
       v[5] = plan.size();
       v[6] = bytes;
-      v[7] = outer_matrix().matrix_bytes() + n0 * 8 * 2 + n0 * 8 * 5 + n0 * (8 + vb) * 2 + n0 * (8 + vb * 2);
+      // q = A p; x, r and the cycle's entry; r.z (in the cycle's last launch it reads r alone); p
+      v[7] = (out_m ? 0 : outer_matrix().matrix_bytes()) + n0 * 8 * 2 + n0 * 8 * 6 +
+             (entered() ? n0 * vb * (entry_x() ? 3 : 1) : 0) + n0 * (last_blocks() ? 8 : 8 + vb) + n0 * (16 + vb);
       v[8] = sizeof(DT);
       v[9] = sizeof(VT);
       v[10] = L.front()->A.sell_d16 ? 1 : 0;
@@ -3155,8 +3177,16 @@ namespace
       v[13] = L.front()->A.ndiag;
       v[14] = tail0 + 1 < L.size() ? L.size() - tail0 : 0;
       v[15] = tail_lds;
-      for(const auto& l : L) v[16] += l->P.tensor ? 1 : 0;
-      for(int i = 0; i < cap && i < 17; ++i) out[i] = v[i];
+      for(const auto& l : L)
+      {
+        v[16] += l->P.tensor ? 1 : 0;
+        v[18] += l->lat >= 0 && !l->cols ? 1 : 0;
+        v[19] += l->cols ? 1 : 0;
+      }
+      v[17] = L.front()->cols ? 2 : (L.front()->lat >= 0 ? 1 : 0);
+      v[20] = out_m ? 1 : 0;
+      v[21] = tail_mats.size();
+      for(int i = 0; i < cap && i < int(v.size()); ++i) out[i] = v[i];
       return rt::kOk;
     }
   };

@@ -196,6 +196,7 @@ namespace
     virtual int time_kernel(int which, int reps, double* ms, u64* bytes) = 0;
     virtual bool set_tolerances(const Config& c) = 0;
     virtual int set_values(int level, const double* dvals) = 0;
+    virtual void info(u64 (&v)[7]) const = 0;
   };
 
   // device-side refresh of a level's values (feat3_batch_set_values): storage conversion and
@@ -1336,6 +1337,22 @@ namespace
       return rt::kOk;
     }
 
+    void info(u64 (&v)[7]) const override
+    {
+      for(u64& q : v) q = 0;
+      v[0] = L.size();
+      v[1] = tail0 + 1 < L.size() ? L.size() - tail0 : 0;
+      for(std::size_t i = 0; i < tail0; ++i)
+      {
+        const Level& l = *L[i];
+        v[2] += l.m ? 1 : 0;
+        v[3] += l.fm ? 1 : 0;
+        if(l.fm) v[4] = u64(kFieldSteps);
+        v[5] += l.pdim ? 1 : 0;
+      }
+      v[6] = out_m ? 1 : 0;
+    }
+
     // which: 0 finest smoothing sweep (all systems), 2 outer FP64 q = A p with dot, 3 one V-cycle
     int time_kernel(int which, int reps, double* ms, u64* bytes) override
     {
@@ -1557,6 +1574,15 @@ int feat3_batch_time_kernel(feat3_batch* h, int which, int reps, double* avg_ms,
 {
   if(!h || !h->eng || !avg_ms) return rt::kErrState;
   return h->eng->time_kernel(which, reps, avg_ms, bytes);
+}
+
+int feat3_batch_info(feat3_batch* h, u64* out, int cap)
+{
+  if(!h || !h->eng || !out) return rt::kErrState;
+  u64 v[7];
+  h->eng->info(v);
+  for(int i = 0; i < cap && i < 7; ++i) out[i] = v[i];
+  return rt::kOk;
 }
 
 } // extern "C"

@@ -12,7 +12,9 @@ the fastest:
 The objective is the measured time of one full V-cycle (feat3_*_time_kernel(3)), which covers
 every level, the transfers and the coarse solve, i.e. what a PCG iteration spends in the
 preconditioner.  Stage 1 searches format and chunk shape at the default grid, stage 2 the rows
-per workgroup for the winner, stage 3 the rows per workgroup of its transfer kernels.  Results can be cached in a JSON file keyed by the problem shape.
+per workgroup for the winner, stage 3 the rows per workgroup of its transfer kernels.  Levels
+smoothed in bricks or by columns (solver.MGPCG.info) use none of these shapes: there the stages choose for
+the remaining levels and the outer product only.  Results can be cached in a JSON file keyed by the problem shape.
 """
 from __future__ import annotations
 

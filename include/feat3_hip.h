@@ -357,6 +357,11 @@ int feat3_mgpcg_set_launch(feat3_mgpcg* h, int graph, int lanes, uint64_t sell_C
  * "transfer_rows_per_block" (row positions per workgroup of the transfer kernels, default 128;
  * 0 = derived from the row count), "symmetric_band" (1, default: an FP64 band equal to its mirror
  * image bit for bit stores only its center and upper diagonals; 0: the full band; same results),
+ * "lattice" (1, default: levels that are lattices with one matrix row for all inner nodes, one per
+ * parity of the coordinates (2D Q2) or any (2D Q1) are smoothed in bricks, several steps with the
+ * transfers in one launch, or, in 3D from 2^20 nodes on, by columns, as is the FP64 product there:
+ * the sums of the banded format bit for bit; CSR and SELL-C-sigma differ from it by rounding;
+ * 0: one launch per step on the level's format),
  * "cycle" (the multigrid cycle, MultiGridCycle of multigrid.hpp:26-34: 0 V, default, 1 F,
  * 2 W; the coarse-tail kernel runs the cycle's steps on the small levels for each of them);
  * "plane_order" (order in which the blocks of a banded row kernel take their row ranges: 0
@@ -387,14 +392,19 @@ int feat3_mgpcg_vcycle(feat3_mgpcg* h, void* caller_stream, double* cor, const d
 int feat3_mgpcg_history(feat3_mgpcg* h, double* out_host, uint64_t cap, uint64_t* len);
 /* average duration of `reps` launches of one hot-path kernel on the solver's stream
  * (which: 0 finest smoothing sweep, 1 finest defect, 2 outer FP64 product q = A p with its dot
- * partials, 3 full cycle) and its algorithmic bytes */
+ * partials, 3 full cycle) and its algorithmic bytes.  0 and 1 are one step and one defect on the
+ * finest level's format, or by columns; the cycle launches neither where that level is smoothed in
+ * bricks (feat3_mgpcg_info) */
 int feat3_mgpcg_time_kernel(feat3_mgpcg* h, int which, int reps, double* avg_ms, uint64_t* bytes);
 /* [levels, n, nnz, lanes, sell size, kernels per cycle, cycle bytes, outer bytes,
  *  sizeof inner, sizeof stored value, 16-bit SELL columns on the finest level, SELL chunks
  *  of the finest level, finest level banded (0 no, 1 yes, 2 with symmetric storage: center and
  *  upper diagonals only, 3 value-coded), its number of diagonals, levels run by the
- *  single-workgroup coarse tail (0: none), LDS bytes of the tail, levels whose transfers are
- *  evaluated as tensor products of their 1D factors] */
+ *  coarse tail (0: none), LDS bytes of the tail, levels whose transfers are
+ *  evaluated as tensor products of their 1D factors, the finest level's smoothing (0 one launch per
+ *  step on its format, 1 in bricks, 2 by columns), levels smoothed in bricks, by columns, outer
+ *  product by columns (0/1), matrices of the coarse tail's segments (0: the tail runs step by step)];
+ * the bytes are what the launches move: matrices in their formats, each vector once per launch */
 int feat3_mgpcg_info(feat3_mgpcg* h, uint64_t* out, int cap);
 /* Per-level statistics of the multigrid cycle (MultiGridHierarchy::get_time_smooth/_defect/
  * _transfer/_coarse, multigrid.hpp:858-956, and the flop counter of Statistics,
@@ -470,8 +480,14 @@ int feat3_batch_set_values(feat3_batch* h, int level, const double* values);
 /* defect norms of system `system` in the last solve */
 int feat3_batch_history(feat3_batch* h, int system, double* out_host, uint64_t cap, uint64_t* len);
 /* which: 0 finest smoothing sweep (all systems), 2 outer FP64 q = A p with q.p partials,
- * 3 one V-cycle; algorithmic bytes of one launch (0, 2) */
+ * 3 one V-cycle; algorithmic bytes of one launch (0, 2).  0 is one step of its own; the cycle takes
+ * several in a pass on 2D lattices with values per system (feat3_batch_info) */
 int feat3_batch_time_kernel(feat3_batch* h, int which, int reps, double* avg_ms, uint64_t* bytes);
+/* how the solver runs: [levels, levels in the workgroup-per-system coarse tail (0: none), 3D lattice
+ * levels by lines, 2D lattice levels with several steps in a pass, the most steps of such a pass (0: no
+ * such level), levels above the tail whose prolongation takes its closed form, outer product by
+ * lines (0/1)] */
+int feat3_batch_info(feat3_batch* h, uint64_t* out, int cap);
 
 /* ===================================================================================== */
 /* Adjoint gradient of the variable-coefficient diffusion solve (no counterpart in the    */

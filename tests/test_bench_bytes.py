@@ -34,3 +34,14 @@ def test_sweep_bytes_per_format():
     assert bench.sweep_algorithmic_bytes(sell, n, nnz, 16) == nnz * 6 + 8 * 16 + 16 * n
     band = dict(csr, banded=1, ndiag=9)
     assert bench.sweep_algorithmic_bytes(band, n, nnz, 0) == nnz * 4 + 4 * 9 + 16 * n
+
+
+def test_sweep_bytes_are_those_of_the_kernel_that_ran():
+    """By columns (finest_lattice 2) and with value-coded bands the solver's count is taken; the label says
+    which kernel ran, and that bricks replace the step in the cycle."""
+    for banded in (0, 1, 2, 3):
+        for finest in (0, 1, 2):
+            got = bench.launch_bytes(dict(banded=banded, finest_lattice=finest), 10, 1000)
+            assert got == (10 if banded == 3 or finest == 2 else 1000)
+    assert bench.sweep_kernel_name(2).startswith("k_columns") and bench.sweep_kernel_name(0).startswith("k_sweep")
+    assert "does not launch it" in bench.sweep_kernel_name(1)

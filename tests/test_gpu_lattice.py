@@ -197,3 +197,30 @@ def test_row_kernels_with_and_without_tensor_transfers(torch_cuda, dim, deg, lvl
             out.append((st, it, x.cpu().numpy()))
             s.done()
         assert out[0][:2] == out[1][:2] and np.array_equal(out[0][2], out[1][2])
+
+
+@pytest.mark.parametrize("dim,deg,lvl,coef,route", [(2, 1, 7, False, 1), (2, 1, 7, True, 1), (2, 2, 6, False, 1), (3, 1, 5, False, 1),
+                                                    (3, 1, 7, False, 2), (3, 2, 3, False, 0)])
+def test_info_tells_the_route_and_its_bytes(torch, dim, deg, lvl, coef, route):
+    """info() names the way the finest level is smoothed; the cycle's bytes are those of its launches: on
+    lattice levels vectors only (at most five of the level and three of the next one a launch; ten more
+    with a row of values per node), so fewer than with one launch per step."""
+    from feat3_amd.solver import MGPCG
+    k = torch.exp(torch.rand(1 << (2 * lvl), dtype=torch.float64, device="cuda")) if coef else None
+    levels = pb.hierarchy(dim, deg, lvl, 1) if deg == 2 and dim == 3 else pb.hierarchy_device(dim, deg, lvl, 1, k)
+    info = []
+    for lattice in (1, 0):
+        s = MGPCG(levels, inner="f32", options={"lattice": lattice}).init()
+        info.append(s.info())
+        s.done()
+    a, b = info
+    upper = a["levels"] - a["tail_levels"]
+    assert a["finest_lattice"] == route and b["finest_lattice"] == 0
+    assert (a["brick_levels"], a["column_levels"]) == {0: (0, 0), 1: (upper, 0), 2: (upper - 1, 1)}[route]
+    assert b["brick_levels"] == b["column_levels"] == b["outer_columns"] == 0 and a["outer_columns"] == (route == 2)
+    assert a["tail_matrices"] == b["tail_matrices"] == 1
+    assert (a["vcycle_bytes"] < b["vcycle_bytes"]) == (route > 0) and (a["outer_bytes"] < b["outer_bytes"]) == (route > 0)
+    if route == 1:
+        m = ((deg << lvl) + 1) ** dim
+        tail = 2 * 4 * 1100 + 8 * 1100 ** 2
+        assert a["vcycle_bytes"] <= a["kernels_per_vcycle"] * 4 * m * (8 + (10 if coef else 0)) + tail

@@ -23,8 +23,10 @@ def solve(torch, H, B, nsys, vals, block, inner, lattice, x0=None, iters=4):
     st, it = s.correct(x, torch.from_numpy(np.ascontiguousarray(B)).cuda())
     h = [s.history(k)[: iters + 1] for k in range(nsys)]
     nbytes = s.time_kernel(0, 1)[1]
+    route = {k: s.info()[k] for k in ("line_levels", "outer_lines", "lattice_prolongations")}
+    assert lattice or not any(route.values())
     s.done()
-    return list(st), list(it), x.cpu().numpy(), np.array(h), nbytes
+    return list(st), list(it), x.cpu().numpy(), np.array(h), nbytes, route
 
 
 @pytest.mark.parametrize("inner", ["f64", "f32", "f16"])
@@ -41,6 +43,7 @@ def test_lines_match_the_row_kernels(torch_cuda, inner, level, block, nsys):
     b = solve(torch, H, B, nsys, vals, block, inner, 0, x0)
     assert a[0] == b[0] and a[1] == b[1]
     assert a[4] < b[4]   # the route was taken: no matrix among the sweep's bytes
+    assert a[5] == {"line_levels": level - 1, "outer_lines": 1, "lattice_prolongations": level - 1}
     assert np.allclose(a[3], b[3], rtol=1e-10, atol=0)
     assert np.linalg.norm(a[2] - b[2]) <= 1e-10 * np.linalg.norm(b[2])
     assert np.array_equal(a[3][:, 0] > 0, b[3][:, 0] > 0)
@@ -68,7 +71,7 @@ def test_unequal_rows_keep_the_row_kernels(torch_cuda, change):
     for inner in ("f64", "f32"):
         a = solve(torch, H, B, 4, vals, 1, inner, 1, iters=2)
         b = solve(torch, H, B, 4, vals, 1, inner, 0, iters=2)
-        assert a[4] == b[4]
+        assert a[4] == b[4] and a[5]["outer_lines"] == 0 and a[5]["line_levels"] == len(H.levels) - 2
         assert np.array_equal(a[3], b[3])
         assert np.linalg.norm(a[2] - b[2]) <= 1e-11 * np.linalg.norm(b[2])
 
@@ -89,8 +92,10 @@ def test_new_values_leave_the_lines(torch_cuda):
         s = BatchMGPCG(H, 4, inner="f64", tol_rel=0.0, min_iter=3, max_iter=3, options={"lattice": lattice}).init()
         x = torch.zeros(s.shape, dtype=torch.float64, device="cuda")
         s.correct(x, B)
+        lines = s.info()["line_levels"]
         dv = torch.from_numpy(new).cuda()
         capi.call("feat3_batch_set_values", s._h, 0, ctypes.c_void_p(dv.data_ptr()))
+        assert s.info()["outer_lines"] == 0 and s.info()["line_levels"] == max(0, lines - 1)
         x.zero_()
         s.correct(x, B)
         out.append(x.cpu().numpy())

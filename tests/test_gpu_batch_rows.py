@@ -31,6 +31,9 @@ def test_rows_match_single_steps(torch_cuda, inner, level, nsys, pre, post):
     for lattice in (1, 0):
         s = BatchMGPCG(H, nsys, values=vals, shared=False, inner=inner, pre=pre, post=post, tol_rel=0.0, min_iter=3,
                        max_iter=3, options={"lattice": lattice}).init()
+        info = s.info()      # the route: levels of 100 nodes per axis or more
+        assert info["pass_levels"] == (level - 6 if lattice else 0)
+        assert info["steps_per_pass"] == ({"f64": 2, "f32": 4, "f16": 3}[inner] if lattice else 0)
         x = torch.from_numpy(x0).cuda()
         s.correct(x, torch.from_numpy(np.ascontiguousarray(B)).cuda())
         out.append((x.cpu().numpy(), np.array([s.history(k) for k in range(nsys)])))
@@ -58,6 +61,14 @@ def test_field_tail_is_identical(torch_cuda, inner, dim, level, nsys, tail):
     out = []
     for t in (tail, 0):
         s = BatchMGPCG(H, nsys, values=sets[0], shared=False, inner=inner, options={"tail_max_n": t}).init()
+        # the deepest levels within the limit whose five vectors fit 160 KB of LDS
+        used, want = 0, 0
+        for L in reversed(H.levels):
+            used += 5 * L.A.rows * (8 if inner == "f64" else 4)
+            if want and (L.A.rows > t or used > 160 * 1024):
+                break
+            want += 1
+        assert s.info()["tail_levels"] == (want if want > 1 else 0)
         res = []
         for new in (False, True):
             if new:
@@ -92,6 +103,7 @@ def test_lattice_prolongation_is_identical(torch_cuda, case):
         for lattice in (1, 0):
             s = BatchMGPCG(H, nsys, values=vals, shared=False, inner="f32", tol_rel=0.0, min_iter=2, max_iter=2,
                            options={"lattice": lattice}).init()
+            assert s.info()["lattice_prolongations"] == (1 if lattice and case == "q1" else 0)
             x = torch.zeros(s.shape, dtype=torch.float64, device="cuda")
             s.correct(x, B)
             out.append(x.cpu().numpy())

@@ -161,6 +161,8 @@ def test_columns_are_bitwise_the_steps(torch, inner):
     out = []
     for lattice in (1, 0):
         s = MGPCG(levels, inner=inner, fmt="banded", options={"lattice": lattice}).init()
+        info = s.info()
+        assert (info["column_levels"], info["outer_columns"]) == (lattice, lattice)
         c = torch.empty_like(b)
         for _ in range(2):
             s.vcycle(c, b)
@@ -224,3 +226,134 @@ def test_info_tells_the_route_and_its_bytes(torch, dim, deg, lvl, coef, route):
         m = ((deg << lvl) + 1) ** dim
         tail = 2 * 4 * 1100 + 8 * 1100 ** 2
         assert a["vcycle_bytes"] <= a["kernels_per_vcycle"] * 4 * m * (8 + (10 if coef else 0)) + tail
+
+
+@pytest.mark.parametrize("inner,fmt,cycle,pre,post", [
+    ("f32", "banded", "v", 1, 3),      # the entry writes the first iterate and the defect follows it
+    ("f64", "banded", "v", 2, 2),      # the step that forms the entry's iterate, then the defect
+    ("f32", "banded", "f", 3, 1),      # the cycle's last step is the only one behind the prolongation
+    ("f16", "banded", "v", 4, 4), ("f16", "banded", "f", 1, 1), ("f64", "banded", "f", 4, 4),
+    ("f32", "csr", "v", 4, 4), ("f16", "sell", "v", 2, 3)])
+def test_columns_in_every_cycle(torch, inner, fmt, cycle, pre, post):
+    """129^3 nodes by columns against one launch per step: the cycle bit for bit with bands (rounding of the
+    products in the general formats, as test_other_formats_agree), the solve's iterations alike."""
+    from feat3_amd.solver import MGPCG
+    print(f"case columns {inner} {fmt} {cycle}({pre},{post})", flush=True)
+    levels = pb.hierarchy_device(3, 1, 7, 1)
+    n = levels[0].A.rows
+    b = torch.rand(n, dtype=torch.float64, device="cuda", generator=torch.Generator("cuda").manual_seed(3)) - 0.5
+    b[levels[0].bnd.long()] = 0.0
+    out = []
+    for lattice in (1, 0):
+        s = MGPCG(levels, inner=inner, fmt=fmt, cycle=cycle, pre=pre, post=post, options={"lattice": lattice}).init()
+        assert (s.info()["column_levels"], s.info()["outer_columns"]) == (lattice, lattice)
+        c, x = torch.empty_like(b), torch.zeros_like(b)
+        for _ in range(2):
+            s.vcycle(c, b)
+        r = s.correct(x, b)
+        out.append((c, x, r))
+        s.done()
+    (c, x, r), (d, y, q) = out
+    eps = 2.0 ** -52 if inner == "f64" else 2.0 ** -23
+    if fmt == "banded":
+        assert torch.equal(c, d)
+    else:
+        assert float((c - d).norm()) <= 27 * eps * float(d.norm())
+    assert r == q and r[0] == 2
+    # FP64 dot products of 2e6 terms grouped by other blocks; other formats: cycles that differ by rounding
+    assert float((x - y).norm()) <= (1e-12 if fmt == "banded" else 1e-8) * float(y.norm())
+
+
+@pytest.mark.parametrize("dim,lvl,inner", [(2, 11, "f32"), (3, 8, "f32"), (3, 8, "f64")])
+def test_sums_of_more_blocks_than_are_folded(torch, dim, lvl, inner):
+    """The cycle's last launch and, in 3D, the outer product leave more partial sums than every block of
+    the next kernel adds up (2048): a launch of its own adds them.  2049^2 nodes: 3182 blocks; 257^3
+    nodes: 8385 (FP32) and 8450.  Against one launch per step: the same iterations.  The dot products are
+    grouped otherwise (2e7 terms, 1e-16 each), so the defects differ in their last digits, and a value
+    of them may round to the other FP32 neighbour for the cycle: that changes a correction by at most
+    u = 6e-8 of its norm, the next defect by as much of the one before, and the solution by as much."""
+    from feat3_amd.solver import MGPCG
+    print(f"case many partials {dim}D L{lvl} {inner}", flush=True)
+    levels = pb.hierarchy_device(dim, 1, lvl, 1)
+    n = levels[0].A.rows
+    b = torch.rand(n, dtype=torch.float64, device="cuda", generator=torch.Generator("cuda").manual_seed(5)) - 0.5
+    b[levels[0].bnd.long()] = 0.0
+    out = []
+    for lattice in (1, 0):
+        s = MGPCG(levels, inner=inner, fmt="banded", options={"lattice": lattice}).init()
+        assert s.info()["finest_lattice"] == lattice * (dim - 1) and s.info()["outer_columns"] == lattice * (dim - 2)
+        x = torch.zeros_like(b)
+        out.append((s.correct(x, b), x, s.history()))
+        s.done()
+    (r, x, h), (q, y, g) = out
+    assert r == q and r[0] == 2
+    assert h[0] == pytest.approx(g[0], rel=1e-12)
+    assert (np.abs(h - g)[1:] <= 2.0 ** -24 * g[:-1]).all(), (h, g)
+    assert float((x - y).norm()) <= 2.0 ** -24 * float(y.norm())
+
+
+def lattice_hierarchy(dim, deg, cells):
+    """Laplacians of 2^k * c cells per axis with the two-level transfers, coarsened while the cells are even."""
+    import scipy.sparse as sp
+    H = pb.Hierarchy(dim, deg)
+
+    def csr(M):
+        M = sp.csr_matrix(M)
+        M.sort_indices()
+        return pb.Csr(M.shape[0], M.shape[1], M.indptr.astype(np.uint32), M.indices.astype(np.uint32), M.data.astype(np.float64))
+
+    def line(c):
+        k = np.array([[1, -1], [-1, 1]]) if deg == 1 else np.array([[7, -8, 1], [-8, 16, -8], [1, -8, 7]]) / 3.0
+        w = np.array([[2, 1], [1, 2]]) / 6.0 if deg == 1 else np.array([[4, 2, -1], [2, 16, 2], [-1, 2, 4]]) / 30.0
+        K, M = np.zeros((deg * c + 1,) * 2), np.zeros((deg * c + 1,) * 2)
+        for e in range(c):
+            i = slice(deg * e, deg * e + deg + 1)
+            K[i, i] += k
+            M[i, i] += w
+        return sp.csr_matrix(K), sp.csr_matrix(M)
+
+    def prol(c):
+        m = deg * c + 1
+        P = np.zeros((m, deg * c // 2 + 1))
+        for i in range(m):
+            if deg == 1:
+                P[i, i // 2] += 0.5
+                P[i, (i + 1) // 2] += 0.5
+            else:
+                e, t = min(i // 4, c // 2 - 1), (i - 4 * min(i // 4, c // 2 - 1)) / 4.0
+                P[i, 2 * e:2 * e + 3] = [(1 - t) * (1 - 2 * t), 4 * t * (1 - t), t * (2 * t - 1)]
+        return sp.csr_matrix(P)
+
+    def kron(fs):
+        out = fs[0]
+        for f in fs[1:]:
+            out = sp.kron(f, out, format="csr")
+        return out
+    while True:
+        K, M = line(cells)
+        A = sum(kron([K if a == ax else M for a in range(dim)]) for ax in range(dim))
+        m = deg * cells + 1
+        edge = np.zeros((m,) * dim, bool)
+        for ax in range(dim):
+            edge[(slice(None),) * ax + (0,)] = edge[(slice(None),) * ax + (-1,)] = True
+        L = pb.Level(csr(A), np.flatnonzero(edge.ravel()).astype(np.uint32))
+        H.levels.append(L)
+        if cells % 2 or m ** dim <= 130:
+            return H
+        P = kron([prol(cells)] * dim)
+        L.P, L.R = csr(P), csr(P.T)
+        cells //= 2
+
+
+@pytest.mark.parametrize("inner", ["f64", "f32", "f16"])
+@pytest.mark.parametrize("dim,deg,cells", [(2, 1, 20), (2, 1, 44), (2, 1, 104), (2, 2, 12), (2, 2, 20), (2, 2, 44), (3, 1, 10),
+                                           (3, 1, 12), (3, 1, 20), (3, 1, 36)])
+def test_lattices_of_other_sizes(torch, dim, deg, cells, inner):
+    """Lattices whose cells per axis are no power of two (and coarse ones with an even number of nodes)."""
+    H = lattice_hierarchy(dim, deg, cells)
+    d = defect(H)
+    for cycle, pre, post in (("v", 4, 4), ("f", 1, 2)):
+        a, ka = cycles(torch, H, d, inner, 1, cycle=cycle, pre=pre, post=post)
+        b, kb = cycles(torch, H, d, inner, 0, cycle=cycle, pre=pre, post=post)
+        assert ka < kb, (ka, kb)
+        assert np.array_equal(a, b), (cycle, pre, post, np.abs(a - b).max())

@@ -34,6 +34,7 @@ def test_tail_matrix_matches_the_steps(torch, dim, deg, lvl, cycle, inner):
     for tail in (1100, 0):
         s = MGPCG(H, inner=inner, cycle=cycle, options={"tail_max_n": tail}).init()
         assert (s.info()["tail_levels"] > 0) == (tail > 0 and lvl > 1)
+        assert (s.info()["tail_matrices"] > 0) == (tail > 0 and lvl > 1)
         c = torch.empty_like(dd)
         for _ in range(2):      # a second cycle starts from the first one's buffers
             s.vcycle(c, dd)

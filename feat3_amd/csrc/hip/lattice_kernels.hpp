@@ -23,7 +23,8 @@
 //
 // Every node's row sum takes the terms of its matrix row in ascending column order with fused
 // multiply-adds, and the steps' expressions are those of k_sweep, k_defect, k_restrict and
-// k_prolong: the iterates are those of the banded kernels bit for bit.
+// k_prolong: the iterates are those of the banded kernels bit for bit (the general formats round their
+// products before adding them and differ by that).
 #pragma once
 
 #include "device_common.hpp"

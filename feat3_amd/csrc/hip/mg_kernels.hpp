@@ -1179,8 +1179,8 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
   // the result as the steps' errors do (2D Q1, 33 x 33 nodes, checkerboard b: |M| |b| is 100 times M b).
   // So M is formed and kept with twice the digits of the cycle's arithmetic -- FP64 for FP32 cycles, an
   // unevaluated sum of two FP64 values (Dd) for FP64 ones -- and the product is summed alike: its
-  // result is M b rounded once.  Relative error there, steps -> matrix: FP32 5e-8 -> 2.4e-8, FP64
-  // 7e-17 -> 6e-17 (with entries of the cycle's own precision 1.3e-6 and 7e-15).
+  // result is M b rounded once.  Relative error there, steps -> matrix: FP32 4e-8 -> 1.7e-8, FP64
+  // 7e-17 -> 3e-17 (with entries of the cycle's own precision 1.2e-6 and 6e-15).
   constexpr u64 kTailMatRows = 2048;   // levels of at most this many rows (a 67 MB matrix in FP64)
 
   struct Dd

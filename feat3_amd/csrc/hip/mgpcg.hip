@@ -2209,14 +2209,17 @@ namespace
       return rt::kOk;
     }
 
+    // 3D levels from this many rows on take one step per launch, by columns.  129^3 nodes in FP32: 7.8 us a
+    // step, two steps 29.5 us in a brick launch.  V-cycles with the finest level in bricks / by columns,
+    // 65^3 nodes: FP32 69.7 / 88.9 us, binary16 values 69.5 / 88.8 us, FP64 97.8 / 117.9 us (row kernels
+    // 113, 114, 162 us).
+    static constexpr u64 kColumnRows = u64(1) << 20;
+
     // Decides whether a level is smoothed in bricks (or columns): its prolongation is that of a Q1 or 2D
     // Q2 space on a lattice (checked entry by entry when its factors were built), its matrix couples
     // only the nodes of a box, and all inner rows of a class are the same with the Dirichlet nodes the
-    // lattice's boundary -- or, 2D Q1, any values.  Everything else keeps its format's kernels.
-    // 3D levels from this many rows on take one step per launch: 129^3 nodes in FP32, two steps 29.5 us
-    // in a brick launch; 65^3 nodes, a level's way down and up 39 us in bricks, ten launches of 4 us
-    static constexpr u64 kColumnRows = u64(1) << 20;
-
+    // lattice's boundary -- or, 2D Q1, any values.  Everything else keeps its format's kernels.  The format's
+    // copy of the matrix stays also where the cycle does not read it: statistics and time_kernel run on it.
     int setup_lattice(Level<DT, VT>& l)
     {
       l.lat = -1;

@@ -89,7 +89,9 @@ namespace
     // LDS-resident workgroup per system (batch::k_tail_sys); 0 = every level keeps its launches
     u64 tail_nodes = 1000;
     // the same limit with values per system.  Forward, adjoint and gradient of 16 fields at 2D level 10:
-    // no tail 33.0 ms, from 17^2 nodes 31.6, 33^2 31.4, 65^2 32.0 (16 workgroups on 256 CUs)
+    // no tail 33.0 ms, from 17^2 nodes 31.6, 33^2 31.4, 65^2 32.0 (16 workgroups on 256 CUs).  A solve on
+    // 65^2 nodes without / with it, 1, 16 and 64 systems: FP32 1.00 / 0.74, 1.05 / 0.77, 1.41 / 1.00 ms,
+    // FP64 1.08 / 0.84, 1.08 / 0.86, 1.45 / 1.12 ms
     u64 tail_fields = 1100;
     // 3D lattice levels whose inner rows are all alike take their steps by lines along z
     // (batch_lattice.hpp), 2D lattice levels with one matrix per system several steps a pass
@@ -605,7 +607,12 @@ namespace
     // Steps of one pass at most (batch::k_field_rows): the registers of 1024 threads (128 each) hold the
     // rows of four FP32 steps, of three with binary16 values (converted at each use) or two FP64 ones.
     static constexpr int kFieldSteps = sizeof(DT) == 8 ? 2 : sizeof(VT) == 2 ? 3 : 4;
-    static constexpr u32 kFieldNodes = 100;   // 129^2: 17 us a pass against 4 x 4.9 us; 65^2: 4 x 4.3 us
+    // 129^2 nodes, 16 systems: 17 us a pass against 4 x 4.9 us; 65^2: 4 x 4.3 us.  Solves with one launch per
+    // step -> passes (no coarse tail; 1, 8, 64 systems): 129^2 FP32 1.25 -> 1.21, 1.30 -> 1.34, 2.08 -> 1.85 ms,
+    // FP64 1.36 -> 1.27, 1.38 -> 1.52, 2.53 -> 2.36 ms; 257^2 FP32 1.78 -> 1.52, 1.77 -> 1.68, 4.47 -> 3.46 ms,
+    // FP64 2.17 -> 1.65, 2.00 -> 2.04, 7.17 -> 5.60 ms: 4 to 16 systems in FP64 lose up to 10% on the two
+    // smallest levels and gain from 513^2 on
+    static constexpr u32 kFieldNodes = 100;
 
     // the next pass of `left` steps on level f: its number of steps (1: the row kernels)
     static int field_pass(const Level& f, int left)

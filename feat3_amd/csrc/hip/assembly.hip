@@ -110,7 +110,7 @@ namespace
       assemble_row(G, R, hs, nfields, t / u64(nfields), t % u64(nfields), kf, rp, col, val);
   }
 
-  // Q1 in the plane: a block takes kAsmNodes nodes of a mesh line and up to kAsmFields fields.  The
+  // Q1 in the plane: a block takes kAsmNodes nodes of a mesh line and up to fb <= kAsmFields fields.  The
   // cells' coefficients lie [field][cell] and the values are written [entry][field], so the block
   // loads its two rows of cells along x, turns them in LDS (17 doubles a cell: no bank repeats) and
   // writes along the fields.  An inner node with the 9 neighbours in its row sums its 1, 2 or 4
@@ -118,15 +118,15 @@ namespace
   // is the store of the values.  Measured at 1025^2 nodes and 16 fields (1.2 GB of values, 240 us at
   // the rate of a copy): 1505 us by assemble_row alone, 414 us here, 549 with the graph checked per value.
   constexpr u32 kAsmNodes = 64, kAsmFields = 16, kAsmStride = kAsmFields + 1;
-  __global__ __launch_bounds__(256) void k_assemble_q1_2d(GridDev G, RefMatrix R, double hs, int nfields,
+  __global__ __launch_bounds__(256) void k_assemble_q1_2d(GridDev G, RefMatrix R, double hs, int nfields, u32 fb,
                                                           const double* __restrict__ kf, const u32* __restrict__ rp,
                                                           const u32* __restrict__ col, double* __restrict__ val)
   {
     __shared__ double kc[2][(kAsmNodes + 1) * kAsmStride];
     __shared__ u32 first[kAsmNodes], other[kAsmNodes];   // a row's first entry; nonzero: not the nine neighbours
     const u32 m = u32(G.m), cells = u32(G.cells), tiles = (m + kAsmNodes - 1) / kAsmNodes;
-    const u32 x0 = blockIdx.x % tiles * kAsmNodes, y = blockIdx.x / tiles % m, f0 = blockIdx.x / tiles / m * kAsmFields;
-    const u32 F = u32(nfields) - f0 < kAsmFields ? u32(nfields) - f0 : kAsmFields;
+    const u32 x0 = blockIdx.x % tiles * kAsmNodes, y = blockIdx.x / tiles % m, f0 = blockIdx.x / tiles / m * fb;
+    const u32 F = u32(nfields) - f0 < fb ? u32(nfields) - f0 : fb;   // (fb <= kAsmFields)
     const u64 ncell = u64(cells) * cells;
     if(threadIdx.x < kAsmNodes && x0 + threadIdx.x < m)
     {
@@ -538,10 +538,16 @@ int feat3_assemble_laplace_fields(void* stream, int dim, int degree, int level, 
   for(int d = 2; d < dim; ++d) hs *= h;
   if(dim == 2 && degree == 1)
   {
-    const u64 nb = (G.m + kAsmNodes - 1) / kAsmNodes * G.m * ((u64(nfields) + kAsmFields - 1) / kAsmFields);
+    const u64 tiles = (G.m + kAsmNodes - 1) / kAsmNodes * G.m;
+    u32 fb = kAsmFields;
+    // few blocks (eight per CU): four fields each, one value row per thread.  129^2 nodes, 8 / 16 / 40 fields: row by
+    // row 28 / 38 / 75 us, 16 fields a block 30 / 55 / 60 us, four 20 / 29 / 49 us; 33^2 nodes, 16
+    // fields 22, 35, 18 us
+    if(tiles * ((u64(nfields) + fb - 1) / fb) < 2048) fb = 4;
+    const u64 nb = tiles * ((u64(nfields) + fb - 1) / fb);
     if(nb < (u64(1) << 31))
     {
-      k_assemble_q1_2d<<<unsigned(nb), 256, 0, static_cast<hipStream_t>(stream)>>>(G, R, hs, nfields, kfields, row_ptr,
+      k_assemble_q1_2d<<<unsigned(nb), 256, 0, static_cast<hipStream_t>(stream)>>>(G, R, hs, nfields, fb, kfields, row_ptr,
                                                                                     col_ind, val);
       return rt::check_launch();
     }

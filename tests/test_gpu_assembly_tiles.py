@@ -1,4 +1,4 @@
-"""Device assembly of Q1 values in the plane (k_assemble_q1_2d: tiles of 64 nodes and 16 fields) against
+"""Device assembly of Q1 values in the plane (k_assemble_q1_2d: tiles of 64 nodes and 4 or 16 fields) against
 the host setup, bit for bit: node lines of 2 to 129 (one and several tiles, remainders), 1 to 33 fields,
 and rows whose graph is not the nine neighbours in ascending order, which take the general route."""
 import ctypes
@@ -11,7 +11,7 @@ from feat3_amd import problems as pb
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("level,nfields", [(1, 1), (2, 16), (5, 17), (6, 3), (6, 33), (7, 16)])
+@pytest.mark.parametrize("level,nfields", [(1, 1), (2, 16), (5, 17), (6, 3), (6, 33), (7, 16), (7, 7), (8, 20)])
 def test_tiles_are_bitwise_host_assembly(torch_cuda, level, nfields):
     from feat3_amd.autograd import DiffusionProblem
     torch = torch_cuda

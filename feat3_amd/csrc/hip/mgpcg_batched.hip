@@ -528,9 +528,11 @@ namespace
       }
       a.bx = (m + a.nx - 1) / a.nx;
       a.by = (m + a.ny - 1) / a.ny;
-      // planes per block: about 1500 blocks (six a CU), at least 4 planes (each block reads two more)
+      // planes per block: about 1500 blocks (six a CU), at least 2 planes (each block reads two more).  Solves
+      // of 16 FP32 systems by the row kernels / with at least 4 planes / 2: 17^3 nodes 799 / 879 / 794 us,
+      // 33^3 nodes 1273 / 1303 / 1242 us; of 4: 17^3 815 / 862 / 791, 33^3 1221 / 1254 / 1100 us
       const u32 lines = a.bx * a.by * a.groups;
-      const u32 chunks = std::max<u32>(1, std::min<u32>((1500 + lines - 1) / lines, m / 4));
+      const u32 chunks = std::max<u32>(1, std::min<u32>((1500 + lines - 1) / lines, m / 2));
       a.zlen = (m + chunks - 1) / chunks;
       nb = lines * ((m + a.zlen - 1) / a.zlen);
       return a;

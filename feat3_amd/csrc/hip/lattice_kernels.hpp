@@ -687,6 +687,29 @@ namespace lat
 
   // ---- setup ---------------------------------------------------------------------------------
 
+  // The matrix row and dinv (null: not wanted) of one inner node of each class, by taps; rep, repd and flags
+  // zero before.  Raises the flags 1 and 2 for an entry outside the box.  One block of 64 threads.
+  template<typename DT_, typename VT_>
+  __global__ __launch_bounds__(64) void k_lattice_rep(u32 m, int dim, int rad, int per, const u32* __restrict__ rp,
+                                                      const u32* __restrict__ col, const VT_* __restrict__ val,
+                                                      const DT_* __restrict__ dinv, int ntap, DT_* __restrict__ rep,
+                                                      DT_* __restrict__ repd, int* flags)
+  {
+    const int nl = 2 * rad + 1;
+    for(int c = 0; c < (per == 2 ? 4 : 1); ++c)
+    {
+      const int x = 4 + (c & 1), y = 4 + (c >> 1), z = dim == 3 ? 4 : 0;
+      const u32 r = (u32(z) * m + u32(y)) * m + u32(x), e = rp[r], n = rp[r + 1] - e;
+      if(n > 64u) { if(threadIdx.x == 0) atomicOr(flags, 3); return; }
+      if(dinv && threadIdx.x == 0) repd[c] = dinv[r];
+      if(threadIdx.x >= n) continue;
+      const u32 k = col[e + threadIdx.x], kl = k / m, kz = kl / m;
+      const int dx = int(k - kl * m) - x, dy = int(kl - kz * m) - y, dz = int(kz) - z, rz = dim == 3 ? rad : 0;
+      if(dx < -rad || dx > rad || dy < -rad || dy > rad || dz < -rz || dz > rz) { atomicOr(flags, 3); continue; }
+      rep[c * ntap + ((dz + rz) * nl + dy + rad) * nl + dx + rad] = dev::ld<DT_>(val, e + threadIdx.x);
+    }
+  }
+
   // Flags raised: 1 an entry outside the box of RAD nodes around its row's node, or a second one of the
   // same column (the general formats add both; the lattice kernels have one value per neighbour); 2 an inner row that
   // differs (any value or its dinv, as bit patterns) from its class's row in rep, a Dirichlet row with a

@@ -1573,6 +1573,7 @@ namespace
     HostRing* ring = nullptr;
     HostRing* ring_dev = nullptr;
     hipEvent_t t0 = nullptr, t1 = nullptr;
+    DevMem lat_check;      // lattice_rows
     DevMem timing_state;   // solver state "in progress" for timing the outer product alone
 
     ~Engine() override
@@ -2163,47 +2164,27 @@ namespace
     {
       *box = *uniform = false;
       const int nl = 2 * rad + 1, ntap = dim == 3 ? nl * nl * nl : nl * nl, per = rad == 2 ? 2 : 1, ncls = per == 2 ? 4 : 1;
-      rep.assign(std::size_t(ncls) * ntap, T(0));
-      repd.assign(ncls, T(0));
-      bool finite = true;
-      for(int c = 0; c < ncls; ++c)
-      {
-        const u64 x = 4 + u64(c & 1), y = 4 + u64(c >> 1), z = dim == 3 ? 4 : 0, r = (z * m + y) * m + x;
-        u32 e[2];
-        F3_CHECK(hipMemcpy(e, A.rp.template as<u32>() + r, sizeof(e), hipMemcpyDeviceToHost));
-        if(e[1] - e[0] > 64) return rt::kOk;
-        std::vector<u32> col(e[1] - e[0]);
-        std::vector<V> val(e[1] - e[0]);
-        if(!col.empty())
-        {
-          F3_CHECK(hipMemcpy(col.data(), A.col.template as<u32>() + e[0], sizeof(u32) * col.size(), hipMemcpyDeviceToHost));
-          F3_CHECK(hipMemcpy(val.data(), A.val.template as<V>() + e[0], sizeof(V) * val.size(), hipMemcpyDeviceToHost));
-        }
-        if(dinv) F3_CHECK(hipMemcpy(&repd[c], dinv + r, sizeof(T), hipMemcpyDeviceToHost));
-        for(std::size_t k = 0; k < col.size(); ++k)
-        {
-          const int dx = int(col[k] % m) - int(x), dy = int(col[k] / m % m) - int(y), dz = int(col[k] / (m * m)) - int(z);
-          if(std::abs(dx) > rad || std::abs(dy) > rad || std::abs(dz) > (dim == 3 ? rad : 0)) return rt::kOk;
-          const T v = T(val[k]);
-          finite = finite && std::isfinite(double(v));
-          rep[std::size_t(c) * ntap + ((dim == 3 ? dz + rad : 0) * nl + dy + rad) * nl + dx + rad] = v;
-        }
-        finite = finite && std::isfinite(double(repd[c]));
-      }
-      DevMem drep, drepd, dflag;
-      F3_RC(drep.alloc(sizeof(T) * rep.size()));
-      F3_RC(drepd.alloc(sizeof(T) * repd.size()));
-      F3_RC(dflag.alloc(sizeof(int)));
-      F3_CHECK(hipMemcpyAsync(drep.p, rep.data(), sizeof(T) * rep.size(), hipMemcpyHostToDevice, s));
-      F3_CHECK(hipMemcpyAsync(drepd.p, repd.data(), sizeof(T) * repd.size(), hipMemcpyHostToDevice, s));
-      F3_CHECK(hipMemsetAsync(dflag.p, 0, sizeof(int), s));
+      // rows, dinv and flags in one buffer, found and compared on the device: one copy to the host per level
+      struct Check { T rep[4 * 27], repd[4]; int flags; };
+      if(!lat_check.p) F3_RC(lat_check.alloc(4096));
+      static_assert(sizeof(Check) <= 4096 && 4 * 25 <= 4 * 27, "one buffer for every level");
+      Check* d = lat_check.template as<Check>();
+      F3_CHECK(hipMemsetAsync(d, 0, sizeof(Check), s));
+      lat::k_lattice_rep<T, V><<<1, 64, 0, s>>>(m, dim, rad, per, A.rp.template as<u32>(), A.col.template as<u32>(), A.val.template as<V>(),
+                                               dinv, ntap, d->rep, d->repd, &d->flags);
       lat::k_lattice_check<T, V><<<setup_blocks(A.rows), 256, 0, s>>>(
         A.rows, m, mg::udiv_magic_for(m), dim, rad, per, A.rp.template as<u32>(), A.col.template as<u32>(), A.val.template as<V>(),
-        mask.template as<u32>(), dinv, drep.template as<T>(), drepd.template as<T>(), ntap, dflag.template as<int>());
+        mask.template as<u32>(), dinv, d->rep, d->repd, ntap, &d->flags);
       F3_RC(rt::check_launch());
-      int flag = 3;
-      F3_CHECK(hipMemcpyAsync(&flag, dflag.p, sizeof(int), hipMemcpyDeviceToHost, s));
+      Check h;
+      F3_CHECK(hipMemcpyAsync(&h, d, sizeof(Check), hipMemcpyDeviceToHost, s));
       F3_CHECK(hipStreamSynchronize(s));
+      const int flag = h.flags;
+      rep.assign(h.rep, h.rep + std::size_t(ncls) * ntap);
+      repd.assign(h.repd, h.repd + ncls);
+      bool finite = true;
+      for(T v : rep) finite = finite && std::isfinite(double(v));
+      for(T v : repd) finite = finite && std::isfinite(double(v));
       *box = !(flag & 1);
       *uniform = finite && flag == 0;
       return rt::kOk;

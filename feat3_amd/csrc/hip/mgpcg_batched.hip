@@ -451,6 +451,7 @@ namespace
       for(T& v : k) v = T(0);
       u32 taps = 0;
       std::int64_t off[27];
+      double k64[27] = {};   // the first row as given: a value equal to it needs no conversion
       u64 r = 0;
       for(u32 z = 0; z < m; ++z)
         for(u32 y = 0; y < m; ++y)
@@ -463,7 +464,7 @@ namespace
             {
               // (the row kernels carry a value that is not finite into the cycle, and the solve reports it)
               for(u64 e = rp[r] * per; e < rp[r + 1] * per; ++e)
-                if(!std::isfinite(double(T(to_storage<V>(val[e]))))) return 0;
+                if(!(std::fabs(val[e]) <= 6e4) && !std::isfinite(double(T(to_storage<V>(val[e]))))) return 0;   // (binary16: to 65504)
               continue;
             }
             const u32 e0 = rp[r], count = rp[r + 1] - e0;
@@ -481,7 +482,8 @@ namespace
                 if(t == 27) return 0;
                 taps |= 1u << t;
                 off[i] = o;
-                k[t] = T(to_storage<V>(val[u64(e0 + i) * per]));
+                k64[t] = val[u64(e0 + i) * per];
+                k[t] = T(to_storage<V>(k64[t]));
                 if(!std::isfinite(double(k[t]))) return 0;
               }
               if(taps != lat::kTapsAll && taps != lat::kTapsNoFaces) return 0;
@@ -494,7 +496,7 @@ namespace
               if(std::int64_t(col[e0 + i]) - std::int64_t(r) != off[i]) return 0;
               const double* v = val.data() + u64(e0 + i) * per;
               for(u64 h = 0; h < per; ++h)
-                if(per > u64(B) && h % u64(B + 1) != 0 ? v[h] != 0.0 : T(to_storage<V>(v[h])) != k[t]) return 0;
+                if(per > u64(B) && h % u64(B + 1) != 0 ? v[h] != 0.0 : v[h] != k64[t] && T(to_storage<V>(v[h])) != k[t]) return 0;
             }
           }
       faces = taps == lat::kTapsAll;

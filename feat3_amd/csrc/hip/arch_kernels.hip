@@ -97,7 +97,8 @@ namespace
   template<int BS, typename DT>
   constexpr int stream_cap() { return kStreamBytes / (BS * int(sizeof(DT))); }
 
-  template<int BS, typename DT, typename VT, typename IT>
+  // AHEAD: products of a row read from LDS before they are summed (launch_csr_stream)
+  template<int BS, typename DT, typename VT, typename IT, int AHEAD>
   __global__ __launch_bounds__(kBlock) void k_csr_stream(DT* __restrict__ r, DT a, const DT* __restrict__ x, DT b,
                                                          const DT* y, const VT* __restrict__ val, const IT* __restrict__ col,
                                                          const IT* __restrict__ rp, u64 rows, u64 R, int use_y)
@@ -153,22 +154,21 @@ namespace
         DT s[BS];
 #pragma unroll
         for(int h = 0; h < BS; ++h) s[h] = DT(0);
-        // eight products are read ahead of their sums (a row alone waits for each LDS read otherwise):
-        // FP32, 300,007 irregular rows of 23 entries on average 21.9 -> 18.3 us (four: 20.1)
         u32 k = u32(k0);
         const u32 ke = u32(k1);
-        for(; k + 8 <= ke; k += 8)
-        {
-          DT p[8][BS];
+        if constexpr(AHEAD > 1)
+          for(; k + AHEAD <= ke; k += AHEAD)
+          {
+            DT p[AHEAD][BS];
 #pragma unroll
-          for(int j = 0; j < 8; ++j)
+            for(int j = 0; j < AHEAD; ++j)
 #pragma unroll
-            for(int h = 0; h < BS; ++h) p[j][h] = prod[(k + u32(j)) * BS + h];
+              for(int h = 0; h < BS; ++h) p[j][h] = prod[(k + u32(j)) * BS + h];
 #pragma unroll
-          for(int j = 0; j < 8; ++j)
+            for(int j = 0; j < AHEAD; ++j)
 #pragma unroll
-            for(int h = 0; h < BS; ++h) s[h] += p[j][h];
-        }
+              for(int h = 0; h < BS; ++h) s[h] += p[j][h];
+          }
         for(; k < ke; ++k)
 #pragma unroll
           for(int h = 0; h < BS; ++h) s[h] += prod[k * BS + h];
@@ -214,7 +214,15 @@ namespace
     const u64 R = fit < 1.0 ? 1 : (fit > 1024.0 ? 1024 : u64(fit));
     const u64 nb = (rows + R - 1) / R;
     if(nb > 0x7fffffffull) return rt::kErrArg;
-    k_csr_stream<BS, DT, VT, IT><<<unsigned(nb), kBlock, 0, s>>>(r, a, x, b, y, val, col, rp, rows, R, use_y);
+    // A row alone waits for each LDS read of a product, so eight are read ahead of their sums while the
+    // matrix fits the 256 MB Infinity Cache: irregular rows, one / eight at a time, FP32 300,007 rows of 23
+    // entries 22.3 / 17.2 us, 30,001 of 60 25.4 / 16.4, FP64 26.3 / 22.6 and 26.3 / 15.6 us.  Beyond, HBM
+    // bounds the product and the faster sums only crowd it: 1,000,003 rows, FP64 of 40 entries 124 /
+    // 135, of 60 194 / 213 us, FP32 of 60 141 / 146 us.
+    if(double(nnz) * double(sizeof(VT) + sizeof(IT)) <= 268435456.0)
+      k_csr_stream<BS, DT, VT, IT, 8><<<unsigned(nb), kBlock, 0, s>>>(r, a, x, b, y, val, col, rp, rows, R, use_y);
+    else
+      k_csr_stream<BS, DT, VT, IT, 1><<<unsigned(nb), kBlock, 0, s>>>(r, a, x, b, y, val, col, rp, rows, R, use_y);
     return rt::check_launch();
   }
 

@@ -105,3 +105,27 @@ def test_tail_matrix_rounds_once(torch, dim, lvl, inner):
         print(f"  {dim}D level {lvl} {inner} {name}: {err / u:.3f} u", flush=True)
         assert err <= 1.001 * u
     s.done()
+
+
+@pytest.mark.parametrize("inner,cells,matrices", [("f64", 44, 0), ("f32", 44, 1), ("f64", 40, 1), ("f32", 64, 0)])
+def test_tails_that_keep_their_steps(torch, inner, cells, matrices):
+    """A tail of 2025 rows whose vectors with twice the digits exceed the LDS in FP64, and one of 4225 rows,
+    run step by step; with 1681 rows FP64 has its matrix too.  Against the launches level by level."""
+    from feat3_amd.solver import MGPCG
+    from test_gpu_lattice import lattice_hierarchy
+    H = lattice_hierarchy(2, 1, cells)
+    d = np.random.default_rng(5).uniform(-1.0, 1.0, H.n)
+    d[H.levels[0].bnd] = 0.0
+    dd = torch.from_numpy(d).cuda()
+    out = []
+    for tail in (4300, 0):
+        s = MGPCG(H, inner=inner, options={"tail_max_n": tail}).init()
+        info = s.info()
+        if tail:
+            assert info["tail_levels"] == len(H.levels) and info["tail_matrices"] == matrices, info
+        c = torch.empty_like(dd)
+        s.vcycle(c, dd)
+        out.append(c.cpu().numpy())
+        s.done()
+    err = np.linalg.norm(out[0] - out[1]) / np.linalg.norm(out[1])
+    assert err <= (1e-12 if inner == "f64" else 64 * np.finfo(np.float32).eps)

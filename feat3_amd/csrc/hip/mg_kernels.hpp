@@ -1177,7 +1177,8 @@ _Pragma(F3_STR(unroll F3_BAND_UNROLL))
   //
   // Precision: an entry's error counts against |M| |b| and not against |M b|, so it does not shrink with
   // the result as the steps' errors do (2D Q1, 33 x 33 nodes, checkerboard b: |M| |b| is 100 times M b).
-  // So M is formed and kept with twice the digits of the cycle's arithmetic -- FP64 for FP32 cycles, an
+  // So M is formed and kept with twice the digits of the cycle's arithmetic -- FP64 for FP32 cycles (from the
+  // FP64 level matrices, unless the values are stored in binary16), an
   // unevaluated sum of two FP64 values (Dd) for FP64 ones -- and the product is summed alike: its
   // result is M b rounded once.  Relative error there, steps -> matrix: FP32 4e-8 -> 1.7e-8, FP64
   // 7e-17 -> 3e-17 (with entries of the cycle's own precision 1.2e-6 and 6e-15).

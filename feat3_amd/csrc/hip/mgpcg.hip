@@ -1698,7 +1698,7 @@ namespace
       L.back()->xfinal = L.back()->x.template as<DT>();
       F3_RC(setup_tail(lv));
       for(std::size_t i = 0; cfg.lattice && i < tail0; ++i) F3_RC(setup_lattice(*L[i]));
-      F3_RC(build_cycle());
+      F3_RC(build_cycle(lv));
 
       // outer PCG
       const HostLevel& h0 = lv.front();
@@ -1837,13 +1837,14 @@ namespace
     std::size_t tail0 = 0;
     mg::TailDesc<DT, VT> tail{};
     u64 tail_lds = 0, tail_cap = 0;   // LDS bytes of k_tail, the device's limit per workgroup
-    std::vector<std::unique_ptr<DevMem>> tail_mem;
+    DevMem tail_mem, tail64;   // tail_levels
 
     // ELL copy for the tail kernel: 16-bit columns, the entries band_keeps(v, row diagonal, thin)
     // (thin = 0: exact zeros dropped; the level matrices take level_thin()), entry k of row r at
     // k * rows + r, padded with column 0 and value 0; with FP32 arithmetic a width of at most 32
     // other than 9, 21, 25 or 27 is padded to a multiple of 8 (the kernel's fixed-width row sums)
-    int tail_ell(const HostCsr& h, mg::TailEll<VT>& e, double thin)
+    template<typename V>
+    static u64 ell_arrays(const HostCsr& h, double thin, std::vector<std::uint16_t>& col, std::vector<V>& val)
     {
       std::vector<double> dg(h.rows, 0.0);
       for(u64 r = 0; r < h.rows; ++r)
@@ -1857,8 +1858,8 @@ namespace
         w = std::max(w, c);
       }
       if(sizeof(DT) == 4 && w <= 32 && w != 9 && w != 21 && w != 25 && w != 27) w = (w + 7) / 8 * 8;
-      std::vector<std::uint16_t> col(w * h.rows, 0);
-      std::vector<VT> val(w * h.rows, to_storage<VT>(0.0));
+      col.assign(w * h.rows, 0);
+      val.assign(w * h.rows, to_storage<V>(0.0));
       for(u64 r = 0; r < h.rows; ++r)
       {
         u64 j = 0;
@@ -1866,29 +1867,78 @@ namespace
           if(band_keeps(h.val[k], dg[r], thin))
           {
             col[j * h.rows + r] = std::uint16_t(h.col[k]);
-            val[j * h.rows + r] = to_storage<VT>(h.val[k]);
+            val[j * h.rows + r] = to_storage<V>(h.val[k]);
             ++j;
           }
       }
-      std::unique_ptr<DevMem> mc(new DevMem()), mv(new DevMem());
-      F3_RC(mc->alloc(sizeof(std::uint16_t) * col.size()));
-      F3_RC(mv->alloc(sizeof(VT) * val.size()));
-      if(!col.empty())
+      return w;
+    }
+    // The tail's levels with values of type V in one buffer.  Arithmetic D = DT: the level's dinv; else (FP64
+    // beside an FP32 cycle) dinv from the FP64 diagonals.
+    template<typename D, typename V>
+    int tail_levels(const std::vector<HostLevel>& lv, double thin, mg::TailDesc<D, V>& d, DevMem& mem)
+    {
+      std::vector<char> blob;
+      auto put = [&](const auto& v) {
+        const std::size_t at = (blob.size() + 15) / 16 * 16, bytes = v.size() * sizeof(v[0]);
+        blob.resize(at + bytes);
+        if(bytes) std::memcpy(blob.data() + at, v.data(), bytes);
+        return reinterpret_cast<const void*>(at);   // an offset until the buffer is allocated
+      };
+      auto ell = [&](const HostCsr& h, double eps2) {
+        std::vector<std::uint16_t> col;
+        std::vector<V> val;
+        const u64 w = ell_arrays(h, eps2, col, val);
+        const void* c = put(col);
+        return mg::TailEll<V>{static_cast<const std::uint16_t*>(c), static_cast<const V*>(put(val)), u32(h.rows), u32(w)};
+      };
+      d.nlev = int(L.size() - tail0);
+      d.ncoarse = u32(ncoarse);
+      d.ainv = ainv.template as<double>();
+      u64 off = 0;
+      for(int i = 0; i < d.nlev; ++i)
       {
-        F3_CHECK(hipMemcpyAsync(mc->p, col.data(), sizeof(std::uint16_t) * col.size(), hipMemcpyHostToDevice, s));
-        F3_CHECK(hipMemcpyAsync(mv->p, val.data(), sizeof(VT) * val.size(), hipMemcpyHostToDevice, s));
+        const HostLevel& h = lv[tail0 + std::size_t(i)];
+        const Level<DT, VT>& l = *L[tail0 + std::size_t(i)];
+        mg::TailLevel<D, V>& t = d.lv[i];
+        t.n = u32(l.n);
+        t.off = u32(off);
+        off += 5 * l.n;
+        t.mask = l.mask.template as<u32>();
+        t.A = ell(h.A, thin);
+        if(i + 1 < d.nlev) { t.P = ell(h.P, 0.0); t.R = ell(h.R, 0.0); }
+        if constexpr(std::is_same<D, DT>::value) t.dinv = l.dinv.template as<DT>();
+        else
+        {
+          std::vector<D> dinv(h.A.rows, D(0));   // as mg::k_make_dinv
+          for(u64 r = 0; r < h.A.rows; ++r)
+          {
+            double g = 0.0;
+            for(u32 k = h.A.rp[r]; k < h.A.rp[r + 1]; ++k)
+              if(u64(h.A.col[k]) == r) { g = h.A.val[k]; break; }
+            dinv[r] = D(cfg.omega_r * (cfg.omega_j / g));
+          }
+          for(u32 r : h.fidx) dinv[r] = D(0);
+          t.dinv = static_cast<const D*>(put(dinv));
+        }
       }
-      F3_CHECK(hipStreamSynchronize(s));   // host staging vectors go out of scope
-      e = mg::TailEll<VT>{mc->template as<std::uint16_t>(), mv->template as<VT>(), u32(h.rows), u32(w)};
-      tail_mem.push_back(std::move(mc));
-      tail_mem.push_back(std::move(mv));
+      F3_RC(mem.alloc(blob.size()));
+      F3_CHECK(hipMemcpyAsync(mem.p, blob.data(), blob.size(), hipMemcpyHostToDevice, s));
+      F3_CHECK(hipStreamSynchronize(s));   // blob leaves scope
+      auto move = [&](auto*& p) { p = reinterpret_cast<std::decay_t<decltype(p)>>(mem.template as<char>() + reinterpret_cast<std::size_t>(p)); };
+      for(int i = 0; i < d.nlev; ++i)
+      {
+        mg::TailLevel<D, V>& t = d.lv[i];
+        move(t.A.col); move(t.A.val);
+        if(i + 1 < d.nlev) { move(t.P.col); move(t.P.val); move(t.R.col); move(t.R.val); }
+        if constexpr(!std::is_same<D, DT>::value) move(t.dinv);
+      }
       return rt::kOk;
     }
 
     int setup_tail(const std::vector<HostLevel>& lv)
     {
       const std::size_t nl = L.size();
-      tail_mem.clear();
       int dev = 0, cap = 65536;
       if(hipGetDevice(&dev) == hipSuccess) (void)hipDeviceGetAttribute(&cap, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
       tail_cap = u64(cap);
@@ -1904,29 +1954,10 @@ namespace
       tail = mg::TailDesc<DT, VT>{};
       tail_lds = 0;
       if(tail0 + 1 >= nl) return rt::kOk;
-      tail.nlev = int(nl - tail0);
-      tail.ncoarse = u32(ncoarse);
-      tail.ainv = ainv.template as<double>();
+      F3_RC(tail_levels(lv, std::max(0.0, level_thin()), tail, tail_mem));
       tail.rhs_in = L[tail0]->rhs.template as<DT>();
       tail.x_out = L[tail0]->xfinal;
-      u64 off = 0;
-      for(std::size_t i = tail0; i < nl; ++i)
-      {
-        Level<DT, VT>& l = *L[i];
-        mg::TailLevel<DT, VT>& t = tail.lv[i - tail0];
-        t.n = u32(l.n);
-        t.off = u32(off);
-        off += 5 * l.n;
-        F3_RC(tail_ell(lv[i].A, t.A, std::max(0.0, level_thin())));
-        if(i + 1 < nl)
-        {
-          F3_RC(tail_ell(lv[i].P, t.P, 0.0));
-          F3_RC(tail_ell(lv[i].R, t.R, 0.0));
-        }
-        t.mask = l.mask.template as<u32>();
-        t.dinv = l.dinv.template as<DT>();
-      }
-      tail_lds = off * sizeof(DT);
+      tail_lds = arena(tail0);
       if(tail_lds > 65536)
         F3_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&mg::k_tail<DT, VT>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(tail_lds)));
@@ -1954,9 +1985,25 @@ namespace
     // Tails of more than kTailMatRows rows (option tail_max_n; 4225 rows would read 143 MB per
     // segment, longer than k_tail takes), whose vectors do not fit the LDS with twice the digits, and further
     // kinds beyond eight run k_tail.
-    int build_tail_mats(const std::vector<u32>& ops)
+    int build_tail_mats(const std::vector<HostLevel>& lv, const std::vector<u32>& ops)
     {
-      typedef typename std::conditional<sizeof(DT) == 8, mg::Dd, double>::type C;
+      // FP32 values: from the FP64 matrices, whose rounding to FP32 the product then need not carry.  V(4,4)
+      // cycles to the exact ones (2-norm, steps / FP32 matrices / FP64 ones): 3D Q1 L5 5.1e-8 / 5.2e-8 /
+      // 4.5e-8, 2D Q1 L6 1.1e-7 / 6.7e-8 / 4.8e-8, 2D Q2 L5 3.1e-7 / 3.1e-7 / 1.1e-7
+      if constexpr(std::is_same<VT, float>::value)
+      {
+        mg::TailDesc<double, double> d{};
+        F3_RC(tail_levels(lv, 0.0, d, tail64));
+        return form_tail_mats<double>(d, ops);
+      }
+      else
+        return form_tail_mats<typename std::conditional<sizeof(DT) == 8, mg::Dd, double>::type>(tail, ops);
+    }
+
+    // C: the arithmetic of the columns
+    template<typename C, typename D, typename V>
+    int form_tail_mats(const mg::TailDesc<D, V>& levels, const std::vector<u32>& ops)
+    {
       tail_mats.clear();
       const u64 n = L[tail0]->n, lds = tail_lds / sizeof(DT) / 5 * 4 * sizeof(C);
       if(n > mg::kTailMatRows || lds > tail_cap) return rt::kOk;
@@ -1966,7 +2013,7 @@ namespace
                std::equal(ops.begin() + a.first, ops.begin() + a.first + a.count, ops.begin() + b.first);
       };
       if(lds > 65536)
-        F3_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&mg::k_tail_columns<C, DT, VT>),
+        F3_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(&mg::k_tail_columns<C, D, V>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
       for(TailSeg& g : tail_segs)
       {
@@ -1978,8 +2025,8 @@ namespace
           std::unique_ptr<DevMem> m(new DevMem());
           F3_RC(m->alloc(sizeof(C) * n * n));
           double* hi = m->template as<double>();
-          mg::k_tail_columns<C, DT, VT><<<unsigned(n), mg::kTailThreads, lds, s>>>(tail, tail_ops.template as<u32>() + g.first, g.count,
-                                                                                   g.out_buf, hi, hi + n * n);
+          mg::k_tail_columns<C, D, V><<<unsigned(n), mg::kTailThreads, lds, s>>>(levels, tail_ops.template as<u32>() + g.first, g.count,
+                                                                                 g.out_buf, hi, hi + n * n);
           F3_RC(rt::check_launch());
           tail_mats.push_back(std::move(m));
           kinds.push_back(&g);
@@ -2069,7 +2116,7 @@ namespace
       return o;
     }
 
-    int build_cycle()
+    int build_cycle(const std::vector<HostLevel>& lv)
     {
       const std::vector<CycleOp> full = cycle_schedule();
       const std::size_t nl = L.size();
@@ -2126,7 +2173,7 @@ namespace
         if(!ops.empty())
         {
           F3_CHECK(hipMemcpyAsync(tail_ops.p, ops.data(), sizeof(u32) * ops.size(), hipMemcpyHostToDevice, s));
-          F3_RC(build_tail_mats(ops));
+          F3_RC(build_tail_mats(lv, ops));
           F3_CHECK(hipStreamSynchronize(s));   // ops leaves scope
         }
       }

@@ -107,6 +107,29 @@ def test_tail_matrix_rounds_once(torch, dim, lvl, inner):
     s.done()
 
 
+@pytest.mark.parametrize("dim,deg,lvl,cycle,coef", [(2, 1, 5, "v", False), (2, 1, 5, "f", False), (2, 1, 4, "w", True), (2, 2, 4, "v", False),
+                                                    (3, 1, 3, "v", False), (2, 1, 5, "v", True)])
+def test_fp32_tail_does_not_carry_the_rounded_values(torch, dim, deg, lvl, cycle, coef):
+    """The matrix of an FP32 cycle's tail is formed from the FP64 level matrices: with a right-hand side that
+    FP32 holds, the result is the FP64 cycle's rounded once (at most the unit roundoff, 2-norm)."""
+    from feat3_amd.solver import MGPCG
+    k = np.exp(np.random.default_rng(7).uniform(-1.0, 1.0, 1 << (2 * lvl))) if coef else None
+    H = pb.hierarchy(dim, deg, lvl, 1, kcell=k)
+    d = np.random.default_rng(5).integers(-1000, 1000, H.n).astype(np.float64)
+    d[H.levels[0].bnd] = 0.0
+    out = []
+    for inner in ("f64", "f32"):
+        s = MGPCG(H, inner=inner, cycle=cycle).init()
+        assert s.info()["tail_levels"] == lvl
+        c = torch.empty(H.n, dtype=torch.float64, device="cuda")
+        s.vcycle(c, torch.from_numpy(d).cuda())
+        out.append(c.cpu().numpy())
+        s.done()
+    err = np.linalg.norm(out[1] - out[0]) / np.linalg.norm(out[0])
+    print(f"  {dim}D Q{deg} level {lvl} {cycle} coefficient {coef}: {err * 2 ** 24:.3f} u", flush=True)
+    assert err <= 1.001 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("inner,cells,matrices", [("f64", 44, 0), ("f32", 44, 1), ("f64", 40, 1), ("f32", 64, 0)])
 def test_tails_that_keep_their_steps(torch, inner, cells, matrices):
     """A tail of 2025 rows whose vectors with twice the digits exceed the LDS in FP64, and one of 4225 rows,
